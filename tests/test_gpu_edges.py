@@ -1,0 +1,23 @@
+"""GPU kernels at the edges of their tiles and grids, against plain numpy or the
+oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+# 256 points per partial, at most 1,024 partials, 256 threads in the final block
+@pytest.mark.parametrize("n", [1, 2, 255, 256, 257, 65_536, 65_537, 262_144, 262_145, 1_000_003])
+@pytest.mark.parametrize("ct", [O.CT_F32, O.CT_F64, O.CT_U32, O.CT_U64])
+def test_bbox_reduction_sizes(ft, n, ct):
+    rng = np.random.default_rng(n)
+    p = [(rng.normal(size=n) * 1e3 + (0 if ct in (O.CT_F32, O.CT_F64) else 1e5))
+         .astype(O.COORD_DTYPES[ct]) for _ in range(3)]
+    # the extremes sit at the ends and in the last, partly filled stride
+    p[0][n - 1] = p[0].max() + 1
+    p[2][n // 2] = p[2].min()
+    want = [f(a) for a in p for f in (np.min, np.max)]
+    got = ft.compute_bbox(*p)  # host arrays: staged
+    assert np.array_equal(got, np.array(want, O.COORD_DTYPES[ct]))
