@@ -20,6 +20,7 @@
 #include "ft_internal.hpp"
 
 #include <cmath>
+#include <cstddef>
 #include <vector>
 
 namespace ft {
@@ -130,37 +131,43 @@ __global__ __launch_bounds__(256) void features_kernel(DTree<T> t, const int32_t
 // orientations (W[in][out] for dz W^T, Wt[out][in] for x W).  Per wave: the
 // normalised input and the activations as bf16 row-major [16][64] (next
 // layer's A operand) and transposed [64][16] (A operand of dW = a^T dz).
+// Rows of 64 are NP = 68 apart: an operand load takes 8 bytes from each of 16
+// rows, and rows 128 bytes apart would all start in one of two LDS banks.
 // ===========================================================================
-struct MlpSmem {
-    uint16_t w1[NF * NH], w1t[NH * NF];
-    uint16_t w2[NH * NH], w2t[NH * NH];
-    uint16_t w3[NH * NH], w3t[NH * NH];
+constexpr int NP = NH + 4;
+struct alignas(16) MlpSmem {
+    uint16_t w1t[NH * NF];
+    uint16_t w2[NH * NP], w2t[NH * NP];
+    uint16_t w3[NH * NP], w3t[NH * NP];
     float b1[NH], b2[NH], b3[NH], w4[NH], b4;
     float fmean[NF], finv[NF], ymean, ystd;
 };
-struct MlpWave {
+struct alignas(16) MlpWave {
     uint16_t x[16 * NF], xt[NF * 16];
-    uint16_t a1[16 * NH], a1t[NH * 16];
-    uint16_t a2[16 * NH], a2t[NH * 16];
-    uint16_t dz[16 * NH];
+    uint16_t a1[16 * NP], a1t[NH * 16];
+    uint16_t a2[16 * NP], a2t[NH * 16];
+    uint16_t dz[16 * NP];
 };
+static_assert(offsetof(MlpSmem, w2) % 8 == 0 && offsetof(MlpWave, a1t) % 8 == 0 &&
+                  offsetof(MlpWave, a2t) % 8 == 0 && offsetof(MlpWave, dz) % 8 == 0 &&
+                  sizeof(MlpWave) % 8 == 0 && NP % 4 == 0,
+              "operands are read and written as 8-byte words");
 
 __device__ inline void stage_weights(MlpSmem &S, const float *__restrict__ prm,
                                      const float *__restrict__ norm) {
     for (int i = threadIdx.x; i < NF * NH; i += blockDim.x) {
         const int in = i / NH, out = i % NH;
         const uint16_t b = to_bf16(prm[P_W1 + i]);
-        S.w1[i] = b;
         S.w1t[out * NF + in] = b;
     }
     for (int i = threadIdx.x; i < NH * NH; i += blockDim.x) {
         const int in = i / NH, out = i % NH;
         const uint16_t b2 = to_bf16(prm[P_W2 + i]);
         const uint16_t b3 = to_bf16(prm[P_W3 + i]);
-        S.w2[i] = b2;
-        S.w2t[out * NH + in] = b2;
-        S.w3[i] = b3;
-        S.w3t[out * NH + in] = b3;
+        S.w2[in * NP + out] = b2;
+        S.w2t[out * NP + in] = b2;
+        S.w3[in * NP + out] = b3;
+        S.w3t[out * NP + in] = b3;
     }
     for (int i = threadIdx.x; i < NH; i += blockDim.x) {
         S.b1[i] = prm[P_B1 + i];
@@ -190,11 +197,17 @@ __device__ inline bf16x4 ld4(const uint16_t *p) {
 }
 __device__ inline bf16x4 pack4(f32x4 f) {
     bf16x4 v;
-    v[0] = (short)to_bf16(f[0]);
-    v[1] = (short)to_bf16(f[1]);
-    v[2] = (short)to_bf16(f[2]);
-    v[3] = (short)to_bf16(f[3]);
+    v[0] = bf16_hw(f[0]);
+    v[1] = bf16_hw(f[1]);
+    v[2] = bf16_hw(f[2]);
+    v[3] = bf16_hw(f[3]);
     return v;
+}
+// Four samples' bf16 values of one unit: as one word of the transposed array
+// (t, or null) and down a column of the row-major one.
+__device__ inline void put4(uint16_t *rows, uint16_t *t, int lg, int unit, bf16x4 v) {
+    if (t) *(bf16x4 *)(t + unit * 16 + 4 * lg) = v;
+    for (int i = 0; i < 4; ++i) rows[(4 * lg + i) * NP + unit] = (uint16_t)v[i];
 }
 
 // Forward of one 16-sample tile.  Leaves z1..z3 (pre-activations, D layout,
@@ -205,19 +218,15 @@ struct Fwd {
     f32x4 out;
 };
 
-__device__ inline void mlp_tile_forward(const MlpSmem &S, MlpWave &W, const float *__restrict__ feat,
-                                        int s0, int n, Fwd &F) {
+__device__ inline void mlp_tile_forward(const MlpSmem &S, MlpWave &W, float4 v, Fwd &F) {
     const int l = threadIdx.x & 63;
     const int lr = l & 15, lg = l >> 4;
-    // normalised inputs: A layout x[l%16][4*(l/16)+i]
+    // normalised inputs: A layout x[l%16][4*(l/16)+i], this lane's four in v
     {
-        const int s = s0 + lr;
-        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (s < n) v = ((const float4 *)(feat + (size_t)s * NF))[lg];
         const float vi[4] = {v.x, v.y, v.z, v.w};
         for (int i = 0; i < 4; ++i) {
             const int f = 4 * lg + i;
-            const uint16_t b = to_bf16((vi[i] - S.fmean[f]) * S.finv[f]);
+            const uint16_t b = (uint16_t)bf16_hw((vi[i] - S.fmean[f]) * S.finv[f]);
             W.x[lr * NF + f] = b;
             W.xt[f * 16 + lr] = b;
         }
@@ -230,13 +239,12 @@ __device__ inline void mlp_tile_forward(const MlpSmem &S, MlpWave &W, const floa
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         acc = mfma16(ax, ld4(&S.w1t[(nt * 16 + lr) * NF + 4 * lg]), acc);
         const float b = S.b1[nt * 16 + lr];
+        f32x4 a;
         for (int i = 0; i < 4; ++i) {
             acc[i] += b;
-            const float a = acc[i] > 0.f ? acc[i] : 0.f;
-            const uint16_t h = to_bf16(a);
-            W.a1[(4 * lg + i) * NH + nt * 16 + lr] = h;
-            W.a1t[(nt * 16 + lr) * 16 + 4 * lg + i] = h;
+            a[i] = acc[i] > 0.f ? acc[i] : 0.f;
         }
+        put4(W.a1, W.a1t, lg, nt * 16 + lr, pack4(a));
         F.z1[nt] = acc;
     }
     __builtin_amdgcn_wave_barrier();
@@ -245,16 +253,15 @@ __device__ inline void mlp_tile_forward(const MlpSmem &S, MlpWave &W, const floa
     for (int nt = 0; nt < 4; ++nt) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         for (int kc = 0; kc < 4; ++kc)
-            acc = mfma16(ld4(&W.a1[lr * NH + kc * 16 + 4 * lg]),
-                         ld4(&S.w2t[(nt * 16 + lr) * NH + kc * 16 + 4 * lg]), acc);
+            acc = mfma16(ld4(&W.a1[lr * NP + kc * 16 + 4 * lg]),
+                         ld4(&S.w2t[(nt * 16 + lr) * NP + kc * 16 + 4 * lg]), acc);
         const float b = S.b2[nt * 16 + lr];
+        f32x4 a;
         for (int i = 0; i < 4; ++i) {
             acc[i] += b;
-            const float a = acc[i] > 0.f ? acc[i] : 0.f;
-            const uint16_t h = to_bf16(a);
-            W.a2[(4 * lg + i) * NH + nt * 16 + lr] = h;
-            W.a2t[(nt * 16 + lr) * 16 + 4 * lg + i] = h;
+            a[i] = acc[i] > 0.f ? acc[i] : 0.f;
         }
+        put4(W.a2, W.a2t, lg, nt * 16 + lr, pack4(a));
         F.z2[nt] = acc;
     }
     __builtin_amdgcn_wave_barrier();
@@ -264,8 +271,8 @@ __device__ inline void mlp_tile_forward(const MlpSmem &S, MlpWave &W, const floa
     for (int nt = 0; nt < 4; ++nt) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         for (int kc = 0; kc < 4; ++kc)
-            acc = mfma16(ld4(&W.a2[lr * NH + kc * 16 + 4 * lg]),
-                         ld4(&S.w3t[(nt * 16 + lr) * NH + kc * 16 + 4 * lg]), acc);
+            acc = mfma16(ld4(&W.a2[lr * NP + kc * 16 + 4 * lg]),
+                         ld4(&S.w3t[(nt * 16 + lr) * NP + kc * 16 + 4 * lg]), acc);
         const float b = S.b3[nt * 16 + lr];
         const float w = S.w4[nt * 16 + lr];
         for (int i = 0; i < 4; ++i) {
@@ -396,20 +403,41 @@ __global__ __launch_bounds__(256) void mlp_infer_kernel(const float *__restrict_
 // Gradient of L = (1/total) * sum (out - t)^2 over the samples of this call,
 // t = (y - ymean) / ystd, accumulated into grad[NPARAM] (fp32 atomics) and
 // loss[0].
-__global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__ prm,
+//
+// Bound by the latency of a tile's chain (six LDS exchanges between dependent
+// MFMA groups, about 6 us) and by the sums.  The waves of a block sum their
+// gradients in LDS and the block adds them to the global ones once: with an
+// add per wave, 64k samples made 39 million global atomics (9,488 from each of
+// 4,096 waves) and took 253 us; now 38 us, 16k samples 88 -> 25 us, 1M 866 ->
+// 223 us.  LDS atomics for that sum took 100 us (200 cycles a wave's add), so
+// the waves take turns instead.  GRAD_WAVES waves share one block's staged
+// weights (131 KB of LDS: one block per CU, two waves per SIMD); 128 blocks
+// took 43 us at 64k and 402 at 1M against 39 and 224 with one per CU.
+// Loading the next tile's samples ahead spilled (256 VGPRs) and took 68 us.
+constexpr int GRAD_WAVES = 8;
+constexpr int GRAD_BLOCKS = 256;
+constexpr int GRAD_TILES = 144 * 64;                // weight gradients, by register and lane
+constexpr int GRAD_SUMS = GRAD_TILES + 4 * NH + 2;  // b1, b2, b3, w4, b4 and the loss
+union alignas(16) GradShared {
+    MlpWave w[GRAD_WAVES];
+    float sum[2][GRAD_SUMS];
+};
+static_assert(sizeof(float) * 2 * GRAD_SUMS <= sizeof(MlpWave) * GRAD_WAVES,
+              "the sums fit where the waves' tiles were");
+__global__ __launch_bounds__(64 * GRAD_WAVES) void mlp_grad_kernel(const float *__restrict__ prm,
                                                        const float *__restrict__ norm,
                                                        const float *__restrict__ feat,
                                                        const float *__restrict__ target, int n,
                                                        float inv_total, float *__restrict__ grad,
                                                        float *__restrict__ loss) {
     __shared__ MlpSmem S;
-    __shared__ MlpWave Wv[4];
+    __shared__ GradShared G;
     stage_weights(S, prm, norm);
     __syncthreads();
-    MlpWave &W = Wv[threadIdx.x >> 6];
+    MlpWave &W = G.w[threadIdx.x >> 6];
     const int l = threadIdx.x & 63, lg = l >> 4, lr = l & 15;
-    const int wave = blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int nwaves = gridDim.x * 4;
+    const int wave = blockIdx.x * GRAD_WAVES + (threadIdx.x >> 6);
+    const int nwaves = gridDim.x * GRAD_WAVES;
     f32x4 gW1[4], gW2[4][4], gW3[4][4];
     float gb1[4], gb2[4], gb3[4], gw4[4], gb4 = 0.f, lsum = 0.f;
     for (int a = 0; a < 4; ++a) {
@@ -421,8 +449,10 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
         }
     }
     for (int s0 = wave * 16; s0 < n; s0 += nwaves * 16) {
+        const float4 x = s0 + lr < n ? ((const float4 *)(feat + (size_t)(s0 + lr) * NF))[lg]
+                                     : make_float4(0.f, 0.f, 0.f, 0.f);
         Fwd F;
-        mlp_tile_forward(S, W, feat, s0, n, F);
+        mlp_tile_forward(S, W, x, F);
         // dout for samples 4*lg + i
         f32x4 dout;
         for (int i = 0; i < 4; ++i) {
@@ -454,7 +484,7 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
             for (int mt = 0; mt < 4; ++mt)
                 gW3[mt][nt] = mfma16(ld4(&W.a2t[(mt * 16 + lr) * 16 + 4 * lg]), bz, gW3[mt][nt]);
             gb3[nt] += dz3[nt][0] + dz3[nt][1] + dz3[nt][2] + dz3[nt][3];
-            for (int i = 0; i < 4; ++i) W.dz[(4 * lg + i) * NH + nt * 16 + lr] = to_bf16(dz3[nt][i]);
+            put4(W.dz, nullptr, lg, nt * 16 + lr, bz);
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -463,8 +493,8 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
         for (int nt = 0; nt < 4; ++nt) {
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
             for (int kc = 0; kc < 4; ++kc)
-                acc = mfma16(ld4(&W.dz[lr * NH + kc * 16 + 4 * lg]),
-                             ld4(&S.w3[(nt * 16 + lr) * NH + kc * 16 + 4 * lg]), acc);
+                acc = mfma16(ld4(&W.dz[lr * NP + kc * 16 + 4 * lg]),
+                             ld4(&S.w3[(nt * 16 + lr) * NP + kc * 16 + 4 * lg]), acc);
             for (int i = 0; i < 4; ++i) dz2[nt][i] = F.z2[nt][i] > 0.f ? acc[i] : 0.f;
         }
         __builtin_amdgcn_wave_barrier();
@@ -474,7 +504,7 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
             for (int mt = 0; mt < 4; ++mt)
                 gW2[mt][nt] = mfma16(ld4(&W.a1t[(mt * 16 + lr) * 16 + 4 * lg]), bz, gW2[mt][nt]);
             gb2[nt] += dz2[nt][0] + dz2[nt][1] + dz2[nt][2] + dz2[nt][3];
-            for (int i = 0; i < 4; ++i) W.dz[(4 * lg + i) * NH + nt * 16 + lr] = to_bf16(dz2[nt][i]);
+            put4(W.dz, nullptr, lg, nt * 16 + lr, bz);
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
@@ -482,8 +512,8 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
         for (int nt = 0; nt < 4; ++nt) {
             f32x4 acc = {0.f, 0.f, 0.f, 0.f};
             for (int kc = 0; kc < 4; ++kc)
-                acc = mfma16(ld4(&W.dz[lr * NH + kc * 16 + 4 * lg]),
-                             ld4(&S.w2[(nt * 16 + lr) * NH + kc * 16 + 4 * lg]), acc);
+                acc = mfma16(ld4(&W.dz[lr * NP + kc * 16 + 4 * lg]),
+                             ld4(&S.w2[(nt * 16 + lr) * NP + kc * 16 + 4 * lg]), acc);
             f32x4 dz1;
             for (int i = 0; i < 4; ++i) dz1[i] = F.z1[nt][i] > 0.f ? acc[i] : 0.f;
             gW1[nt] = mfma16(ld4(&W.xt[lr * 16 + 4 * lg]), pack4(dz1), gW1[nt]);
@@ -492,41 +522,71 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const float *__restrict__
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
     }
-    // Bias and w4 sums: reduce over the four lane groups (same unit l%16).
+    // Bias and w4 sums over the four lane groups (same unit l%16), the loss over
+    // them too.
     auto grp = [](float v) {
         v += __shfl_xor(v, 16, 64);
         v += __shfl_xor(v, 32, 64);
         return v;
     };
     for (int nt = 0; nt < 4; ++nt) {
-        const float a = grp(gb1[nt]), b = grp(gb2[nt]), c = grp(gb3[nt]), d = grp(gw4[nt]);
-        if (lg == 0) {
-            atomicAdd(&grad[P_B1 + nt * 16 + lr], a);
-            atomicAdd(&grad[P_B2 + nt * 16 + lr], b);
-            atomicAdd(&grad[P_B3 + nt * 16 + lr], c);
-            atomicAdd(&grad[P_W4 + nt * 16 + lr], d);
-        }
+        gb1[nt] = grp(gb1[nt]);
+        gb2[nt] = grp(gb2[nt]);
+        gb3[nt] = grp(gb3[nt]);
+        gw4[nt] = grp(gw4[nt]);
     }
-    float gb4s = gb4;
-    gb4s += __shfl_xor(gb4s, 16, 64);
-    gb4s += __shfl_xor(gb4s, 32, 64);
-    if (l == 0) atomicAdd(&grad[P_B4], gb4s);
-    // Weight tiles: lane holds dW[mt*16 + 4*lg + i][nt*16 + lr].
-    for (int nt = 0; nt < 4; ++nt) {
-        for (int i = 0; i < 4; ++i) {
-            const int in = 4 * lg + i, out = nt * 16 + lr;
-            atomicAdd(&grad[P_W1 + in * NH + out], gW1[nt][i]);
-            for (int mt = 0; mt < 4; ++mt) {
-                const int in2 = mt * 16 + 4 * lg + i;
-                atomicAdd(&grad[P_W2 + in2 * NH + out], gW2[mt][nt][i]);
-                atomicAdd(&grad[P_W3 + in2 * NH + out], gW3[mt][nt][i]);
+    gb4 = grp(gb4);
+    lsum = grp(lsum) * inv_total;
+    // Half of the waves' sums in each of two copies, a wave after the other:
+    // the first writes, the others add.
+    for (int round = 0; round < GRAD_WAVES / 2; ++round) {
+        __syncthreads();  // (first: every wave is done with its tiles)
+        const int w = (int)(threadIdx.x >> 6) - 2 * round;
+        if (w != 0 && w != 1) continue;
+        float *o = G.sum[w];
+        auto add = [&](int at, float v) { o[at] = round ? o[at] + v : v; };
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                add((nt * 4 + i) * 64 + l, gW1[nt][i]);
+#pragma unroll
+                for (int mt = 0; mt < 4; ++mt) {
+                    add((16 + (mt * 4 + nt) * 4 + i) * 64 + l, gW2[mt][nt][i]);
+                    add((80 + (mt * 4 + nt) * 4 + i) * 64 + l, gW3[mt][nt][i]);
+                }
+            }
+        if (lg == 0) {
+            for (int nt = 0; nt < 4; ++nt) {
+                add(GRAD_TILES + nt * 16 + lr, gb1[nt]);
+                add(GRAD_TILES + NH + nt * 16 + lr, gb2[nt]);
+                add(GRAD_TILES + 2 * NH + nt * 16 + lr, gb3[nt]);
+                add(GRAD_TILES + 3 * NH + nt * 16 + lr, gw4[nt]);
             }
         }
+        if (l == 0) {
+            add(GRAD_TILES + 4 * NH, gb4);
+            add(GRAD_TILES + 4 * NH + 1, lsum);
+        }
     }
-    float ls = lsum;
-    ls += __shfl_xor(ls, 16, 64);
-    ls += __shfl_xor(ls, 32, 64);
-    if (l == 0) atomicAdd(loss, ls * inv_total);
+    __syncthreads();
+    for (int at = threadIdx.x; at < GRAD_SUMS; at += blockDim.x) {
+        const float v = G.sum[0][at] + G.sum[1][at];
+        if (at < GRAD_TILES) {
+            // tile register r of lane `lane` holds dW[mt*16 + 4*(lane/16) + i][nt*16 + lane%16]
+            const int r = at >> 6, lane = at & 63;
+            const int base = r < 16 ? P_W1 : (r < 80 ? P_W2 : P_W3);
+            const int q = r < 16 ? r : (r < 80 ? r - 16 : r - 80);
+            const int row = (q >> 4) * 16 + 4 * (lane >> 4) + (q & 3);
+            atomicAdd(&grad[base + row * NH + ((q >> 2) & 3) * 16 + (lane & 15)], v);
+        } else if (at < GRAD_TILES + 4 * NH + 1) {
+            const int j = at - GRAD_TILES;
+            const int base = j < NH ? P_B1 : (j < 2 * NH ? P_B2 : (j < 3 * NH ? P_B3 : P_W4));
+            atomicAdd(&grad[j < 4 * NH ? base + (j & (NH - 1)) : P_B4], v);
+        } else {
+            atomicAdd(loss, v);
+        }
+    }
 }
 
 // Adam on the fp32 master weights.  The padded input rows of W1 stay zero.
@@ -545,9 +605,11 @@ __global__ void adam_kernel(float *__restrict__ prm, const float *__restrict__ g
     prm[i] -= lr * (mi * c1) / (sqrtf(vi * c2) + eps);
 }
 
-__global__ void zero_f32_kernel(float *p, int n) {
+// Clears a gradient and its loss (they may lie apart).
+__global__ void zero_grad_kernel(float *grad, float *loss) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.f;
+    if (i < NPARAM) grad[i] = 0.f;
+    else if (i == NPARAM) loss[0] = 0.f;
 }
 
 }  // namespace ft
@@ -654,12 +716,11 @@ int ft_mlp_grad(ft_stream s, ft_mlp *mdl, const float *features, const float *ta
                 float *grad, float *loss) {
     if (!mdl) return fail(FT_EINVAL, "null model");
     const hipStream_t hs = as_stream(s);
-    hipLaunchKernelGGL(zero_f32_kernel, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, hs, grad,
-                       NPARAM);
-    hipLaunchKernelGGL(zero_f32_kernel, dim3(1), dim3(64), 0, hs, loss, 1);
+    hipLaunchKernelGGL(zero_grad_kernel, dim3((NPARAM + 1 + 255) / 256), dim3(256), 0, hs, grad,
+                       loss);
     if (n > 0) {
-        const int blocks = std::min((n + 63) / 64, 1024);
-        hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(256), 0, hs,
+        const int blocks = std::min((n + 16 * GRAD_WAVES - 1) / (16 * GRAD_WAVES), GRAD_BLOCKS);
+        hipLaunchKernelGGL(mlp_grad_kernel, dim3(blocks), dim3(64 * GRAD_WAVES), 0, hs,
                            (const float *)mdl->prm, (const float *)mdl->norm, features, target,
                            n, 1.0f / (float)n, grad, loss);
     }

@@ -36,3 +36,29 @@ def test_build_histogram_grid(ft, orc, n):
     got = tree.to_host()
     assert np.array_equal(got["sorted_keys"], keys[order])
     assert np.array_equal(got["orig_idx"][n - 1:], order.astype(np.int32))
+
+
+# 16 samples a tile, 8 waves a block, 256 blocks: part of a tile, a tile and one
+# sample, a block and one tile, more tiles than waves (a wave takes two)
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 128, 129, 4096, 32_768, 32_785, 65_537])
+def test_gradient_sample_counts(ft, n):
+    """Against the float64 oracle with the same bf16 roundings.  The products'
+    operands agree exactly up to activations that fall on the other side of a
+    bf16 rounding step (2^-9 relative, a few of them per sum), so the gradient
+    is held to 1 % of its largest component and the loss to 1e-3."""
+    from fasttree_amd import learned as L
+    from oracle import mlp as M
+
+    rng = np.random.default_rng(n)
+    f = np.zeros((n, 16), np.float32)
+    f[:, :12] = rng.normal(size=(n, 12)) * 3 + 5
+    y = (f[:, 0] * 0.5 + rng.normal(size=n)).astype(np.float32)
+    p = L.init_params(n)
+    p[9408:9472] *= 10  # an output layer whose gradient reaches the lower layers
+    norm = L.norm_from(f, y) if n > 1 else L.default_norm()
+    m = L.MLP(p, norm, 0.0)
+    g, loss = m.grad(ft.DeviceArray.from_host(f.ravel()), ft.DeviceArray.from_host(y), n)
+    el, eg = M.loss_and_grad(p, norm.astype(np.float64), f, y, rounding=True)
+    assert abs(loss - el) <= 1e-3 * el + 1e-7
+    assert np.abs(g - eg).max() <= 1e-2 * np.abs(eg).max()
+    assert not g[9473:].any()
