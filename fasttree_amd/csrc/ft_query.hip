@@ -31,17 +31,33 @@ int radix_sort_u64(hipStream_t s, Scratch &S, const uint64_t *keys_in, size_t n,
 // ===========================================================================
 // Query positions.  A "slot" is a position in the launch's query order; the
 // query it holds is order[slot] (external queries sorted along the curve) or
-// the slot itself.  Results are written at the query's own row.  Re-run lists
-// hold slots in ascending order (compacted from per-slot flags), so a listed
-// pass walks its queries in curve order too.
+// the slot itself.  Results are written at the query's own row.  A direct pass
+// appends the slots it leaves unanswered to a list that a listed pass takes.
 // ===========================================================================
 struct QueryMap {
-    const uint32_t *order;      // slot -> query (null: identity)
-    const int32_t *list;        // LISTED: slots to run (-1: already answered)
-    const uint32_t *list_count; // LISTED: number of list entries (device)
-    uint8_t *redo;              // direct passes: per-slot flag, set when the slot
-                                // must be re-run exactly
+    const uint32_t *order;  // slot -> query (null: identity)
+    int32_t *list;          // direct passes: slots left to the listed pass, appended;
+                            // LISTED: the slots to run
+    uint32_t *count;        // [0] list entries, [1] those that count as exact re-runs
 };
+
+// Appends the wave's slots with `left` set, one atomic per wave.  `rerun`: they
+// count as exact re-runs (a query the direct pass could not answer exactly,
+// rather than a packet handed over).  Called by whole waves.
+__device__ inline void append_slots(const QueryMap &qm, bool left, int slot, bool rerun) {
+    const uint64_t m = __ballot(left);
+    if (!m) return;
+    const int lane = threadIdx.x & 63;
+    uint32_t base = 0;
+    if (lane == 0) {
+        base = atomicAdd(&qm.count[0], (uint32_t)__popcll(m));
+        if (rerun) atomicAdd(&qm.count[1], (uint32_t)__popcll(m));
+    }
+    base = (uint32_t)uni((int)base);
+    if (left)
+        qm.list[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = slot;
+}
 
 __device__ inline int slot_query(const QueryMap &qm, int slot) {
     return qm.order ? (int)qm.order[slot] : slot;
@@ -49,65 +65,31 @@ __device__ inline int slot_query(const QueryMap &qm, int slot) {
 
 // ===========================================================================
 // Per-lane DFS with the canonical register top-k (k <= M <= 32): the
-// reference's grouped self-kNN / knn_query_small_k walk on wave64 lanes.
-// Direct passes use the reference's 64-entry stack and flag a query whose
-// walk would need more; LISTED passes (the exact re-runs) use 128 entries,
-// and for self queries first insert the leaves within LISTED_WINDOW ranks of
-// the query's own leaf, so that the walk starts with a finite bound and skips
-// those leaves (the top-k set does not depend on the order of insertion).
+// reference's grouped self-kNN / knn_query_small_k walk on wave64 lanes, with
+// the reference's 64-entry stack.  A query whose walk would need more is left
+// to the listed pass.
 // ===========================================================================
-constexpr int LISTED_WINDOW = 32;
-
-template <typename T, int M, bool GROUPED, bool LISTED, int MK>
+template <typename T, int M, bool GROUPED, int MK>
 __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_reg_kernel(
     DTree<T> t, QSrc<T> qs, int nq, int k, int excl, QueryMap qm, uint64_t *__restrict__ res,
     typename CoordTraits<T>::D *__restrict__ dists, uint64_t *__restrict__ stats) {
     using D = typename CoordTraits<T>::D;
-    constexpr int DEPTH = LISTED ? LANE_STACK_CANON : STACK_DEPTH;
-    __shared__ int32_t stk[DEPTH * LANE_BLOCK];
+    __shared__ int32_t stk[STACK_DEPTH * LANE_BLOCK];
     const int lane = threadIdx.x;
-    const int nlist = LISTED ? (int)*qm.list_count : nq;
     uint64_t visits = 0, inserts = 0;
-    for (int base = (LISTED ? (int)blockIdx.x : xcd_block()) * LANE_BLOCK; base < nlist;
-         base += (LISTED ? gridDim.x * LANE_BLOCK : nlist)) {
-        const int pos = base + lane;
-        const int lslot = (LISTED && pos < nlist) ? qm.list[pos] : 0;
-        const bool active = pos < nlist && (!LISTED || lslot >= 0);
-        const int slot = active ? (LISTED ? lslot : pos) : 0;
-        const int q = active ? slot_query(qm, slot) : 0;
-        T px = T(0), py = T(0), pz = T(0);
-        int self = -1;
-        if (active) load_query(t, qs, q, px, py, pz, self);
-        if (!excl) self = -1;
-        TopK<D, M> h;
-        h.init(k, dist_max<D>());
-        int wlo = 0, whi = 0;
-        if constexpr (LISTED) {
-            if (active && self >= 0) {
-                const int off = t.n - 1;
-                wlo = self - LISTED_WINDOW > 0 ? self - LISTED_WINDOW : 0;
-                whi = self + LISTED_WINDOW + 1 < t.n ? self + LISTED_WINDOW + 1 : t.n;
-                for (int r = wlo; r < whi; ++r) {
-                    if (r == self) continue;
-                    const int leaf = off + r;
-                    const D d2 = leaf_d2_k<T, MK>(t.m, px, py, pz, t.mnx[leaf], t.mny[leaf],
-                                                  t.mnz[leaf]);
-                    const int32_t ri = ret_index(t, leaf);
-                    const bool take = h.beats_worst(d2, ri);
-                    h.insert(take, d2, ri);
-                    inserts += take ? 1 : 0;
-                }
-            }
-        }
-        const bool ovf = lane_reg_walk<T, M, GROUPED, DEPTH, MK>(t, active, px, py, pz, self, h,
-                                                                 stk, LANE_BLOCK, lane, visits,
-                                                                 inserts, wlo, whi);
-        if (active) {
-            if (!LISTED && ovf) qm.redo[slot] = 1;
-            else h.store(k, res, dists, (size_t)q);
-        }
-        if (!LISTED) break;
-    }
+    const int slot = xcd_block() * LANE_BLOCK + lane;
+    const bool active = slot < nq;
+    const int q = active ? slot_query(qm, slot) : 0;
+    T px = T(0), py = T(0), pz = T(0);
+    int self = -1;
+    if (active) load_query(t, qs, q, px, py, pz, self);
+    if (!excl) self = -1;
+    TopK<D, M> h;
+    h.init(k, dist_max<D>());
+    const bool ovf = lane_reg_walk<T, M, GROUPED, STACK_DEPTH, MK>(
+        t, active, px, py, pz, self, h, stk, LANE_BLOCK, lane, visits, inserts);
+    if (active && !ovf) h.store(k, res, dists, (size_t)q);
+    append_slots(qm, active && ovf, slot, true);
     wave_add_stats(stats, 0, visits);
     wave_add_stats(stats, 4, inserts);
 }
@@ -129,14 +111,13 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_lds_kernel(
     int32_t *stk = hi + (size_t)k * lanes;              // [DEPTH][lanes]
     const int lane = threadIdx.x;
     const bool lane_ok = lane < lanes;
-    const int nlist = LISTED ? (int)*qm.list_count : nq;
+    const int nlist = LISTED ? (int)qm.count[0] : nq;
     uint64_t visits = 0, drops = 0, inserts = 0;
     for (int base = (LISTED ? (int)blockIdx.x : xcd_block()) * lanes; base < nlist;
          base += (LISTED ? gridDim.x * lanes : nlist)) {
         const int pos = base + lane;
-        const int lslot = (LISTED && lane_ok && pos < nlist) ? qm.list[pos] : 0;
-        const bool active = lane_ok && pos < nlist && (!LISTED || lslot >= 0);
-        const int slot = active ? (LISTED ? lslot : pos) : 0;
+        const bool active = lane_ok && pos < nlist;
+        const int slot = active ? (LISTED ? qm.list[pos] : pos) : 0;
         const int q = active ? slot_query(qm, slot) : 0;
         T px = T(0), py = T(0), pz = T(0);
         int self = -1;
@@ -145,10 +126,9 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_lds_kernel(
         LdsHeap<D, REF> h{hd, hi, lanes, lane, 0};
         const bool ovf = lane_heap_walk<T, REF, GROUPED, DEPTH, MK>(
             t, k, active, px, py, pz, self, h, stk, lanes, lane, visits, drops, inserts);
+        const bool left = active && !REF && !LISTED && ovf;
         if (active) {
-            if (!REF && !LISTED && ovf) {
-                qm.redo[slot] = 1;
-            } else {
+            if (!left) {
                 h.sort();
                 const size_t o = (size_t)q * k;
                 for (int s = 0; s < k; ++s) {
@@ -158,6 +138,7 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_lds_kernel(
                 }
             }
         }
+        if constexpr (!REF && !LISTED) append_slots(qm, left, slot, true);
         if (!LISTED) break;
     }
     wave_add_stats(stats, 0, visits);
@@ -296,14 +277,16 @@ __global__ __launch_bounds__(64) void merge_knn_kernel(DTree<T> t, QSrc<T> qs, i
 // Packet traversal: a wavefront of 64 queries (consecutive slots) shares one
 // DFS (packet_walk).  Results are canonical.
 // SEEDED: each lane's k-th distance starts at its seed bound; a lane that ends
-// with fewer than k neighbours inside the seed flags its slot for an exact
+// with fewer than k neighbours inside the seed leaves its slot for an exact
 // re-run.  PACKED: 64-bit (d2, index) keys; queries the packed form cannot
-// order exactly are flagged too.  The re-run (launch_exact_listed) takes the
-// compacted list of flagged slots, unseeded and lexicographic, so exact.
+// order exactly are left too, and so are all queries of a packet whose walk
+// passes its budget.  The listed pass (launch_listed) answers the slots left,
+// unseeded and lexicographic, so exact.
 // ===========================================================================
 struct PacketArgs {
     int nq, k, excl, bucket, ibits;
     int width;   // queries per packet (16, 32 or 64): lanes at or above it idle
+    uint32_t stop;  // leaves a packet may scan before its queries are handed over
     int window;  // self queries over all leaves: leaves pre-scanned on each side
     uint64_t *stats;
 };
@@ -320,25 +303,20 @@ struct PacketArgs {
 // anchor their first leaves at their own rank, external ones at the leaf a
 // greedy descent reaches.
 //
-// LISTED: the first step of the exact re-run of a direct pass's flagged
-// slots (qm.list, *qm.list_count).  The waves take list entries in turn, and
-// an entry whose query they answer is set to -1 in done_list (the list
-// itself), so the per-lane re-run that follows takes only the entries whose
-// walk would overflow the wave's stack (none for a tree this library built).
+// LISTED: the slots that a direct pass left (qm.list, qm.count[0] of them);
+// the waves take list entries in turn.
 // ===========================================================================
 template <typename T, int S, int MK, bool LISTED = false>
 __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, int nq, int k,
                                                        int excl, QueryMap qm,
                                                        uint64_t *__restrict__ res,
                                                        typename CoordTraits<T>::D *__restrict__ dists,
-                                                       uint64_t *__restrict__ stats,
-                                                       int32_t *__restrict__ done_list) {
+                                                       uint64_t *__restrict__ stats) {
     __shared__ WaveBuf wbuf[4];
     const int lane = threadIdx.x & 63;
     const int wave = uni(xcd_block() * 4 + (int)(threadIdx.x >> 6));
     WaveCounters c;
-    // Answers the query of one slot; false if its walk would overflow.
-    auto answer = [&](int slot) -> bool {
+    auto answer = [&](int slot) {
         const int q = uni(slot_query(qm, slot));
         T px = T(0), py = T(0), pz = T(0);
         int rank = -1;
@@ -347,17 +325,14 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
         const int anchor = rank >= 0 ? rank : descend_rank_v<T, MK>(t, px, py, pz);
         WaveList<S> L;
         L.init(k);
-        if (wave_walk<T, S, MK>(t, px, py, pz, self, anchor, L, c, &wbuf[threadIdx.x >> 6]))
-            return false;
+        wave_walk<T, S, MK>(t, px, py, pz, self, anchor, L, c, &wbuf[threadIdx.x >> 6]);
         L.store(k, res, dists, (size_t)q, lane);
-        return true;
     };
     if constexpr (LISTED) {
-        const int cnt = (int)*qm.list_count;
-        for (int e = wave; e < cnt; e += (int)gridDim.x * 4)
-            if (answer(uni(qm.list[e])) && lane == 0) done_list[e] = -1;
+        const int cnt = (int)qm.count[0];
+        for (int e = wave; e < cnt; e += (int)gridDim.x * 4) answer(uni(qm.list[e]));
     } else if (wave < nq) {
-        if (!answer(wave) && lane == 0) qm.redo[wave] = 1;
+        answer(wave);
     }
     if (stats) {  // one atomic per block and counter: a wave per query would contend
         __shared__ unsigned long long s_st[3];
@@ -375,11 +350,11 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
     }
 }
 
-// Packed-key packets: at least 4 waves per SIMD (128 VGPRs).  The k = 32
-// kernel spills 72 bytes and still runs 11 % faster than at 3 waves (144
-// VGPRs); the passes of 32 for k = 64 run 19 % faster than at 2 waves.  Double
-// coordinates keep their natural 3 waves (forcing 4 spilled 116 bytes and was
-// 32 % slower).
+// Packed-key packets: at least 4 waves per SIMD (128 VGPRs), 11 % faster than
+// 3 at k = 32 and 19 % in the passes of 32 for k = 64, spills included.  With
+// the walk's counters in 32 bits the k = 32 kernel spills nothing (72 bytes a
+// lane before: 10M clustered points 16.9 -> 16.7 ms).  Double coordinates keep
+// their natural 3 waves (forcing 4 spilled 116 bytes and was 32 % slower).
 template <typename T, int M, bool HEAP, bool SEEDED, bool PACKED, int MK, bool MULTI = false>
 __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     DTree<T> t, QSrc<T> qs, PacketArgs a, QueryMap qm,
@@ -444,7 +419,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             else h.init(kk, (SEEDED && active) ? seed[qv] : dist_max<D>());
             // one walk instance for every pass (the first with no floor)
             packet_walk<T, H, MK, true>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo,
-                                        whi, r0, lo);
+                                        whi, r0, lo, 0, 0, a.stop);
             if (active) {
                 bool r = false;
                 if constexpr (PACKED) r = h.needs_exact(kk);
@@ -454,7 +429,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             }
             lo = h.next_floor();
         }
-        if (active && redo) qm.redo[slot] = 1;
+        append_slots(qm, active && (redo || c.leaves > a.stop), slot, c.leaves <= a.stop);
     } else {
         H h;
         if constexpr (HEAP) h.key = heap_mem;
@@ -466,19 +441,20 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             // window (>= 32 leaves on each side) covers every filled rank
             if (!qs.qx && !qs.leaf_ids && a.window >= 32) {
                 __shared__ FillStage<T> fst;
-                c.inserts += (uint64_t)fill_from_run<T, MK>(t, h, k, active, self >= 0, rank, px,
+                c.inserts += (uint32_t)fill_from_run<T, MK>(t, h, k, active, self >= 0, rank, px,
                                                             py, pz, r0, &fst, flo, fhi);
             }
         }
         packet_walk<T, H, MK>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo, whi, r0,
-                              H::no_floor(), flo, fhi);
+                              H::no_floor(), flo, fhi, a.stop);
+        bool left = false;
         if (active) {
-            bool redo = false;
-            if constexpr (PACKED) redo = h.needs_exact(k);
-            else if constexpr (SEEDED) redo = h.missing(k) > 0;
-            if (redo) qm.redo[slot] = 1;
-            else h.store(k, res, dists, (size_t)q);
+            left = c.leaves > a.stop;
+            if constexpr (PACKED) left = left || h.needs_exact(k);
+            else if constexpr (SEEDED) left = left || h.missing(k) > 0;
+            if (!left) h.store(k, res, dists, (size_t)q);
         }
+        append_slots(qm, left, slot, c.leaves <= a.stop);
     }
     if (lane == 0 && a.stats) {
         atomicAdd((unsigned long long *)&a.stats[0], (unsigned long long)c.nodes);
@@ -858,9 +834,9 @@ template <typename T> static int lds_lanes(int k, int depth, size_t &lds) {
     return lds <= budget ? lanes : 0;
 }
 
-// Per-stream work buffers of the query paths: the re-run buffers (per-slot
-// flags, the compacted slot list, per-tile counts and the list length) and
-// the query-order sort buffers.  Each stream has its own set, grown on
+// Per-stream work buffers of the query paths: the slot list of a direct pass
+// and its counts, flags and per-tile counts of a compaction, and the
+// query-order sort buffers.  Each stream has its own set, grown on
 // demand, so queries on different streams do not share memory; a stream's
 // set is released by ft_stream_destroy / ft_stream_release.
 //
@@ -1003,12 +979,11 @@ static int rerun_ensure(hipStream_t s, size_t n) {
     return FT_OK;
 }
 
-__global__ void fill_u8_kernel(uint8_t *p, size_t n) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (size_t)gridDim.x * blockDim.x)
-        p[i] = 0;
+// Starts a direct pass's list (QueryMap::count).
+__global__ void zero_counts_kernel(uint32_t *count) {
+    if (threadIdx.x < 2) count[threadIdx.x] = 0;
 }
-__global__ void add_count_kernel(uint64_t *stats, const uint32_t *count) { stats[3] += *count; }
+__global__ void add_count_kernel(uint64_t *stats, const uint32_t *count) { stats[3] += count[1]; }
 
 static inline int bit_length(uint64_t v) {
     int b = 0;
@@ -1043,33 +1018,23 @@ static int compact_flags(hipStream_t s, const RerunBuf &g_rerun, int n) {
         else { constexpr int M = 32; __VA_ARGS__; }                 \
     } while (0)
 
-// Exact re-run of the listed slots.  Up to k = 128, one wave per listed query
-// first (the wave-per-query tier, LISTED); it marks the entries it answers.
-// Then the per-lane walk with a 128-entry stack, unseeded, lexicographic top-k
-// (registers for k <= 32, LDS heap above), over the entries left.  The flagged
-// queries of a seeded pass are few and scattered (0.2 % of C2's 10M): one
-// lane each left the re-run latency-bound on a few hundred waves, 1.7 ms; one
-// wave each fills the chip.
+// Answers the slots that a direct pass left, exactly: up to k = 128 one wave
+// per listed query (the wave-per-query tier), above that the per-lane heap
+// walk with a 128-entry stack.  One lane per listed query left the 0.2 % of a
+// seeded 10M-query pass latency-bound on a few hundred waves (1.7 ms against
+// 0.3 ms with one wave each).
 template <typename T, int MK>
-static int launch_exact_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq,
-                               int k, int excl, const uint32_t *order, const RerunBuf &g_rerun,
-                               uint64_t *res, typename CoordTraits<T>::D *d) {
-    const QueryMap qm{order, g_rerun.list, g_rerun.count, nullptr};
+static int launch_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq, int k,
+                         int excl, const QueryMap &qm, uint64_t *res,
+                         typename CoordTraits<T>::D *d) {
     if (k <= 128) {
         const dim3 g(xcd_grid(std::min<unsigned>(blocks_for(nq, 4), 2048u))), b(256);
         if (k <= 64)
             hipLaunchKernelGGL((wave_knn_kernel<T, 1, MK, true>), g, b, 0, s, dt, qs, nq, k, excl,
-                               qm, res, d, (uint64_t *)nullptr, g_rerun.list);
+                               qm, res, d, (uint64_t *)nullptr);
         else
             hipLaunchKernelGGL((wave_knn_kernel<T, 2, MK, true>), g, b, 0, s, dt, qs, nq, k, excl,
-                               qm, res, d, (uint64_t *)nullptr, g_rerun.list);
-        FT_CHECK_LAUNCH();
-    }
-    if (k <= 32) {
-        const unsigned g = std::min<unsigned>(blocks_for(nq, LANE_BLOCK), 2048u);
-        FT_BY_M(k, hipLaunchKernelGGL((lane_knn_reg_kernel<T, M, true, true, MK>), dim3(g),
-                                      dim3(LANE_BLOCK), 0, s, dt, qs, nq, k, excl, qm, res, d,
-                                      (uint64_t *)nullptr));
+                               qm, res, d, (uint64_t *)nullptr);
     } else {
         size_t lds = 0;
         const int lanes = lds_lanes<T>(k, LANE_STACK_CANON, lds);
@@ -1109,10 +1074,10 @@ static void launch_packet_m(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs
     else launch_pk<T, M, HEAP, false, INTD, MK>(s, dt, qs, a, qm, seed, res, d);
 }
 
-// One canonical query launch: a direct pass (packet or per-lane walk) that
-// flags the slots it cannot answer exactly (packed keys that saturate, seeds
-// that were too small, per-lane stacks that would overflow), compaction of
-// the flags, and the exact listed re-run.  No host round trip.
+// One canonical query launch: a direct pass, and where it can leave slots
+// unanswered (packed keys that saturate, seeds that were too small, per-lane
+// stacks that would overflow) the listed pass over the slots it appended.  No
+// host round trip.  The wave tier answers every query itself.
 template <typename T, int MK>
 static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq, int k,
                          int excl, int algo, int bucket, int topk, int window, int width,
@@ -1120,14 +1085,17 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
                          const typename CoordTraits<T>::D *seed, uint64_t *res,
                          typename CoordTraits<T>::D *d, uint64_t *stats, const RerunBuf *rr) {
     constexpr bool INTD = !CoordTraits<T>::fp;
-    if (!rr) {  // the stream's own re-run buffers, grown to nq
-        FT_TRY(rerun_ensure(s, (size_t)nq));
-        rr = &stream_bufs(s).rr;
+    const uint32_t stop = ~0u;
+    const bool leaves_slots = algo == FT_ALGO_PACKET ? (INTD || seed || stop != ~0u)
+                                                     : algo != FT_ALGO_WAVE;
+    if (leaves_slots) {
+        if (!rr) {  // the stream's own buffers, grown to nq
+            FT_TRY(rerun_ensure(s, (size_t)nq));
+            rr = &stream_bufs(s).rr;
+        }
+        hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, s, rr->count);
     }
-    const RerunBuf &g_rerun = *rr;
-    hipLaunchKernelGGL(fill_u8_kernel, dim3(std::min<unsigned>(blocks_for(nq, 256), 4096u)),
-                       dim3(256), 0, s, g_rerun.flags, (size_t)nq);
-    const QueryMap qm{order, nullptr, nullptr, g_rerun.flags};
+    const QueryMap qm{order, leaves_slots ? rr->list : nullptr, leaves_slots ? rr->count : nullptr};
     if (algo == FT_ALGO_PACKET) {
         PacketArgs a{};
         a.nq = nq;
@@ -1142,6 +1110,7 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         // 114.7 / 112.7 / 111.9 / 113.8 ms).
         const int spread = qs.leaf_ids ? (int)std::min<int64_t>(4, std::max<int64_t>(1, dt.n / std::max(nq, 1))) : 1;
         a.window = window * spread;
+        a.stop = stop;
         a.stats = stats;
         // k above 32 with integer coordinates: multi-pass register tier by
         // default, LDS heap tiers on request.
@@ -1158,7 +1127,7 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         const dim3 g(xcd_grid(blocks_for(nq, 4))), b(256);
 #define FT_WAVE_LAUNCH(S_)                                                                      \
     hipLaunchKernelGGL((wave_knn_kernel<T, S_, MK>), g, b, 0, s, dt, qs, nq, k, excl, qm, res, d, \
-                       stats, (int32_t *)nullptr)
+                       stats)
         if (k <= 64) FT_WAVE_LAUNCH(1);
         else if (k <= 128) FT_WAVE_LAUNCH(2);
         else if (k <= 256) FT_WAVE_LAUNCH(4);
@@ -1169,10 +1138,10 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     } else if (k <= 32) {
         const dim3 g(xcd_grid(blocks_for(nq, LANE_BLOCK))), b(LANE_BLOCK);
         if (algo == FT_ALGO_PLAIN)
-            FT_BY_M(k, hipLaunchKernelGGL((lane_knn_reg_kernel<T, M, false, false, MK>), g, b, 0, s,
+            FT_BY_M(k, hipLaunchKernelGGL((lane_knn_reg_kernel<T, M, false, MK>), g, b, 0, s,
                                           dt, qs, nq, k, excl, qm, res, d, stats));
         else
-            FT_BY_M(k, hipLaunchKernelGGL((lane_knn_reg_kernel<T, M, true, false, MK>), g, b, 0, s,
+            FT_BY_M(k, hipLaunchKernelGGL((lane_knn_reg_kernel<T, M, true, MK>), g, b, 0, s,
                                           dt, qs, nq, k, excl, qm, res, d, stats));
     } else {
         size_t lds = 0;
@@ -1187,13 +1156,13 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
                                qs, nq, k, excl, lanes, qm, res, d, stats);
     }
     FT_CHECK_LAUNCH();
-    FT_TRY(compact_flags(s, g_rerun, nq));
+    if (!leaves_slots) return FT_OK;
     if (stats) {
         hipLaunchKernelGGL(add_count_kernel, dim3(1), dim3(1), 0, s, stats,
-                           (const uint32_t *)g_rerun.count);
+                           (const uint32_t *)rr->count);
         FT_CHECK_LAUNCH();
     }
-    return launch_exact_listed<T, MK>(s, dt, qs, nq, k, excl, order, g_rerun, res, d);
+    return launch_listed<T, MK>(s, dt, qs, nq, k, excl, qm, res, d);
 }
 
 template <typename T>
@@ -1256,7 +1225,7 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
         size_t lds = 0;
         const int lanes = lds_lanes<T>(k, STACK_DEPTH, lds);
         if (!lanes) return fail(FT_ELDS, "k too large for local memory: reduce k");
-        const QueryMap qm{nullptr, nullptr, nullptr, nullptr};
+        const QueryMap qm{nullptr, nullptr, nullptr};
         const dim3 g(xcd_grid(blocks_for(nq, lanes))), b(LANE_BLOCK);
         if (algo == FT_ALGO_PLAIN)
             hipLaunchKernelGGL((lane_knn_lds_kernel<T, true, false, false, MK_ANY>), g, b, lds, s,
@@ -1332,18 +1301,14 @@ int knn_entry(hipStream_t s, const ft_tree *tree, const void *qx, const void *qy
 
 // ---- non-allocating self-kNN (no reference counterpart) ----------------------
 // For callers that cannot allocate (code under graph capture, serving loops):
-// the canonical pipeline's re-run buffers (per-slot flags, the compacted slot
-// list, per-tile counts, the list length) live in one file-scope device array
-// instead of per-stream allocations.  Every call on a device shares that
-// device's copy, which keeps the last call's contents; the flags are cleared
-// by a kernel at the start of each call and the other fields are written
-// before they are read.  Calls that overlap on one device race.
+// the canonical pipeline's slot list and its counts live in one file-scope
+// device array instead of per-stream allocations.  Every call on a device
+// shares that device's copy, which keeps the last call's contents; the counts
+// are cleared by a kernel at the start of each call and list entries are
+// written before they are read.  Calls that overlap on one device race.
 constexpr size_t NA_MAX_QUERIES = (size_t)1 << 24;
-constexpr size_t na_al(size_t x) { return (x + 255) & ~(size_t)255; }
-constexpr size_t NA_OFF_LIST = na_al(NA_MAX_QUERIES);
-constexpr size_t NA_OFF_TILES = NA_OFF_LIST + na_al(NA_MAX_QUERIES * 4);
-constexpr size_t NA_OFF_COUNT = NA_OFF_TILES + na_al((NA_MAX_QUERIES / CP_TILE + 2) * 4);
-constexpr size_t NA_BYTES = NA_OFF_COUNT + 256;  // 80 MiB + 16.5 KiB
+constexpr size_t NA_OFF_COUNT = NA_MAX_QUERIES * 4;
+constexpr size_t NA_BYTES = NA_OFF_COUNT + 256;  // 64 MiB + 256 bytes
 static __device__ __align__(256) uint8_t scratch[NA_BYTES];
 
 constexpr int NA_MAX_DEVICES = 64;
@@ -1380,9 +1345,7 @@ int knn_noalloc_entry(hipStream_t s, const ft_tree *tree, int k, int excl, uint6
     FT_TRY(noalloc_scratch(&p));
     char *c = (char *)p;
     RerunBuf rr;
-    rr.flags = (uint8_t *)c;
-    rr.list = (int32_t *)(c + NA_OFF_LIST);
-    rr.tiles = (uint32_t *)(c + NA_OFF_TILES);
+    rr.list = (int32_t *)c;
     rr.count = (uint32_t *)(c + NA_OFF_COUNT);
     rr.cap = NA_MAX_QUERIES;
     FT_DISPATCH_COORD(tree->coord_type, {

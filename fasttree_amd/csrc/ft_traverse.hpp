@@ -687,12 +687,15 @@ template <int M> struct TopKPacked {
 // from the lane's results (-1: none); inactive lanes take no candidates.
 // [fill_lo, fill_hi): leaf ranks the caller already put into this lane's h
 // (fill_from_run); the window pre-scan skips them.
+// stop: the walk ends, with h unfinished, once c.leaves exceeds it (the lanes'
+// regions have too little in common).
 // ===========================================================================
 constexpr int PK_STACK = 128;
 
+// 32 bits each: one packet's counts, kept in registers through the walk.
 struct PacketCounters {
-    uint64_t nodes = 0, leaves = 0, inserts = 0, overflow = 0;
-    uint64_t rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
+    uint32_t nodes = 0, leaves = 0, inserts = 0, overflow = 0;
+    uint32_t rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
 };
 
 // A 32-bit coordinate's bits, and back (LDS staging of leaf coordinates).
@@ -711,7 +714,8 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
                                             PacketCounters &c, int win_lo = 0, int win_hi = 0,
                                             int win_mid = 0,
                                             typename H::Floor lo = H::no_floor(),
-                                            int fill_lo = 0, int fill_hi = 0) {
+                                            int fill_lo = 0, int fill_hi = 0,
+                                            uint32_t stop = ~0u) {
     using D = typename CoordTraits<T>::D;
     const int lane = threadIdx.x & 63;
     const int n = t.n;
@@ -896,7 +900,7 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
                 cand &= ~(hi_m & ~((1ull << a0) - 1));
             }
         }
-        c.leaves += (uint64_t)cnt;
+        c.leaves += (uint32_t)cnt;
         // One insertion round: each lane takes its lowest remaining candidate.
         // Integer periodic metrics need only the low 32 bits of coordinates.
         auto round = [&]() {
@@ -1019,6 +1023,12 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             }
         }
         if (scan_cnt > 0) scan_range(scan_first, scan_cnt, window);
+        // Over the budget: the walk ends as if nothing were left.  (A branch out
+        // of the loop here made the allocator keep two copies of the list.)
+        if (c.leaves > stop) {
+            sp = 0;
+            next = -1;
+        }
         while (next < 0 && sp > 0) {
             const int cn = uni(stk[--sp]);
             if (__any(active && node_dist(cn) <= node_bound())) next = cn;

@@ -62,3 +62,26 @@ def test_gradient_sample_counts(ft, n):
     assert abs(loss - el) <= 1e-3 * el + 1e-7
     assert np.abs(g - eg).max() <= 1e-2 * np.abs(eg).max()
     assert not g[9473:].any()
+
+
+# 64 queries a packet: slots left by whole, partial and several packets, appended
+# by one atomic per wave; all, some or none of the seeds too small
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 129, 4097])
+@pytest.mark.parametrize("ct", [O.CT_U32, O.CT_F64])
+@pytest.mark.parametrize("share", [0.0, 0.3, 1.0])
+def test_slots_left_to_the_listed_pass(ft, orc, n, ct, share):
+    rng = np.random.default_rng(n)
+    fp = ct == O.CT_F64
+    pts = [rng.integers(0, 1 << 20, n).astype(O.COORD_DTYPES[ct]) for _ in range(3)]
+    k = min(8, n - 1)
+    tree = ft.TreeSoA(n, ct, ft.Config(sfc=O.SFC_PH, bits_per_dim=21))
+    ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(a) for a in pts)), tree)
+    t = O.build_bvh(ct, *pts, sfc=O.SFC_PH, bits=21)
+    rb, db = O.knn_bruteforce(t, k, True)
+    small = rng.random(n) < share
+    seed = np.where(small, 0, np.finfo(np.float64).max if fp else (1 << 60))
+    seed = seed.astype(np.float64 if fp else np.uint64)
+    stats = ft.DeviceArray(8, np.uint64).zero()
+    r, d = ft.self_knn_query(tree, k, seed_bound=ft.DeviceArray.from_host(seed), stats=stats)
+    assert np.array_equal(r, rb) and np.array_equal(d, db)
+    assert stats.to_host()[3] == int(np.sum(seed < db[:, -1]))
