@@ -143,7 +143,8 @@ __host__ __device__ __forceinline__ float wrap_filter_bound_pre(uint64_t w, int 
 __host__ __device__ __forceinline__ float wrap_filter_floor_pre(uint64_t lo, int sh) {
     return (float)lo * (1.0f - 0x1p-20f) * (float)(1ull << (2 * sh));
 }
-// Float32 pre-filter for double coordinates.  With u = 2^-24, coordinates of
+// Float32 pre-filter for double coordinates (and for integers in an open box,
+// whose conversion to float is as exact).  With u = 2^-24, coordinates of
 // magnitude at most M and period L, the float gap of one axis (both points
 // rounded to float, one subtraction, for a periodic metric min(g, fl(L) - g))
 // is within (1 + u) g + E of the double gap g, E = 1.01 u (L + 4M) (periodic)
@@ -198,6 +199,23 @@ __host__ __device__ __forceinline__ float wrap_box_gap_pre(T qm, uint32_t qs, T 
     const float a = __builtin_fabsf((float)(int32_t)(qs - ((uint32_t)lo << sh)));
     const float b = __builtin_fabsf((float)(int32_t)(qs - ((uint32_t)hi << sh)));
     return in ? 0.0f : __builtin_fminf(a, b);
+}
+
+// leaf_d2 of float coordinates before it is widened to double.
+template <int MK>
+__host__ __device__ __forceinline__ float leaf_f32(const Metric &m, float px, float py, float pz, float x,
+                                          float y, float z) {
+    float dx = fabsf(px - x), dy = fabsf(py - y), dz = fabsf(pz - z);
+    if constexpr (MK == MK_WRAP) {
+        const float L = (float)m.box;
+        dx = fminf(dx, L - dx);
+        dy = fminf(dy, L - dy);
+        dz = fminf(dz, L - dz);
+    }
+    float s = dx * dx;
+    s = s + dy * dy;
+    s = s + dz * dz;
+    return s;
 }
 
 // leaf_d2 / box_d2 with the metric kind fixed (same values).
@@ -698,16 +716,6 @@ struct PacketCounters {
     uint32_t rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
 };
 
-// A 32-bit coordinate's bits, and back (LDS staging of leaf coordinates).
-template <typename T> __device__ __forceinline__ uint32_t bits32(T v) {
-    if constexpr (std::is_same<T, float>::value) return __float_as_uint(v);
-    else return (uint32_t)v;
-}
-template <typename T> __device__ __forceinline__ T from_bits32(uint32_t b) {
-    if constexpr (std::is_same<T, float>::value) return __uint_as_float(b);
-    else return (T)b;
-}
-
 template <typename T, typename H, int MK, bool FLOOR = false>
 __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
                                             T pz, int self, H &h, int32_t *stk,
@@ -750,22 +758,27 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             qmz = pz & mask;
         }
     }
-    // Double coordinates: the float32 leaf pre-filter (fpf_*), with E from
-    // the largest coordinate magnitude of the root box and the query.  Not in
-    // multi-pass walks (FLOOR): there its registers would push the kernel to
-    // one wave per SIMD.
-    constexpr bool FPF = std::is_same<T, double>::value && MK != MK_ANY && !FLOOR;
+    // Double coordinates, and integers in an open box: the float32 leaf
+    // pre-filter (fpf_*), with E from the largest coordinate magnitude of the
+    // root box and the query.  Not for doubles in multi-pass walks (FLOOR):
+    // there its registers would push the kernel to one wave per SIMD.
+    constexpr bool IPF = !CoordTraits<T>::fp && MK == MK_OPEN;
+    constexpr bool FPF = IPF || (std::is_same<T, double>::value && MK != MK_ANY && !FLOOR);
     [[maybe_unused]] float fqx = 0.f, fqy = 0.f, fqz = 0.f, fL = 0.f;
     [[maybe_unused]] double fE = 0.0;
+    // an integer gap is shifted down by dshift: the filter works in those units
+    [[maybe_unused]] const float fs = IPF ? 1.0f / (float)(1ull << t.m.dshift) : 1.0f;
     if constexpr (FPF) {
-        fqx = (float)px;
-        fqy = (float)py;
-        fqz = (float)pz;
-        const double mr = fmax(fmax(fmax(fabs(t.mnx[0]), fabs(t.mxx[0])),
-                                    fmax(fabs(t.mny[0]), fabs(t.mxy[0]))),
-                               fmax(fabs(t.mnz[0]), fabs(t.mxz[0])));
-        const double mq = fmax(fabs(px), fmax(fabs(py), fabs(pz)));
-        fE = fpf_err(fmax(mr, mq), (double)t.m.box, MK == MK_WRAP);
+        fqx = (float)px * fs;
+        fqy = (float)py * fs;
+        fqz = (float)pz * fs;
+        auto mag = [](T v) { return fabs((double)v); };
+        const double mr = fmax(fmax(fmax(mag(t.mnx[0]), mag(t.mxx[0])),
+                                    fmax(mag(t.mny[0]), mag(t.mxy[0]))),
+                               fmax(mag(t.mnz[0]), mag(t.mxz[0])));
+        const double mq = fmax(mag(px), fmax(mag(py), mag(pz)));
+        fE = fpf_err(fmax(mr, mq) * (double)fs, (double)t.m.box, MK == MK_WRAP);
+        if (IPF && t.m.dshift) fE += 1.0;  // what the shift drops
         fL = (float)t.m.box;
     }
     // Node test.  Integer periodic metric: a float32 squared distance that is
@@ -836,11 +849,12 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
 #pragma unroll UNROLL
             for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | near(j);
         } else if constexpr (FPF) {
-            // float32 pre-filter of double coordinates (fpf_*): never rejects
-            // a leaf within w; the insertion below tests every passing leaf
-            // exactly.
-            s_leaf[lane] = make_uint4(__float_as_uint((float)bx), __float_as_uint((float)by),
-                                      __float_as_uint((float)bz), 0u);
+            // float32 pre-filter (fpf_*): never rejects a leaf within w; the
+            // insertion below tests every passing leaf exactly.  Integers in an
+            // open box took 27 VALU a leaf for the exact 64-bit test, 9 here:
+            // 500k queries k = 8 on 2M points 1.90 -> 1.62 ms.
+            s_leaf[lane] = make_uint4(__float_as_uint((float)bx * fs), __float_as_uint((float)by * fs),
+                                      __float_as_uint((float)bz * fs), 0u);
             const float wf = fpf_upper((double)w, fE);
             [[maybe_unused]] const float lf = FLOOR ? fpf_lower((double)lo_d, fE) : 0.0f;
             constexpr bool WR = MK == MK_WRAP;
@@ -856,21 +870,26 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             for (int j = c0 - 1; j >= 0; --j) clo = (clo << 1) | near(j);
 #pragma unroll 4
             for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | near(j);
-        } else if constexpr (sizeof(T) == 4) {
-            // 32-bit coordinates (integer open box, float): exact test, operands
+        } else if constexpr (std::is_same<T, float>::value && MK != MK_ANY) {
+            // float coordinates: the exact test, whose distances are floats, so
+            // the comparisons are too (a bound no float reaches admits every
+            // finite distance, a floor none reaches no distance); operands
             // broadcast from LDS as above
-            s_leaf[lane] = make_uint4(bits32(bx), bits32(by), bits32(bz), 0u);
-            auto near = [&](int j) -> bool {
+            s_leaf[lane] = make_uint4(__float_as_uint(bx), __float_as_uint(by),
+                                      __float_as_uint(bz), 0u);
+            const float wf = w > (D)FLT_MAX ? FLT_MAX : (float)w;
+            [[maybe_unused]] const float lf = lo_d > (D)FLT_MAX ? HUGE_VALF : (float)lo_d;
+            auto near = [&](int j) -> uint32_t {
                 const uint4 e = s_leaf[j];
-                const D d = leaf_d2_k<T, MK>(t.m, px, py, pz, from_bits32<T>(e.x),
-                                             from_bits32<T>(e.y), from_bits32<T>(e.z));
-                if constexpr (FLOOR) return d <= w && d >= lo_d;
-                else return d <= w;
+                const float d = leaf_f32<MK>(t.m, px, py, pz, __uint_as_float(e.x),
+                                             __uint_as_float(e.y), __uint_as_float(e.z));
+                if constexpr (FLOOR) return (d <= wf && d >= lf) ? 1u : 0u;
+                else return d <= wf ? 1u : 0u;
             };
 #pragma unroll 4
-            for (int j = 0; j < c0; ++j) clo |= near(j) ? (1u << j) : 0u;
+            for (int j = c0 - 1; j >= 0; --j) clo = (clo << 1) | near(j);
 #pragma unroll 4
-            for (int j = 32; j < cnt; ++j) chi |= near(j) ? (1u << (j - 32)) : 0u;
+            for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | near(j);
         } else {
             auto near = [&](int j) -> bool {
                 const D d = leaf_d2_k<T, MK>(t.m, px, py, pz, rl(bx, j), rl(by, j), rl(bz, j));
