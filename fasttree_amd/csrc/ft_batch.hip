@@ -166,7 +166,7 @@ __global__ __launch_bounds__(64) void batch_packet_kernel(BatchView<T> b,
     constexpr bool PACKED = !CoordTraits<T>::fp;
     static_assert(!HEAP || PACKED, "LDS heap tier needs packed integer keys");
     using H = typename std::conditional<HEAP, TopKHeapLds<M>,
-                                        typename TopKSel<D, M, PACKED>::type>::type;
+                                        typename TopKSel<T, M, PACKED>::type>::type;
     __shared__ int32_t stk[PK_STACK];
     [[maybe_unused]] uint64_t *heap_mem = nullptr;
     if constexpr (HEAP) {

@@ -38,7 +38,9 @@ struct QueryMap {
     const uint32_t *order;  // slot -> query (null: identity)
     int32_t *list;          // direct passes: slots left to the listed pass, appended;
                             // LISTED: the slots to run
-    uint32_t *count;        // [0] list entries, [1] those that count as exact re-runs
+    uint32_t *count;        // [0] list entries, [1] those that count as exact re-runs,
+                            // [2] entries of packets
+    int32_t *packets;       // direct passes of cut keys: packets left whole, appended
 };
 
 // Appends the wave's slots with `left` set, one atomic per wave.  `rerun`: they
@@ -57,6 +59,10 @@ __device__ inline void append_slots(const QueryMap &qm, bool left, int slot, boo
     if (left)
         qm.list[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = slot;
+}
+
+__device__ inline void append_packet(const QueryMap &qm, int blk) {
+    if ((threadIdx.x & 63) == 0) qm.packets[atomicAdd(&qm.count[2], 1u)] = blk;
 }
 
 __device__ inline int slot_query(const QueryMap &qm, int slot) {
@@ -353,17 +359,29 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
 // Packed-key packets: at least 4 waves per SIMD (128 VGPRs), 11 % faster than
 // 3 at k = 32 and 19 % in the passes of 32 for k = 64, spills included.  With
 // the walk's counters in 32 bits the k = 32 kernel spills nothing (72 bytes a
-// lane before: 10M clustered points 16.9 -> 16.7 ms).  Double coordinates keep
-// their natural 3 waves (forcing 4 spilled 116 bytes and was 32 % slower).
-template <typename T, int M, bool HEAP, bool SEEDED, bool PACKED, int MK, bool MULTI = false>
+// lane before: 10M clustered points 16.9 -> 16.7 ms).  Exact pairs of doubles
+// keep their natural 3 waves.
+//
+// CUT keys (double coordinates, TopKFp): a packet whose queries have many
+// distances that agree above the cut -- regular grids, coincident particles --
+// is left whole to the LISTED instantiation, which takes its packets from
+// qm.packets and keeps exact (d, index) pairs.  It is found out by its fill
+// (equal neighbours among the k curve neighbours of a quarter of the lanes)
+// or at the end (a quarter of the lanes tied).  A lattice of 1M doubles takes
+// 0.95 / 1.56 / 3.36 ms at k = 8 / 16 / 32 this way (0.78 / 1.34 / 3.04 with
+// exact pairs only; 6.3 / 7.4 / 10.2 with a wave for each tied query).
+constexpr int TIED_LANES = 16;
+template <typename T, int M, bool HEAP, bool SEEDED, bool PACKED, int MK, bool MULTI = false,
+          bool LISTED = false>
 __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     DTree<T> t, QSrc<T> qs, PacketArgs a, QueryMap qm,
     const typename CoordTraits<T>::D *__restrict__ seed, uint64_t *__restrict__ res,
     typename CoordTraits<T>::D *__restrict__ dists) {
     using D = typename CoordTraits<T>::D;
     using H = typename std::conditional<HEAP, TopKHeapLds<M>,
-                                        typename TopKSel<D, M, PACKED>::type>::type;
-    static_assert(!HEAP || PACKED, "LDS heap tier needs packed integer keys");
+                                        typename TopKSel<T, M, PACKED>::type>::type;
+    static_assert(!HEAP || (PACKED && !CoordTraits<T>::fp), "LDS heap tier needs packed integer keys");
+    constexpr bool FPK = PACKED && CoordTraits<T>::fp;
     static_assert(HEAP || M <= 32, "register tiers hold at most 32 entries");
     __shared__ int32_t stk[PK_STACK];
     [[maybe_unused]] uint64_t *heap_mem = nullptr;
@@ -374,7 +392,10 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     const int lane = threadIdx.x;
     const int k = a.k;
     PacketCounters c;
-    const int blk = xcd_block();
+    if constexpr (LISTED) {
+        if (blockIdx.x >= qm.count[2]) return;
+    }
+    const int blk = LISTED ? uni(qm.packets[blockIdx.x]) : xcd_block();
     const int W = a.width;
     if (blk * W >= a.nq) return;  // padding block of the XCD-ordered grid
     const int slot = blk * W + lane;
@@ -405,7 +426,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
         // k above M (register tier): ceil(k / M) passes, each taking the M
         // nearest (d2, index) above the previous pass's last one, stored in
         // place.
-        bool redo = false;
+        bool redo = false, whole = false;
         typename H::Floor lo = H::no_floor();
         for (int base = 0; base < k; base += M) {
             const int kk = k - base < M ? k - base : M;
@@ -415,26 +436,44 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             // the kernel two registers.
             int qv = q;
             asm volatile("" : "+v"(qv));
-            if constexpr (PACKED) h.init(kk, (SEEDED && active) ? (uint64_t)seed[qv] : ~0ull, a.ibits);
-            else h.init(kk, (SEEDED && active) ? seed[qv] : dist_max<D>());
+            const D bound = (SEEDED && active) ? seed[qv] : dist_max<D>();
+            if constexpr (PACKED) h.init(kk, bound, a.ibits);
+            else h.init(kk, bound);
             // one walk instance for every pass (the first with no floor)
             packet_walk<T, H, MK, true>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo,
                                         whi, r0, lo, 0, 0, a.stop);
             if (active) {
                 bool r = false;
-                if constexpr (PACKED) r = h.needs_exact(kk);
+                if constexpr (FPK) r = h.tied() || (SEEDED && h.missing(kk));
+                else if constexpr (PACKED) r = h.needs_exact(kk);
                 else if constexpr (SEEDED) r = h.missing(kk) > 0;
                 redo = redo || r;
-                if (!redo) h.store_part(kk, res, dists, (size_t)q, k, base);
+                if constexpr (FPK) {
+                    int bad = 0;
+                    if (!redo) {
+                        bad = h.template store_row<MK>(kk, res, dists, (size_t)q, k, base, t, px,
+                                                       py, pz);
+                        asm volatile("" : "+v"(bad));
+                    }
+                    redo = redo || bad != 0;
+                } else {
+                    if (!redo) h.store_part(kk, res, dists, (size_t)q, k, base);
+                }
             }
             lo = h.next_floor();
+            if constexpr (H::kRankKeys) {
+                whole = !SEEDED && __popcll(__ballot(redo)) >= TIED_LANES;
+                if (whole) break;
+            }
         }
-        append_slots(qm, active && (redo || c.leaves > a.stop), slot, c.leaves <= a.stop);
+        if (whole) append_packet(qm, blk);
+        else append_slots(qm, active && (redo || c.leaves > a.stop), slot, c.leaves <= a.stop);
     } else {
         H h;
         if constexpr (HEAP) h.key = heap_mem;
-        if constexpr (PACKED) h.init(k, (SEEDED && active) ? (uint64_t)seed[q] : ~0ull, a.ibits);
-        else h.init(k, (SEEDED && active) ? seed[q] : dist_max<D>());
+        const D bound = (SEEDED && active) ? seed[q] : dist_max<D>();
+        if constexpr (PACKED) h.init(k, bound, a.ibits);
+        else h.init(k, bound);
         int flo = 0, fhi = 0;
         if constexpr (H::kSortFill) {
             // self queries over all leaves: lane = leaf rank r0 + lane; the
@@ -443,6 +482,12 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
                 __shared__ FillStage<T> fst;
                 c.inserts += (uint32_t)fill_from_run<T, MK>(t, h, k, active, self >= 0, rank, px,
                                                             py, pz, r0, &fst, flo, fhi);
+                if constexpr (H::kRankKeys) {
+                    if (__popcll(__ballot(active && h.agreeing(k))) >= TIED_LANES) {
+                        append_packet(qm, blk);
+                        return;
+                    }
+                }
             }
         }
         packet_walk<T, H, MK>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo, whi, r0,
@@ -450,11 +495,26 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
         bool left = false;
         if (active) {
             left = c.leaves > a.stop;
-            if constexpr (PACKED) left = left || h.needs_exact(k);
+            if constexpr (FPK) left = left || h.tied() || (SEEDED && h.missing(k));
+            else if constexpr (PACKED) left = left || h.needs_exact(k);
             else if constexpr (SEEDED) left = left || h.missing(k) > 0;
-            if (!left) h.store(k, res, dists, (size_t)q);
+            if constexpr (!FPK) {
+                if (!left) h.store(k, res, dists, (size_t)q);
+            }
         }
-        append_slots(qm, left, slot, c.leaves <= a.stop);
+        if constexpr (FPK) {
+            // (a 32-bit word kept opaque: as a lane mask, the lanes that had
+            // left before this branch lost their bit in it)
+            int bad = 0;
+            if (active && !left) {
+                bad = h.template store_row<MK>(k, res, dists, (size_t)q, k, 0, t, px, py, pz);
+                asm volatile("" : "+v"(bad));
+            }
+            left = left || bad != 0;
+        }
+        if (H::kRankKeys && c.leaves <= a.stop && __popcll(__ballot(left)) >= TIED_LANES && !SEEDED)
+            append_packet(qm, blk);
+        else append_slots(qm, left, slot, c.leaves <= a.stop);
     }
     if (lane == 0 && a.stats) {
         atomicAdd((unsigned long long *)&a.stats[0], (unsigned long long)c.nodes);
@@ -850,6 +910,7 @@ struct RerunBuf {
     int32_t *list = nullptr;
     uint32_t *tiles = nullptr;
     uint32_t *count = nullptr;
+    int32_t *packets = nullptr;  // one entry per packet of 16 queries or more
     size_t cap = 0;
     void *block = nullptr;
 };
@@ -966,7 +1027,7 @@ static int rerun_ensure(hipStream_t s, size_t n) {
     const size_t cap = n + n / 2 + 1024;
     const size_t tiles = cap / CP_TILE + 2;
     auto al = [](size_t x) { return (x + 255) & ~(size_t)255; };
-    const size_t bytes = al(cap) + al(cap * 4) + al(tiles * 4) + 256;
+    const size_t bytes = al(cap) + al(cap * 4) + al(tiles * 4) + 256 + al((cap / 16 + 1) * 4);
     void *p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) return fail(FT_ENOMEM, "re-run buffer allocation failed");
     char *c = (char *)p;
@@ -975,13 +1036,14 @@ static int rerun_ensure(hipStream_t s, size_t n) {
     g_rerun.list = (int32_t *)(c + al(cap));
     g_rerun.tiles = (uint32_t *)(c + al(cap) + al(cap * 4));
     g_rerun.count = (uint32_t *)(c + al(cap) + al(cap * 4) + al(tiles * 4));
+    g_rerun.packets = (int32_t *)(c + al(cap) + al(cap * 4) + al(tiles * 4) + 256);
     g_rerun.cap = cap;
     return FT_OK;
 }
 
 // Starts a direct pass's list (QueryMap::count).
 __global__ void zero_counts_kernel(uint32_t *count) {
-    if (threadIdx.x < 2) count[threadIdx.x] = 0;
+    if (threadIdx.x < 3) count[threadIdx.x] = 0;
 }
 __global__ void add_count_kernel(uint64_t *stats, const uint32_t *count) { stats[3] += count[1]; }
 
@@ -1048,6 +1110,13 @@ static int launch_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     return FT_OK;
 }
 
+// Top-k container of the packet kernels: packed keys, but for floating-point
+// coordinates' shortest list.  Self-kNN of 3M clustered points, exact pairs
+// against packed keys: double (periodic) k = 8 / 16 / 32 3.15 / 5.12 / 11.1
+// against 2.69 / 3.54 / 5.75 ms, float 2.38 / 3.93 / 9.82 against 1.88 / 2.43 /
+// 4.35 ms; 20 % of 20M doubles, k = 64 in passes, 97 against 31 ms.
+template <typename T, int M> constexpr bool packs_keys() { return !CoordTraits<T>::fp || M >= 4; }
+
 template <typename T, int M, bool HEAP, bool SEEDED, bool PACKED, int MK>
 static void launch_pk(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, const PacketArgs &a,
                       const QueryMap &qm, const typename CoordTraits<T>::D *seed, uint64_t *res,
@@ -1064,14 +1133,31 @@ static void launch_pk(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, cons
                        qs, a, qm, seed, res, d);
 }
 
+// The packets that a pass of cut keys left whole, with exact (d, index) pairs.
+template <typename T, int MK>
+static void launch_packets_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs,
+                                  const PacketArgs &a, const QueryMap &qm, uint64_t *res,
+                                  typename CoordTraits<T>::D *d) {
+    const dim3 g(blocks_for(a.nq, a.width));
+#define FT_LISTED(M_, MULTI_)                                                                     \
+    hipLaunchKernelGGL((packet_knn_kernel<T, M_, false, false, false, MK, MULTI_, true>), g,      \
+                       dim3(64), 0, s, dt, qs, a, qm, (const double *)nullptr, res, d)
+    if (a.k <= 4) FT_LISTED(4, false);
+    else if (a.k <= 8) FT_LISTED(8, false);
+    else if (a.k <= 16) FT_LISTED(16, false);
+    else if (a.k <= 32) FT_LISTED(32, false);
+    else FT_LISTED(32, true);
+#undef FT_LISTED
+}
+
 template <typename T, int M, bool HEAP, int MK>
 static void launch_packet_m(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs,
                             const PacketArgs &a, const QueryMap &qm,
                             const typename CoordTraits<T>::D *seed, uint64_t *res,
                             typename CoordTraits<T>::D *d) {
-    constexpr bool INTD = !CoordTraits<T>::fp;
-    if (seed) launch_pk<T, M, HEAP, true, INTD, MK>(s, dt, qs, a, qm, seed, res, d);
-    else launch_pk<T, M, HEAP, false, INTD, MK>(s, dt, qs, a, qm, seed, res, d);
+    constexpr bool PACKED = packs_keys<T, M>();
+    if (seed) launch_pk<T, M, HEAP, true, PACKED, MK>(s, dt, qs, a, qm, seed, res, d);
+    else launch_pk<T, M, HEAP, false, PACKED, MK>(s, dt, qs, a, qm, seed, res, d);
 }
 
 // One canonical query launch: a direct pass, and where it can leave slots
@@ -1086,7 +1172,9 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
                          typename CoordTraits<T>::D *d, uint64_t *stats, const RerunBuf *rr) {
     constexpr bool INTD = !CoordTraits<T>::fp;
     const uint32_t stop = ~0u;
-    const bool leaves_slots = algo == FT_ALGO_PACKET ? (INTD || seed || stop != ~0u)
+    // (float coordinates' keys are exact: nothing to leave without a seed)
+    const bool cuts = INTD || (std::is_same<T, double>::value && k > 1);
+    const bool leaves_slots = algo == FT_ALGO_PACKET ? (cuts || seed || stop != ~0u)
                                                      : algo != FT_ALGO_WAVE;
     if (leaves_slots) {
         if (!rr) {  // the stream's own buffers, grown to nq
@@ -1095,7 +1183,8 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         }
         hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, s, rr->count);
     }
-    const QueryMap qm{order, leaves_slots ? rr->list : nullptr, leaves_slots ? rr->count : nullptr};
+    const QueryMap qm{order, leaves_slots ? rr->list : nullptr, leaves_slots ? rr->count : nullptr,
+                      leaves_slots ? rr->packets : nullptr};
     if (algo == FT_ALGO_PACKET) {
         PacketArgs a{};
         a.nq = nq;
@@ -1117,6 +1206,11 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         const bool heap = INTD && topk == FT_TOPK_LDS_HEAP;
         if (!heap) {
             FT_BY_M(k, (launch_packet_m<T, M, false, MK>(s, dt, qs, a, qm, seed, res, d)));
+            if constexpr (std::is_same<T, double>::value) {
+                a.stats = nullptr;
+                a.stop = ~0u;
+                if (k > 1) launch_packets_listed<T, MK>(s, dt, qs, a, qm, res, d);
+            }
         } else if constexpr (INTD) {
             if (k <= 32) launch_packet_m<T, 32, true, MK>(s, dt, qs, a, qm, seed, res, d);
             else if (k <= 64) launch_packet_m<T, 64, true, MK>(s, dt, qs, a, qm, seed, res, d);
@@ -1225,7 +1319,7 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
         size_t lds = 0;
         const int lanes = lds_lanes<T>(k, STACK_DEPTH, lds);
         if (!lanes) return fail(FT_ELDS, "k too large for local memory: reduce k");
-        const QueryMap qm{nullptr, nullptr, nullptr};
+        const QueryMap qm{nullptr, nullptr, nullptr, nullptr};
         const dim3 g(xcd_grid(blocks_for(nq, lanes))), b(LANE_BLOCK);
         if (algo == FT_ALGO_PLAIN)
             hipLaunchKernelGGL((lane_knn_lds_kernel<T, true, false, false, MK_ANY>), g, b, lds, s,
@@ -1307,8 +1401,9 @@ int knn_entry(hipStream_t s, const ft_tree *tree, const void *qx, const void *qy
 // are cleared by a kernel at the start of each call and list entries are
 // written before they are read.  Calls that overlap on one device race.
 constexpr size_t NA_MAX_QUERIES = (size_t)1 << 24;
-constexpr size_t NA_OFF_COUNT = NA_MAX_QUERIES * 4;
-constexpr size_t NA_BYTES = NA_OFF_COUNT + 256;  // 64 MiB + 256 bytes
+constexpr size_t NA_OFF_PACKETS = NA_MAX_QUERIES * 4;
+constexpr size_t NA_OFF_COUNT = NA_OFF_PACKETS + (NA_MAX_QUERIES / 16 + 64) * 4;
+constexpr size_t NA_BYTES = NA_OFF_COUNT + 256;  // 68 MiB + 512 bytes
 static __device__ __align__(256) uint8_t scratch[NA_BYTES];
 
 constexpr int NA_MAX_DEVICES = 64;
@@ -1346,6 +1441,7 @@ int knn_noalloc_entry(hipStream_t s, const ft_tree *tree, int k, int excl, uint6
     char *c = (char *)p;
     RerunBuf rr;
     rr.list = (int32_t *)c;
+    rr.packets = (int32_t *)(c + NA_OFF_PACKETS);
     rr.count = (uint32_t *)(c + NA_OFF_COUNT);
     rr.cap = NA_MAX_QUERIES;
     FT_DISPATCH_COORD(tree->coord_type, {

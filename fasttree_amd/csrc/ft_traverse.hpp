@@ -314,6 +314,7 @@ __device__ __forceinline__ double f64_min(double a, double b) {
 }
 
 template <typename D, int M> struct TopK {
+    static constexpr bool kRankKeys = false;
     static constexpr bool kPacked = false;
     static constexpr bool kSortFill = false;
     static constexpr int kRoundsPerTrip = 2;
@@ -533,7 +534,8 @@ template <typename D, bool REF> struct LdsHeap {
 __device__ __forceinline__ double key_f64(uint64_t k) { return __longlong_as_double((long long)k); }
 __device__ __forceinline__ uint64_t key_u64(double k) { return (uint64_t)__double_as_longlong(k); }
 
-template <int M> struct TopKPacked {
+// The M sorted key slots and what works on whole keys.
+template <int M> struct KeySlots {
     static constexpr bool kPacked = true;
     static constexpr bool kSortFill = true;
     // insertion rounds per trip of the leaf loop (measured: two from 32 slots)
@@ -541,22 +543,12 @@ template <int M> struct TopKPacked {
     static constexpr uint64_t BIAS = 1ull << 62;
     static constexpr uint64_t NOKEY = BIAS | (1ull << 61);  // above every key, still finite
     uint64_t key[M];
-    int ib;
-    uint64_t sat, imask;
-    __device__ inline void init(int k, uint64_t bound, int ibits) {
-        ib = ibits;
-        sat = (1ull << (61 - ib)) - 1;
-        imask = (1ull << ib) - 1;
-        const uint64_t sent = BIAS | ((bound < sat ? bound : sat) << ib) | imask;
+    uint64_t imask;  // the index bits; all ones: an empty slot
+    // The k live slots start as the sentinel `sent`.
+    __device__ inline void init_slots(int k, uint64_t sent) {
 #pragma unroll
         for (int s = 0; s < M; ++s) key[s] = (s >= M - k) ? sent : 0ull;
     }
-    __device__ inline uint64_t make(uint64_t d, int32_t i) const {
-        return BIAS | ((d < sat ? d : sat) << ib) | (uint64_t)(uint32_t)i;
-    }
-    __device__ inline uint64_t dist_of(uint64_t kb) const { return (kb & ~BIAS) >> ib; }
-    __device__ inline uint64_t worst_d() const { return dist_of(key[M - 1]); }
-    __device__ inline bool beats_worst(uint64_t d, int32_t i) const { return make(d, i) < key[M - 1]; }
     // Sorted insertion, in place from the top slot down: with the slots
     // sorted, the new content of slot s is the median of key[s-1], c and
     // key[s], i.e. max(key[s-1], min(c, key[s])) -- key[s-1] when c is below
@@ -577,7 +569,6 @@ template <int M> struct TopKPacked {
         }
     }
     __device__ inline bool beats_worst_key(uint64_t kb) const { return kb < key[M - 1]; }
-    __device__ inline void insert(bool take, uint64_t d, int32_t i) { insert_key(take, make(d, i)); }
     __device__ inline void insert_key(bool take, uint64_t kb) {
         const uint64_t c = take ? kb : NOKEY;
         // New keys mostly land near the top: run only the part of the chain a
@@ -634,30 +625,49 @@ template <int M> struct TopKPacked {
         sort_slots();
         return kept;
     }
-    // Sentinels left in live slots, or a saturated k-th distance.
-    __device__ inline bool needs_exact(int k) const {
-        bool bad = dist_of(key[M - 1]) >= sat;
-#pragma unroll
-        for (int s = 0; s < M; ++s) bad |= (s >= M - k) & ((key[s] & imask) == imask);
-        return bad;
-    }
+    __device__ inline bool empty(int s) const { return (key[s] & imask) == imask; }
+    // A live slot is still empty.
     __device__ inline bool missing(int k) const {
         bool bad = false;
 #pragma unroll
-        for (int s = 0; s < M; ++s) bad |= (s >= M - k) & ((key[s] & imask) == imask);
+        for (int s = 0; s < M; ++s) bad |= (s >= M - k) & empty(s);
         return bad;
     }
     // Multi-pass queries: a pass takes only keys at or above the floor.
     using Floor = uint64_t;
     __device__ static inline Floor no_floor() { return 0ull; }
-    __device__ inline uint64_t floor_d(Floor lo) const { return dist_of(lo); }
-    __device__ inline bool above(Floor lo, uint64_t d, int32_t i) const { return make(d, i) >= lo; }
     // Lower key bound of the next pass of a multi-pass query: above the k-th
     // key, or nothing when a slot is still empty (no further neighbours).
-    __device__ inline uint64_t next_floor() const {
-        const uint64_t last = key[M - 1];
-        return ((last & imask) == imask) ? ~0ull : last + 1;
+    __device__ inline uint64_t next_floor() const { return empty(M - 1) ? ~0ull : key[M - 1] + 1; }
+};
+
+// Integer distances.
+template <int M> struct TopKPacked : KeySlots<M> {
+    using B = KeySlots<M>;
+    using B::key;
+    using B::imask;
+    static constexpr bool kRankKeys = false;
+    int ib;
+    uint64_t sat;
+    __device__ inline void init(int k, uint64_t bound, int ibits) {
+        ib = ibits;
+        sat = (1ull << (61 - ib)) - 1;
+        imask = (1ull << ib) - 1;
+        B::init_slots(k, B::BIAS | ((bound < sat ? bound : sat) << ib) | imask);
     }
+    __device__ inline uint64_t make(uint64_t d, int32_t i) const {
+        return B::BIAS | ((d < sat ? d : sat) << ib) | (uint64_t)(uint32_t)i;
+    }
+    __device__ inline uint64_t dist_of(uint64_t kb) const { return (kb & ~B::BIAS) >> ib; }
+    __device__ inline uint64_t worst_d() const { return dist_of(key[M - 1]); }
+    __device__ inline bool beats_worst(uint64_t d, int32_t i) const { return make(d, i) < key[M - 1]; }
+    __device__ inline void insert(bool take, uint64_t d, int32_t i) { B::insert_key(take, make(d, i)); }
+    // Sentinels left in live slots, or a saturated k-th distance.
+    __device__ inline bool needs_exact(int k) const {
+        return (dist_of(key[M - 1]) >= sat) | B::missing(k);
+    }
+    __device__ inline uint64_t floor_d(uint64_t lo) const { return dist_of(lo); }
+    __device__ inline bool above(uint64_t lo, uint64_t d, int32_t i) const { return make(d, i) >= lo; }
     // Entries [base, base + k) of row q (row length k_row).
     template <typename DOut>
     __device__ inline void store_part(int k, uint64_t *res, DOut *dists, size_t q, int k_row,
@@ -667,7 +677,7 @@ template <int M> struct TopKPacked {
         for (int s = 0; s < M; ++s) {
             if (s >= M - k) {
                 const size_t j = o + (size_t)(s - (M - k));
-                const bool ok = (key[s] & imask) != imask;
+                const bool ok = !B::empty(s);
                 res[j] = ok ? (key[s] & imask) : ~0ull;
                 dists[j] = ok ? (DOut)dist_of(key[s]) : missing_dist<DOut>();
             }
@@ -675,20 +685,119 @@ template <int M> struct TopKPacked {
     }
     template <typename DOut>
     __device__ inline void store(int k, uint64_t *res, DOut *dists, size_t q) const {
-        const size_t o = q * (size_t)k;
+        store_part(k, res, dists, q, k, 0);
+    }
+};
+
+// ---------------------------------------------------------------------------
+// Distances of floating-point coordinates as packed keys, so that their chain
+// costs the same two instructions a slot (a compare, a lexicographic tie test
+// and three selects before: 7).  Non-negative doubles and floats order as
+// their bit patterns do.
+//  * float coordinates: every squared distance is a float, so BIAS | its 31
+//    bits << 30 | index holds it exactly (indices are below 2^30 - 1).
+//  * double coordinates: BIAS | the top 61 - ib of the distance's 63 bits << ib
+//    | leaf rank.  The low ib + 2 bits (at most 32 of the 52 of the mantissa)
+//    are cut off, so keys order distances that differ above the cut; bounds
+//    use the largest distance a key can stand for, so every leaf whose cut
+//    distance is at most the k-th is offered to the list.  The result is exact
+//    unless two distances agree above the cut: `rejected` keeps the smallest
+//    key that a full list turned away or dropped, and the row, recomputed from
+//    the ranks in double precision, must come out in order.  A query that
+//    fails either test is answered again, exactly.  Near ties are rare where
+//    distances are continuous (at 20M points the cut keeps 25 bits of the
+//    mantissa: about one query in 100,000); where they are common, on a regular
+//    grid, the packet kernel hands whole packets to its exact instantiation.
+// ---------------------------------------------------------------------------
+template <typename T, int M> struct TopKFp : KeySlots<M> {
+    using B = KeySlots<M>;
+    using B::key;
+    using B::imask;
+    static constexpr bool kCut = std::is_same<T, double>::value;
+    static constexpr bool kRankKeys = kCut;  // keys hold leaf ranks, not returned indices
+    static constexpr int kFloatShift = 30;
+    uint64_t rejected;  // kCut only
+    __device__ inline uint64_t pack(double d, uint64_t i) const {
+        if constexpr (kCut) return B::BIAS | (((uint64_t)__double_as_longlong(d) >> 2) & ~imask) | i;
+        else return B::BIAS | ((uint64_t)__float_as_uint((float)d) << kFloatShift) | i;
+    }
+    __device__ inline void init(int k, double bound, int ibits) {
+        imask = (1ull << (kCut ? ibits : kFloatShift)) - 1;
+        // no key of an infinite or NaN distance is below the sentinel
+        bound = fmax(bound, 0.0);
+        if constexpr (kCut) bound = fmin(bound, DBL_MAX);
+        else bound = (double)__double2float_rd(fmin(bound, (double)FLT_MAX));
+        B::init_slots(k, pack(bound, imask));
+        rejected = B::NOKEY;
+    }
+    __device__ inline uint64_t make(double d, int32_t i) const { return pack(d, (uint32_t)i); }
+    // The largest and the smallest distance a key can stand for.
+    __device__ inline double d_hi(uint64_t kb) const {
+        if constexpr (kCut) return __longlong_as_double((long long)(((kb & ~B::BIAS) << 2) | (imask << 2) | 3));
+        else return (double)__uint_as_float((uint32_t)((kb & ~B::BIAS) >> kFloatShift));
+    }
+    __device__ inline double worst_d() const { return d_hi(key[M - 1]); }
+    __device__ inline double floor_d(uint64_t lo) const {
+        if (lo == ~0ull) return DBL_MAX;  // nothing is left
+        if constexpr (kCut) return __longlong_as_double((long long)(((lo & ~B::BIAS) & ~imask) << 2));
+        else return d_hi(lo);
+    }
+    // Offered to the list (c: NOKEY for a lane that offers nothing): what it
+    // turns away or drops.  Before insert_key.
+    __device__ inline void note(uint64_t c) {
+        if constexpr (kCut)
+            rejected = key_u64(f64_min(key_f64(rejected), f64_max(key_f64(c), key_f64(key[M - 1]))));
+    }
+    // A distance outside the list agrees with the last one above the cut (a
+    // dropped sentinel is no distance, and lies above every key of its bound).
+    __device__ inline bool tied() const {
+        if constexpr (kCut)
+            return ((rejected ^ key[M - 1]) & ~imask) == 0 && !B::empty(M - 1) &&
+                   (rejected & imask) != imask;
+        else return false;
+    }
+    // Two neighbouring live slots agree above the cut.
+    __device__ inline bool agreeing(int k) const {
+        bool any = false;
+#pragma unroll
+        for (int s = 1; s < M; ++s)
+            any |= (s > M - k) & (((key[s] ^ key[s - 1]) & ~imask) == 0) & !B::empty(s);
+        return any;
+    }
+    // Entries [base, base + k) of row q (row length k_row); double coordinates
+    // recompute them.  Returns true if they are not in (d, index) order.
+    template <int MK, typename Tr>
+    __device__ inline bool store_row(int k, uint64_t *res, double *dists, size_t q, int k_row,
+                                     int base, const Tr &t, T px, T py, T pz) const {
+        const size_t o = q * (size_t)k_row + (size_t)base;
+        const int off = t.n - 1;
+        bool bad = false;
+        double pd = -1.0;
+        int32_t pi = -1;
 #pragma unroll
         for (int s = 0; s < M; ++s) {
             if (s >= M - k) {
                 const size_t j = o + (size_t)(s - (M - k));
-                const bool ok = (key[s] & imask) != imask;
-                res[j] = ok ? (key[s] & imask) : ~0ull;
-                dists[j] = ok ? (DOut)dist_of(key[s]) : missing_dist<DOut>();
+                const bool ok = !B::empty(s);
+                int32_t i = (int32_t)(key[s] & imask);
+                double d;
+                if constexpr (kCut) {
+                    const int leaf = ok ? off + i : off;
+                    d = leaf_d2_k<T, MK>(t.m, px, py, pz, t.mnx[leaf], t.mny[leaf], t.mnz[leaf]);
+                    i = ret_index(t, leaf);
+                    bad |= ok & ((d < pd) | ((d == pd) & (i < pi)));
+                    pd = d;
+                    pi = i;
+                } else {
+                    d = d_hi(key[s]);
+                }
+                res[j] = ok ? (uint64_t)(uint32_t)i : ~0ull;
+                dists[j] = ok ? d : missing_dist<double>();
             }
         }
+        return bad;
     }
 };
-
-
 
 // ===========================================================================
 // Packet walk: the 64 lanes of a wavefront share one DFS over tree t.  A node
@@ -739,11 +848,17 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
     // Integer periodic metric: pre-shifted 32-bit query (wrap_gap_pre) and the
     // query masked to B bits for the exact inside-the-box tests.
     constexpr bool PRE = !CoordTraits<T>::fp && MK == MK_WRAP;
+    // (not in the multi-pass walks of unpacked doubles: there the filter's
+    // registers would push the kernel to one wave per SIMD)
+    constexpr bool F64 = std::is_same<T, double>::value && MK != MK_ANY && (!FLOOR || H::kPacked);
     // The leaf filter's operands (pre-shifted integer or float32 coordinates
     // of leaf j in slot j): one 16-byte LDS broadcast read per leaf serves
     // every lane, instead of three readlanes on the vector unit.  The walk
     // runs on one wave, whose LDS operations complete in order.
     __shared__ uint4 s_leaf[64];
+    // Double coordinates of the leaves for the insertion's exact distances: a
+    // lane reads its candidate's three instead of shuffling six words.
+    [[maybe_unused]] __shared__ double s_x[F64 ? 64 : 1], s_y[F64 ? 64 : 1], s_z[F64 ? 64 : 1];
     [[maybe_unused]] const int wsh = PRE ? 32 - t.m.bits : 0;
     [[maybe_unused]] uint32_t qxs = 0, qys = 0, qzs = 0;
     [[maybe_unused]] T qmx = px, qmy = py, qmz = pz;
@@ -760,10 +875,9 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
     }
     // Double coordinates, and integers in an open box: the float32 leaf
     // pre-filter (fpf_*), with E from the largest coordinate magnitude of the
-    // root box and the query.  Not for doubles in multi-pass walks (FLOOR):
-    // there its registers would push the kernel to one wave per SIMD.
+    // root box and the query.
     constexpr bool IPF = !CoordTraits<T>::fp && MK == MK_OPEN;
-    constexpr bool FPF = IPF || (std::is_same<T, double>::value && MK != MK_ANY && !FLOOR);
+    constexpr bool FPF = IPF || F64;
     [[maybe_unused]] float fqx = 0.f, fqy = 0.f, fqz = 0.f, fL = 0.f;
     [[maybe_unused]] double fE = 0.0;
     // an integer gap is shifted down by dshift: the filter works in those units
@@ -818,7 +932,7 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             bx = lx[first + lane];
             by = ly[first + lane];
             bz = lz[first + lane];
-            bo = t.orig_indices ? t.orig[off + first + lane] : first + lane;
+            bo = (t.orig_indices && !H::kRankKeys) ? t.orig[off + first + lane] : first + lane;
         }
         const D w = (D)h.worst_d();
         uint32_t clo = 0, chi = 0;
@@ -855,6 +969,11 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             // 500k queries k = 8 on 2M points 1.90 -> 1.62 ms.
             s_leaf[lane] = make_uint4(__float_as_uint((float)bx * fs), __float_as_uint((float)by * fs),
                                       __float_as_uint((float)bz * fs), 0u);
+            if constexpr (F64) {
+                s_x[lane] = bx;
+                s_y[lane] = by;
+                s_z[lane] = bz;
+            }
             const float wf = fpf_upper((double)w, fE);
             [[maybe_unused]] const float lf = FLOOR ? fpf_lower((double)lo_d, fE) : 0.0f;
             constexpr bool WR = MK == MK_WRAP;
@@ -927,13 +1046,15 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             const int j = has ? (__ffsll((long long)cand) - 1) : 0;
             cand &= cand - 1;
             // index of leaf first + j: its rank, or orig_idx fetched from lane j
-            const int32_t ri = t.orig_indices ? shfl_any(bo, j) : first + j;
+            const int32_t ri = (t.orig_indices && !H::kRankKeys) ? shfl_any(bo, j) : first + j;
             D d;
             if constexpr (PRE) {
                 const uint64_t gx = wrap_gap_pre(qxs, shfl32(ex, j), wsh);
                 const uint64_t gy = wrap_gap_pre(qys, shfl32(ey, j), wsh);
                 const uint64_t gz = wrap_gap_pre(qzs, shfl32(ez, j), wsh);
                 d = gx * gx + gy * gy + gz * gz;
+            } else if constexpr (F64) {
+                d = leaf_d2_k<T, MK>(t.m, px, py, pz, s_x[j], s_y[j], s_z[j]);
             } else {
                 const T x = shfl_any(bx, j), y = shfl_any(by, j), z = shfl_any(bz, j);
                 d = leaf_d2_k<T, MK>(t.m, px, py, pz, x, y, z);
@@ -941,9 +1062,11 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             ++c.rounds;
             bool take;
             if constexpr (H::kSortFill) {  // packed keys: made once for test and insertion
-                const uint64_t kb = h.make((uint64_t)d, ri);
-                take = has && h.beats_worst_key(kb);
-                if constexpr (FLOOR) take = take && kb >= lo;
+                const uint64_t kb = h.make(d, ri);
+                bool offered = has;
+                if constexpr (FLOOR) offered = offered && kb >= lo;
+                take = offered && h.beats_worst_key(kb);
+                if constexpr (H::kRankKeys) h.note(offered ? kb : H::NOKEY);
                 if (__any(take)) {  // a round no lane takes skips the chain
                     h.insert_key(take, kb);
                     ++c.chains;
@@ -1086,7 +1209,7 @@ __device__ __forceinline__ int fill_from_run(const DTree<T> &t, H &h, int k, boo
             st->x[e] = t.mnx[off + j];
             st->y[e] = t.mny[off + j];
             st->z[e] = t.mnz[off + j];
-            st->idx[e] = ret_index(t, off + j);
+            st->idx[e] = H::kRankKeys ? j : ret_index(t, off + j);
         }
     }
     __syncthreads();  // the block is this one wave
@@ -1098,7 +1221,7 @@ __device__ __forceinline__ int fill_from_run(const DTree<T> &t, H &h, int k, boo
         if (!active || j < 0 || j >= n) return ~0ull;
         const int e = j - base;
         const auto d = leaf_d2_k<T, MK>(t.m, px, py, pz, st->x[e], st->y[e], st->z[e]);
-        return h.make((uint64_t)d, st->idx[e]);
+        return h.make(d, st->idx[e]);
     });
     flo = active ? rank - half : 0;
     fhi = active ? rank + (k - half) + (excl ? 1 : 0) : 0;
@@ -1115,6 +1238,7 @@ __device__ __forceinline__ int fill_from_run(const DTree<T> &t, H &h, int k, boo
 // sifts down (log2 k levels); store() heapsorts in place.
 // ---------------------------------------------------------------------------
 template <int KCAP> struct TopKHeapLds {
+    static constexpr bool kRankKeys = false;
     static constexpr bool kPacked = true;
     static constexpr bool kSortFill = false;
     static constexpr int kRoundsPerTrip = 2;
@@ -1189,9 +1313,15 @@ template <int KCAP> struct TopKHeapLds {
 // Top-k container of a packet traversal: registers for M <= 32 (canonical
 // (d, idx) pairs, or packed keys for integer metrics), an LDS heap above that
 // (integer metrics only).
-template <typename D, int M, bool PACKED> struct TopKSel { using type = TopK<D, M>; };
-template <int M> struct TopKSel<uint64_t, M, true> {
+template <typename T, int M, bool PACKED> struct TopKSel {
+    using D = typename CoordTraits<T>::D;
+    using type = typename std::conditional<PACKED && CoordTraits<T>::fp, TopKFp<T, M>, TopK<D, M>>::type;
+};
+template <int M> struct TopKSelInt {
     using type = typename std::conditional<(M > 32), TopKHeapLds<M>, TopKPacked<M>>::type;
+};
+template <int M> struct TopKSel<uint32_t, M, true> : TopKSelInt<M> {};
+template <int M> struct TopKSel<uint64_t, M, true> : TopKSelInt<M> {
 };
 
 // Leaf rank reached from the root by a greedy descent for one point: at every

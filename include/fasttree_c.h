@@ -257,7 +257,7 @@ int ft_self_knn_query(ft_stream s, const ft_tree *tree, int k, uint64_t *results
 /* Non-allocating self_knn_query: no counterpart in the reference.  For callers that     */
 /* cannot allocate device memory (code under hipGraph capture, tight serving loops,       */
 /* harnesses that forbid hipMalloc).  Same arguments and results as ft_self_knn_query;    */
-/* the re-run buffers live in a fixed device array of 64 MiB per GPU, held until the      */
+/* the re-run buffers live in a fixed device array of 68 MiB per GPU, held until the      */
 /* process ends, so at most 16777216 queries (num_leaves; FT_ERANGE above).  results,     */
 /* dists, seed_bound and stats must be device (or pinned host) memory (FT_EINVAL          */
 /* otherwise).  Every call on one GPU shares that array: calls that overlap on one GPU    */

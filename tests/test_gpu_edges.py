@@ -85,3 +85,59 @@ def test_slots_left_to_the_listed_pass(ft, orc, n, ct, share):
     r, d = ft.self_knn_query(tree, k, seed_bound=ft.DeviceArray.from_host(seed), stats=stats)
     assert np.array_equal(r, rb) and np.array_equal(d, db)
     assert stats.to_host()[3] == int(np.sum(seed < db[:, -1]))
+
+
+def _doubles(name, n, seed):
+    i = np.arange(n)
+    rng = np.random.default_rng(seed)
+    if name == "grid":  # distances exactly equal
+        return [(i // 225).astype(float), (i // 15 % 15).astype(float), (i % 15).astype(float)]
+    if name == "rounded grid":  # equal but for the last bits
+        return [(i // 225) * 0.1 + 0.05, (i // 15 % 15) * 0.1 + 0.05, (i % 15) * 0.1 + 0.05]
+    if name == "coincident":
+        return [np.repeat(rng.random(-(-n // 8)), 8)[:n] for _ in range(3)]
+    return [rng.random(n) ** 3 for _ in range(3)]
+
+
+# list widths 4, 8, 16, 32 and passes of 32, full and not; packets of ties
+# beside packets without
+@pytest.mark.parametrize("k", [2, 4, 5, 8, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("name", ["grid", "rounded grid", "coincident", "continuous"])
+@pytest.mark.parametrize("ct", [O.CT_F64, O.CT_F32])
+def test_packed_distances_of_floating_point(ft, orc, k, name, ct):
+    n = 3375
+    pts = [a.astype(O.COORD_DTYPES[ct]) for a in _doubles(name, n, k)]
+    if name == "rounded grid":
+        half = [a.astype(O.COORD_DTYPES[ct]) for a in _doubles("continuous", n, k + 1)]
+        pts = [np.concatenate([a, b + a.max()]) for a, b in zip(pts, half)]
+    n = len(pts[0])
+    ids = np.random.default_rng(k).permutation(n)[: n // 4].astype(np.int32)
+    for periodic, orig in ((0, False), (1, True)):
+        box = float(max(a.max() for a in pts)) * 1.01 if periodic else 0.0
+        tree = ft.TreeSoA(n, ct, ft.Config(sfc=O.SFC_PH, bits_per_dim=21, periodic=periodic,
+                                           box_length=box, return_orig_indices=orig))
+        ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(a) for a in pts)), tree)
+        t = O.build_bvh(ct, *pts, sfc=O.SFC_PH, bits=21, periodic=periodic, box=box,
+                        orig_indices=int(orig))
+        rb, db = O.knn_bruteforce(t, k, True)
+        r, d = ft.self_knn_query(tree, k, max_k=64, algorithm=ft.ALGO_PACKET)
+        assert np.array_equal(d, db) and np.array_equal(r, rb)
+        r, d = ft.self_knn_query_subset(tree, ids, k, algorithm=ft.ALGO_PACKET)
+        assert np.array_equal(d, db[ids]) and np.array_equal(r, rb[ids])
+
+
+def test_packed_distances_that_overflow(ft, orc):
+    """Squared distances beyond the coordinate type's range are no neighbours;
+    huge finite ones are."""
+    for ct, big in ((O.CT_F64, 1e160), (O.CT_F32, 1e19)):
+        rng = np.random.default_rng(5)
+        pts = [(rng.random(200) * 1e-3 * big).astype(O.COORD_DTYPES[ct]) for _ in range(3)]
+        for a in pts:
+            a[100:] += np.array(big * 30, a.dtype)  # d2 to the other half overflows
+        tree = ft.TreeSoA(200, ct, ft.Config(sfc=O.SFC_PH, bits_per_dim=21))
+        ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(a) for a in pts)), tree)
+        for k in (8, 32):
+            want = ft.self_knn_query(tree, k, algorithm=ft.ALGO_PLAIN)
+            got = ft.self_knn_query(tree, k, algorithm=ft.ALGO_PACKET)
+            for a, b in zip(got, want):
+                assert np.array_equal(a, b)
