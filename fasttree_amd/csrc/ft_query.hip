@@ -17,6 +17,7 @@
 #include "ft_traverse.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -1160,6 +1161,53 @@ static void launch_packet_m(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs
     else launch_pk<T, M, HEAP, false, PACKED, MK>(s, dt, qs, a, qm, seed, res, d);
 }
 
+// Whether a call's queries are so few that a wave for each of them finishes
+// before packets of 64 do.  A packet's walk is one wave's serial work (0.2 to
+// 1 ms, more where its queries lie far apart, as few queries of many points
+// do) and few packets leave the chip idle; a wave per query costs 5 to 13 ns of
+// the whole chip.  The line is where both took the same time over trees of 20k
+// to 10M points (packets against waves, us): 30k points k = 8 30k queries
+// 580 / 476, 100k 481 / 1186; 300k points 30k 899 / 374, 100k 821 / 849; 10M
+// points 200k 3003 / 2785, 500k 3039 / 6308; k = 32 of 10M points 200k
+// 5412 / 3282, 500k 5861 / 7408.  1,000 queries k = 32 of 10M points took 21 ms
+// in packets.
+static bool few_queries(int64_t nq, int64_t n, int k) {
+    const double f = k <= 4 ? 0.8 : (k <= 16 ? 1.0 : (k <= 32 ? 1.7 : 5.0));
+    return (double)nq <= 900.0 * f * std::cbrt((double)n);
+}
+
+// Wave-tier queries up to this many run in the caller's order: sorting them
+// along the curve costs 60 us of launches and gains nothing while the waves in
+// flight hold most of them (10M points, k = 32, ordered / unordered: 1k queries
+// 196 / 150 us, 20k 575 / 532, 40k 924 / 938, 80k 1544 / 1794).
+constexpr int UNORDERED_WAVES = 24576;
+
+// Queries per packet: 64, one per lane, or 32 while the packets of 64 would be
+// fewer than about two and a half per SIMD (build + self-kNN of 100k doubles,
+// k = 4 / 8 / 16 / 32: uniform 373 / 436 / 503 / 681 us with 64, 362 / 418 /
+// 481 / 667 with 32; clustered 565 / 638 / 746 / 1174 and 521 / 594 / 703 /
+// 1079; at 400k points 64 are 10 % faster).
+constexpr int WIDE_PACKETS_FROM = 150000;
+
+// Leaves a packet may scan before its queries go to one wave each, so that the
+// few packets whose queries lie far apart do not set the time.  A hand-over
+// costs 60 to 100 us however few the queries, so the limits lie above what
+// packets of uniform points need (2,000 in packets of 64 cost k = 16 of 100k
+// uniform doubles 40 us of 500).  Self-kNN of 300k clustered floats k = 8 /
+// 16 / 32: 885 / 1145 / 1591 us without, 476 / 579 / 959 with; above 600k
+// points packets are enough to cover the slow ones (2M points 3 % slower with
+// 4,000).  Other queries share less of their walks the sparser they are
+// (k = 32, 1M queries of 2M doubles 4.77 ms without, 3.81 with 4,000; of 10M
+// points 7.25 without, 14.6 with 4,000).
+static uint32_t packet_leaf_limit(int64_t nq, int64_t n, int k, int width, bool all_leaves) {
+    const int64_t passes = (k + 31) / 32;
+    if (!all_leaves) return (uint32_t)std::min<int64_t>(passes * (3000 + 1000 * (n / nq)), 1 << 30);
+    if (n > 600000) return ~0u;
+    const int64_t per_pass = width == 64 ? (k <= 16 ? 3000 : 4000)
+                                         : (k <= 8 ? 2000 : (k <= 16 ? 2500 : 3000));
+    return (uint32_t)(passes * per_pass);
+}
+
 // One canonical query launch: a direct pass, and where it can leave slots
 // unanswered (packed keys that saturate, seeds that were too small, per-lane
 // stacks that would overflow) the listed pass over the slots it appended.  No
@@ -1171,7 +1219,10 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
                          const typename CoordTraits<T>::D *seed, uint64_t *res,
                          typename CoordTraits<T>::D *d, uint64_t *stats, const RerunBuf *rr) {
     constexpr bool INTD = !CoordTraits<T>::fp;
-    const uint32_t stop = ~0u;
+    // (the listed pass's wave tier is the one of k <= 128)
+    const uint32_t stop = algo == FT_ALGO_PACKET && !seed && topk != FT_TOPK_LDS_HEAP
+                              ? packet_leaf_limit(nq, dt.n, k, width, !qs.qx && !qs.leaf_ids)
+                              : ~0u;
     // (float coordinates' keys are exact: nothing to leave without a seed)
     const bool cuts = INTD || (std::is_same<T, double>::value && k > 1);
     const bool leaves_slots = algo == FT_ALGO_PACKET ? (cuts || seed || stop != ~0u)
@@ -1331,25 +1382,21 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
         return FT_OK;
     }
     // Canonical mode.  Packet tiers: registers for k <= 32, passes of 32 up
-    // to k = 128.  Above k = 32 the wave-per-query tier, except where packets
-    // of integer queries share their walks best: self queries over all leaves
-    // up to k = 128, and subsets of at least a fifth of the leaves up to
-    // k = 64.  Measured on 10M clustered int64 points, passes against the
-    // wave tier: self k = 33 / 64 / 128 37.6 / 47.3 / 103.3 against 86.9 /
-    // 106.6 / 153.8 ms; a 20 % subset 15.7 / 19.4 / 41.2 against 18.7 / 22.7 /
-    // 32.3 ms; 1M external queries 14.6 / 19.1 / 40.4 against 13.0 / 15.1 /
-    // 20.1 ms.  20M clustered doubles: self k = 33 / 64 176 / 249 against
-    // 172 / 213 ms, a 20 % subset k = 64 98 against 45 ms, 1M external
-    // queries k = 64 79 against 15 ms.  Above k = 1024, the per-lane heap
-    // walk.
+    // to k = 128 where packets share their walks best: every leaf, or queries
+    // at least a fifth as many as the leaves up to k = 64 (10M clustered int64
+    // points, passes against the wave tier: self k = 64 / 128 47 / 103 against
+    // 107 / 154 ms, a 20 % subset k = 64 22.8 against 22.6, 1M external queries
+    // 19.4 against 16.1; 20M doubles: self k = 64 76 against 209 ms, a 20 %
+    // subset k = 64 / 128 31 / 67 against 45 / 62).  The wave tier for the
+    // others up to k = 1,024 and wherever the queries are few; above k = 1,024
+    // the per-lane heap walk.
     const bool packet_ok = k <= 128;  // above 32: passes of 32
     if (algo == FT_ALGO_AUTO) {
-        const bool int_q = !CoordTraits<T>::fp && !external;
-        const bool int_self = int_q && !qs.leaf_ids;
-        const bool int_dense_subset = int_q && qs.leaf_ids && (int64_t)nq * 5 >= (int64_t)dt.n;
+        const bool all_leaves = !external && !qs.leaf_ids;
+        const bool dense = (int64_t)nq * 5 >= (int64_t)dt.n;
         if (k > WAVE_MAX_K) algo = FT_ALGO_GROUPED;
-        else if (k <= 32 || (int_self && k <= 128) || (int_dense_subset && k <= 64))
-            algo = FT_ALGO_PACKET;
+        else if (few_queries(nq, dt.n, k)) algo = FT_ALGO_WAVE;
+        else if (k <= 32 || (all_leaves && k <= 128) || (dense && k <= 64)) algo = FT_ALGO_PACKET;
         else algo = FT_ALGO_WAVE;
     }
     if (o.seed_bound && packet_ok) algo = FT_ALGO_PACKET;
@@ -1359,17 +1406,16 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
     const int bucket = o.leaf_bucket > 0 ? std::min(o.leaf_bucket, 64) : 64;
     const uint32_t *order = nullptr;
     if (algo == FT_ALGO_WAVE && k > WAVE_MAX_K) algo = FT_ALGO_GROUPED;
-    if ((algo == FT_ALGO_PACKET || algo == FT_ALGO_WAVE) && (qs.qx || qs.leaf_ids) && nq > 64)
+    if ((algo == FT_ALGO_PACKET || algo == FT_ALGO_WAVE) && (qs.qx || qs.leaf_ids) && nq > (algo == FT_ALGO_WAVE ? UNORDERED_WAVES : 64))
         FT_TRY(query_order<T>(s, dt, qs, nq, order));
     // auto: 192 leaves on each side (self k = 32 at 10M clustered points: 64 /
     // 128 / 192 / 256 / 384 took 19.17 / 18.93 / 18.80 / 18.77 / 18.81 ms;
     // 192 was also as fast or faster at k = 1 to 64, for subsets and for
     // external queries)
     const int window = o.window < 0 ? 0 : (o.window == 0 ? 192 : std::min(o.window, 1 << 20));
-    // queries per packet: 64 (one per lane) unless 16 or 32 is asked for
     if (o.group_width != 0 && o.group_width != 16 && o.group_width != 32 && o.group_width != 64)
         return fail(FT_EINVAL, "group_width must be 0, 16, 32 or 64");
-    const int width = o.group_width ? o.group_width : 64;
+    const int width = o.group_width ? o.group_width : (nq < WIDE_PACKETS_FROM ? 32 : 64);
     switch (metric_kind<T>(dt.m)) {
     case MK_WRAP:
         return run_canonical<T, MK_WRAP>(s, dt, qs, nq, k, excl, algo, bucket, o.topk, window,

@@ -141,3 +141,43 @@ def test_packed_distances_that_overflow(ft, orc):
             got = ft.self_knn_query(tree, k, algorithm=ft.ALGO_PACKET)
             for a, b in zip(got, want):
                 assert np.array_equal(a, b)
+
+
+# The automatic choice on either side of its lines: few queries (a wave each,
+# unsorted up to 24,576), packets of 32 and 64, packets handed over
+@pytest.mark.parametrize("n,nq", [(3000, 1), (3000, 64), (3000, 65), (40_000, 24_576),
+                                  (40_000, 24_577), (3000, 40_000), (3000, 160_000)])
+@pytest.mark.parametrize("ct,k", [(O.CT_U64, 8), (O.CT_F64, 16), (O.CT_F32, 1), (O.CT_U32, 33)])
+def test_automatic_external_queries(ft, orc, n, nq, ct, k):
+    rng = np.random.default_rng(nq + k)
+    fp = ct in (O.CT_F32, O.CT_F64)
+    hi = 1.0 if fp else float(1 << 21)
+    p = rng.random((3, n)) ** 4 * hi  # dense near the origin: packets far out are wide
+    q = np.concatenate([rng.random((3, nq - nq // 2)) ** 4, rng.random((3, nq // 2))], 1) * hi
+    pts = [a.astype(O.COORD_DTYPES[ct]) for a in p]
+    qs = [np.ascontiguousarray(a[rng.permutation(nq)].astype(O.COORD_DTYPES[ct])) for a in q]
+    tree = ft.TreeSoA(n, ct, ft.Config(sfc=O.SFC_PH, bits_per_dim=21))
+    ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(a) for a in pts)), tree)
+    t = O.build_bvh(ct, *pts, sfc=O.SFC_PH, bits=21)
+    r, d = ft.knn_query(tree, *qs, k)
+    rows = rng.choice(nq, min(nq, 300), replace=False)
+    rb, db = O.knn_bruteforce(t, k, queries=[a[rows] for a in qs])
+    assert np.array_equal(d[rows], db) and np.array_equal(r[rows], rb)
+    w, wd = ft.knn_query(tree, *qs, k, algorithm=ft.ALGO_WAVE)
+    assert np.array_equal(r, w) and np.array_equal(d, wd)
+
+
+# 150,000 queries: packets of 32 below, 64 above; few queries below 900 * 1.7 *
+# cbrt(n); the clustered half makes packets that pass their leaf limit
+@pytest.mark.parametrize("n", [20_000, 60_000, 149_999, 150_001])
+@pytest.mark.parametrize("ct,k", [(O.CT_U32, 8), (O.CT_F64, 32), (O.CT_F64, 64)])
+def test_automatic_self_queries(ft, n, ct, k):
+    rng = np.random.default_rng(n)
+    hi = 1.0 if ct == O.CT_F64 else float(1 << 21)
+    p = np.concatenate([rng.random((3, n // 2)), rng.random((3, n - n // 2)) ** 6], 1) * hi
+    pts = [np.ascontiguousarray(a.astype(O.COORD_DTYPES[ct])) for a in p]
+    tree = ft.TreeSoA(n, ct, ft.Config(sfc=O.SFC_MORTON, bits_per_dim=21))
+    ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(a) for a in pts)), tree)
+    r, d = ft.self_knn_query(tree, k, max_k=64)
+    w, wd = ft.self_knn_query(tree, k, max_k=64, algorithm=ft.ALGO_WAVE)
+    assert np.array_equal(r, w) and np.array_equal(d, wd)
