@@ -181,3 +181,57 @@ def test_automatic_self_queries(ft, n, ct, k):
     r, d = ft.self_knn_query(tree, k, max_k=64)
     w, wd = ft.self_knn_query(tree, k, max_k=64, algorithm=ft.ALGO_WAVE)
     assert np.array_equal(r, w) and np.array_equal(d, wd)
+
+
+# Range queries on both sides of the wave / packet line (400 * cbrt(n)), packets
+# with and without an inner radius, queries too far apart for the relative
+# filter, radii of zero, beyond the box and not a number, rows past the cap and
+# past the CSR pool of 128
+@pytest.mark.parametrize("n,nq", [(1, 70), (2, 5000), (64, 1700), (3000, 1), (3000, 5768),
+                                  (3000, 5770), (30_000, 13_000)])
+@pytest.mark.parametrize("ct", [O.CT_F64, O.CT_F32, O.CT_U64, O.CT_U32])
+@pytest.mark.parametrize("periodic", [0, 1])
+def test_range_queries_against_plain_distances(ft, n, nq, ct, periodic):
+    rng = np.random.default_rng(n + nq)
+    fp = ct in (O.CT_F64, O.CT_F32)
+    side = 100.0 if fp else float(1 << 21)
+    dt = O.COORD_DTYPES[ct]
+    cast = (lambda a: a.astype(dt)) if fp else (lambda a: np.floor(a).astype(dt))
+    pts = [cast(a) for a in rng.random((3, n)) ** 3 * side]
+    q = [cast(a) for a in rng.random((3, nq)) ** 3 * side]
+    r1 = rng.choice([0.0, 0.003, 0.02, 0.1, 0.3], nq) * side
+    r0 = np.where(rng.random(nq) < 0.5, 0.0, r1 * rng.random(nq))
+    r1, r0 = cast(r1), cast(r0)
+    if fp and nq > 100:
+        r1[3], r0[7], r1[11] = np.nan, np.nan, np.inf
+    tree = ft.TreeSoA(n, ct, ft.Config(sfc=O.SFC_PH, bits_per_dim=21, periodic=periodic,
+                                       box_length=side if fp and periodic else 0.0))
+    ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(a) for a in pts)), tree)
+    g = tree.to_host()
+    x = [g[a][n - 1:] for a in ("min_x", "min_y", "min_z")]
+    rows = np.arange(nq) if nq * n < 3e7 else np.unique(np.r_[3, 7, 11, rng.integers(0, nq, 600)])
+    d2 = None
+    for a in range(3):
+        if fp:
+            d = np.abs(q[a][rows, None] - x[a][None, :])
+            d = np.minimum(d, dt(side) - d) if periodic else d
+        else:
+            d = q[a][rows, None].astype(np.int64) - x[a][None, :].astype(np.int64)
+            if periodic:
+                d = (d + (1 << 20)) % (1 << 21) - (1 << 20)
+        d2 = d * d if d2 is None else d2 + d * d
+    if fp:
+        lo, hi = r0.astype(np.float64) ** 2, r1.astype(np.float64) ** 2
+        d2 = d2.astype(np.float64)
+    else:
+        lo, hi = r0.astype(np.int64) ** 2, r1.astype(np.int64) ** 2
+    hit = (d2 >= lo[rows, None]) & (d2 <= hi[rows, None])
+    cap = 20
+    res, counts = ft.range_query(tree, *q, r0, r1, cap)
+    assert np.array_equal(counts[rows], hit.sum(1))
+    rp, cols = ft.range_query_csr(tree, *q, r0, r1)
+    assert np.array_equal(np.diff(rp), counts)
+    for i, row in enumerate(rows):
+        want = np.flatnonzero(hit[i])
+        assert np.array_equal(cols[rp[row]:rp[row + 1]], want)
+        assert np.array_equal(res[row][:min(cap, len(want))], want[:cap])
