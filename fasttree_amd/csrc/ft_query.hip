@@ -358,10 +358,11 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
 }
 
 // Packed-key packets: at least 4 waves per SIMD (128 VGPRs), 11 % faster than
-// 3 at k = 32 and 19 % in the passes of 32 for k = 64, spills included.  With
-// the walk's counters in 32 bits the k = 32 kernel spills nothing (72 bytes a
-// lane before: 10M clustered points 16.9 -> 16.7 ms).  Exact pairs of doubles
-// keep their natural 3 waves.
+// 3 at k = 32.  With the walk's counters in 32 bits the k = 32 kernel spills
+// nothing (72 bytes a lane before: 10M clustered points 16.9 -> 16.7 ms).  The
+// passes of 32 spill (integers 244 bytes, doubles 56) and are faster so than at
+// 3 waves (k = 64 subset of 20M doubles 30.8 against 35.5 ms; of 2M integers
+// 20.5 against 21.4).  Exact pairs of doubles keep their natural 3 waves.
 //
 // CUT keys (double coordinates, TopKFp): a packet whose queries have many
 // distances that agree above the cut -- regular grids, coincident particles --
@@ -392,7 +393,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     }
     const int lane = threadIdx.x;
     const int k = a.k;
-    PacketCounters c;
+    PacketCountersFor<T, MULTI> c;
     if constexpr (LISTED) {
         if (blockIdx.x >= qm.count[2]) return;
     }
@@ -600,23 +601,6 @@ __device__ inline float wave_max_f32(float v) {
     return v;
 }
 
-// Coordinate a relative to c: exact for integers (wrapped to B bits if
-// periodic), in double precision for doubles (wrapped to half a period).
-template <typename T, int MK> __device__ inline float range_rel(const Metric &m, T a, T c) {
-    if constexpr (std::is_same<T, double>::value) {
-        double d = a - c;
-        if constexpr (MK == MK_WRAP) {
-            if (d > 0.5 * m.box) d -= m.box;
-            else if (d < -0.5 * m.box) d += m.box;
-        }
-        return (float)d;
-    } else if constexpr (MK == MK_WRAP) {
-        return (float)wrap_diff32((uint32_t)a, (uint32_t)c, 32 - m.bits);
-    } else {
-        return a >= c ? (float)(T)(a - c) : -(float)(T)(c - a);
-    }
-}
-
 // A node's leaf range and children (uniform across the wave); node 0 of a
 // one-leaf tree is that leaf.
 struct RangeNode {
@@ -687,9 +671,9 @@ __global__ __launch_bounds__(64) void range_packet_kernel(DTree<T> t, RangeSrc<T
         const int mid = (blk * 64 + 32 < nq) ? 32 : 0;
         cx = rl(px, mid); cy = rl(py, mid); cz = rl(pz, mid);
         if (active) {
-            fx = range_rel<T, MK>(t.m, px, cx);
-            fy = range_rel<T, MK>(t.m, py, cy);
-            fz = range_rel<T, MK>(t.m, pz, cz);
+            fx = rel_coord<T, MK>(t.m, px, cx);
+            fy = rel_coord<T, MK>(t.m, py, cy);
+            fz = rel_coord<T, MK>(t.m, pz, cz);
         }
         const float ext = wave_max_f32(fmaxf(fabsf(fx), fmaxf(fabsf(fy), fabsf(fz))));
         const float rad = wave_max_f32((float)sqrt((double)RM2) * (1.0f + 0x1p-20f));
@@ -761,8 +745,8 @@ __global__ __launch_bounds__(64) void range_packet_kernel(DTree<T> t, RangeSrc<T
                     return d <= f_out && d >= g_out;
                 });
             } else if constexpr (REL) {
-                s_leaf[lane] = make_float4(range_rel<T, MK>(t.m, bx, cx), range_rel<T, MK>(t.m, by, cy),
-                                           range_rel<T, MK>(t.m, bz, cz), 0.f);
+                s_leaf[lane] = make_float4(rel_coord<T, MK>(t.m, bx, cx), rel_coord<T, MK>(t.m, by, cy),
+                                           rel_coord<T, MK>(t.m, bz, cz), 0.f);
                 auto dist = [&](const float4 &e) { return fpf_sq(fx - e.x, fy - e.y, fz - e.z); };
                 uint64_t unsure;
                 {
@@ -1350,7 +1334,9 @@ constexpr int WIDE_PACKETS_FROM = 150000;
 // 4,000).  Other queries share less of their walks the sparser they are
 // (k = 32, 1M queries of 2M doubles 4.77 ms without, 3.81 with 4,000; of 10M
 // points 7.25 without, 14.6 with 4,000).
-static uint32_t packet_leaf_limit(int64_t nq, int64_t n, int k, int width, bool all_leaves) {
+static uint32_t packet_leaf_limit(int64_t nq, int64_t n, int k, int width, bool all_leaves,
+                                  bool fp) {
+    if (k > 32 && !fp) return ~0u;  // the integers' passes have no limit (packet_walk)
     const int64_t passes = (k + 31) / 32;
     if (!all_leaves) return (uint32_t)std::min<int64_t>(passes * (3000 + 1000 * (n / nq)), 1 << 30);
     if (n > 600000) return ~0u;
@@ -1372,7 +1358,7 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     constexpr bool INTD = !CoordTraits<T>::fp;
     // (the listed pass's wave tier is the one of k <= 128)
     const uint32_t stop = algo == FT_ALGO_PACKET && !seed && topk != FT_TOPK_LDS_HEAP
-                              ? packet_leaf_limit(nq, dt.n, k, width, !qs.qx && !qs.leaf_ids)
+                              ? packet_leaf_limit(nq, dt.n, k, width, !qs.qx && !qs.leaf_ids, !INTD)
                               : ~0u;
     // (float coordinates' keys are exact: nothing to leave without a seed)
     const bool cuts = INTD || (std::is_same<T, double>::value && k > 1);

@@ -176,6 +176,42 @@ __host__ __device__ __forceinline__ float fpf_lower(double lo, double E) {
     return (float)(b * b * (1.0 - 0x1p-22)) * (1.0f - 0x1p-22f);
 }
 
+// Coordinate a relative to c, as a float: the difference is exact for integers
+// (wrapped to B bits if periodic), in double precision for doubles (wrapped to
+// half a period).
+template <typename T, int MK>
+__host__ __device__ __forceinline__ float rel_coord(const Metric &m, T a, T c) {
+    if constexpr (CoordTraits<T>::fp) {
+        double d = (double)a - (double)c;
+        if constexpr (MK == MK_WRAP) {
+            if (d > 0.5 * m.box) d -= m.box;
+            else if (d < -0.5 * m.box) d += m.box;
+        }
+        return (float)d;
+    } else if constexpr (MK == MK_WRAP) {
+        return (float)wrap_diff32((uint32_t)a, (uint32_t)c, 32 - m.bits);
+    } else {
+        return a >= c ? (float)(T)(a - c) : -(float)(T)(c - a);
+    }
+}
+// Bounds of float32 squared distances taken from relative coordinates.  With
+// u = 2^-24, a query at |q| <= ext and a leaf at gap g on an axis (so |x| <=
+// |q| + g), the float gap is within (1 + 2u) g + E, E = 2.02 u ext (+ what the
+// doubles round), and the sum of squares within a factor 1 + 3.01u.  rel_upper
+// is not below the float distance of any leaf with d2 <= w, rel_lower not
+// above that of any leaf with d2 >= lo: all in float, with the rounding of the
+// conversion, the root (2 ulp) and the products covered; below 1e-30 the
+// floats' underflow is left out of it.
+__host__ __device__ __forceinline__ float rel_upper(float w, float E) {
+    w = w < 1.0e-30f ? 1.0e-30f : w;
+    const float b = __builtin_sqrtf(w * (1.0f + 0x1p-22f)) * (1.0f + 0x1p-21f) + 1.75f * E;
+    return b * b * (1.0f + 0x1p-20f);
+}
+__host__ __device__ __forceinline__ float rel_lower(float lo, float E) {
+    const float b = __builtin_sqrtf(lo * (1.0f - 0x1p-22f)) * (1.0f - 0x1p-21f) - 1.75f * E;
+    return lo < 1.0e-30f || !(b > 0.0f) ? 0.0f : b * b * (1.0f - 0x1p-20f);
+}
+
 // Float32 squared distance of a leaf, pre-shifted coordinates (scaled by
 // 2^(2 sh)); compared with wrap_filter_bound_pre it never rejects a leaf whose
 // exact squared distance is within the bound.
@@ -815,20 +851,27 @@ template <typename T, int M> struct TopKFp : KeySlots<M> {
 // [fill_lo, fill_hi): leaf ranks the caller already put into this lane's h
 // (fill_from_run); the window pre-scan skips them.
 // stop: the walk ends, with h unfinished, once c.leaves exceeds it (the lanes'
-// regions have too little in common).
+// regions have too little in common); not in the integers' multi-pass walks,
+// whose registers it would spill.
 // ===========================================================================
 constexpr int PK_STACK = 128;
 
-// 32 bits each: one packet's counts, kept in registers through the walk.
-struct PacketCounters {
-    uint32_t nodes = 0, leaves = 0, inserts = 0, overflow = 0;
-    uint32_t rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
+// One packet's counts, kept in registers through the walk: 32 bits each, but
+// 64 in the integers' multi-pass walks, whose spills the compiler places better
+// so (75 scratch instructions against 167, k = 64 of 10M points 47.9 ms against
+// 59.5).
+template <typename C> struct PacketCounters {
+    C nodes = 0, leaves = 0, inserts = 0, overflow = 0;
+    C rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
 };
+template <typename T, bool MULTI>
+using PacketCountersFor =
+    PacketCounters<typename std::conditional<MULTI && !CoordTraits<T>::fp, uint64_t, uint32_t>::type>;
 
-template <typename T, typename H, int MK, bool FLOOR = false>
+template <typename T, typename H, int MK, bool FLOOR = false, typename C>
 __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
                                             T pz, int self, H &h, int32_t *stk,
-                                            PacketCounters &c, int win_lo = 0, int win_hi = 0,
+                                            PacketCounters<C> &c, int win_lo = 0, int win_hi = 0,
                                             int win_mid = 0,
                                             typename H::Floor lo = H::no_floor(),
                                             int fill_lo = 0, int fill_hi = 0,
@@ -873,27 +916,47 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             qmz = pz & mask;
         }
     }
-    // Double coordinates, and integers in an open box: the float32 leaf
-    // pre-filter (fpf_*), with E from the largest coordinate magnitude of the
-    // root box and the query.
+    // The float32 leaf filter works on coordinates relative to the first lane's
+    // query (rel_coord): three subtractions, a product and two fmas a leaf.  A
+    // periodic metric needs no wrap there while every lane's bound and the
+    // lanes' extent stay within a quarter period: a leaf within a bound is then
+    // not wrapped, and one beyond half a period is outside either way.  (k = 32
+    // of 10M periodic integers 16.65 -> 15.75 ms against wrapped differences,
+    // subset k = 64 of 20M doubles 31.9 -> 30.8, whose error bound now follows
+    // the packet's extent; packets over the limits keep the older form.)
     constexpr bool IPF = !CoordTraits<T>::fp && MK == MK_OPEN;
-    constexpr bool FPF = IPF || F64;
-    [[maybe_unused]] float fqx = 0.f, fqy = 0.f, fqz = 0.f, fL = 0.f;
-    [[maybe_unused]] double fE = 0.0;
+    constexpr bool REL = PRE || IPF || F64;
+    // (the passes of periodic integers have no registers for it: 20.6 -> 21.4 ms)
+    constexpr bool REL_OK = !(PRE && FLOOR);
+    // largest squared bound the filter may be used with (negative: never)
+    [[maybe_unused]] float rel_w = -1.f, relE = 0.f;
     // an integer gap is shifted down by dshift: the filter works in those units
     [[maybe_unused]] const float fs = IPF ? 1.0f / (float)(1ull << t.m.dshift) : 1.0f;
-    if constexpr (FPF) {
-        fqx = (float)px * fs;
-        fqy = (float)py * fs;
-        fqz = (float)pz * fs;
-        auto mag = [](T v) { return fabs((double)v); };
-        const double mr = fmax(fmax(fmax(mag(t.mnx[0]), mag(t.mxx[0])),
-                                    fmax(mag(t.mny[0]), mag(t.mxy[0]))),
-                               fmax(mag(t.mnz[0]), mag(t.mxz[0])));
-        const double mq = fmax(mag(px), fmax(mag(py), mag(pz)));
-        fE = fpf_err(fmax(mr, mq) * (double)fs, (double)t.m.box, MK == MK_WRAP);
-        if (IPF && t.m.dshift) fE += 1.0;  // what the shift drops
-        fL = (float)t.m.box;
+    if constexpr (REL) {
+        const T cx = rl(px, 0), cy = rl(py, 0), cz = rl(pz, 0);
+        float ext = 0.f;
+        if (active)
+            ext = fmaxf(fabsf(rel_coord<T, MK>(t.m, px, cx)),
+                        fmaxf(fabsf(rel_coord<T, MK>(t.m, py, cy)),
+                              fabsf(rel_coord<T, MK>(t.m, pz, cz))));
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) ext = fmaxf(ext, __shfl_xor(ext, o, 64));
+        ext = rl(ext, 0) * fs;
+        relE = 2.02f * 0x1p-24f * ext;
+        if constexpr (F64) {
+            const double mc = fmax(fabs(cx), fmax(fabs(cy), fabs(cz)));
+            relE += (float)(0x1p-50 * (mc + (double)ext + (MK == MK_WRAP ? t.m.box : 0.0)));
+        }
+        if (IPF && t.m.dshift) relE += 1.0f;  // what the shift drops
+        if constexpr (MK == MK_WRAP) {
+            const float period = PRE ? (float)(1ull << t.m.bits) : (float)t.m.box;
+            const float room = 0.249f * period - ext;
+            // integers up to 22 bits are exact in float (relE covers the rest
+            // only in rel_upper, which they do not use)
+            if (room > 0.f && (!PRE || t.m.bits <= 22)) rel_w = room * room;
+        } else if (ext < 1.0e18f) {
+            rel_w = __builtin_huge_valf();
+        }
     }
     // Node test.  Integer periodic metric: a float32 squared distance that is
     // never above the exact one by more than wrap_filter_bound's margin (gaps
@@ -939,56 +1002,78 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
         const int c0 = cnt < 32 ? cnt : 32;
         [[maybe_unused]] uint32_t ex = 0, ey = 0, ez = 0;  // pre-shifted leaf j in lane j
         if constexpr (PRE) {
-            // float32 pre-filter (wrap_filter_near on pre-shifted coordinates):
-            // never rejects a leaf within w; the insertion below tests every
-            // passing leaf exactly.
             ex = (uint32_t)bx << wsh;
             ey = (uint32_t)by << wsh;
             ez = (uint32_t)bz << wsh;
-            s_leaf[lane] = make_uint4(ex, ey, ez, 0u);
-            const float wf = wrap_filter_bound_pre((uint64_t)w, wsh);
-            [[maybe_unused]] const float lf = wrap_filter_floor_pre((uint64_t)lo_d, wsh);
-            auto near = [&](int j) -> uint32_t {
-                const uint4 e = s_leaf[j];
-                const float d = wrap_sq_pre(qxs, qys, qzs, e.x, e.y, e.z);
-                if constexpr (FLOOR) return (d <= wf && d >= lf) ? 1u : 0u;
-                else return d <= wf ? 1u : 0u;
-            };
-            // leaf j's bit shifted in from the top, leaves taken last to first;
-            // unrolled so that several broadcast reads are in flight (8 for
-            // lists of 32 slots and more, 4 below: measured)
+        }
+        if constexpr (F64) {
+            s_x[lane] = bx;
+            s_y[lane] = by;
+            s_z[lane] = bz;
+        }
+        // Bit j: the filter passes leaf j, shifted in from the top, leaves taken
+        // last to first; unrolled so that several broadcast reads are in flight
+        // (8 for lists of 32 slots and more, 4 below: measured).
+        auto mark = [&](auto &&near) {
             constexpr int UNROLL = H::kRoundsPerTrip == 2 ? 8 : 4;
 #pragma unroll UNROLL
-            for (int j = c0 - 1; j >= 0; --j) clo = (clo << 1) | near(j);
+            for (int j = c0 - 1; j >= 0; --j) clo = (clo << 1) | (near(j) ? 1u : 0u);
 #pragma unroll UNROLL
-            for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | near(j);
-        } else if constexpr (FPF) {
-            // float32 pre-filter (fpf_*): never rejects a leaf within w; the
-            // insertion below tests every passing leaf exactly.  Integers in an
-            // open box took 27 VALU a leaf for the exact 64-bit test, 9 here:
-            // 500k queries k = 8 on 2M points 1.90 -> 1.62 ms.
-            s_leaf[lane] = make_uint4(__float_as_uint((float)bx * fs), __float_as_uint((float)by * fs),
-                                      __float_as_uint((float)bz * fs), 0u);
-            if constexpr (F64) {
-                s_x[lane] = bx;
-                s_y[lane] = by;
-                s_z[lane] = bz;
+            for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | (near(j) ? 1u : 0u);
+        };
+        if constexpr (REL) {
+            // Never rejects a leaf within w; the insertion below tests every
+            // passing leaf exactly.
+            const float wf = PRE ? wrap_filter_bound((uint64_t)w) : (float)w;
+            if (REL_OK && !__any(active && !(wf <= rel_w))) {
+                float fx, fy, fz, up;
+                [[maybe_unused]] float low = 0.f;
+                if constexpr (PRE) {
+                    const uint32_t c0x = rl(qxs, 0), c0y = rl(qys, 0), c0z = rl(qzs, 0);
+                    auto rel = [&](uint32_t v, uint32_t c) { return (float)((int32_t)(v - c) >> wsh); };
+                    fx = rel(qxs, c0x); fy = rel(qys, c0y); fz = rel(qzs, c0z);
+                    s_leaf[lane] = make_uint4(__float_as_uint(rel(ex, c0x)), __float_as_uint(rel(ey, c0y)),
+                                              __float_as_uint(rel(ez, c0z)), 0u);
+                    up = wf;
+                    if constexpr (FLOOR) low = (float)(uint64_t)lo_d * (1.0f - 0x1p-20f);
+                } else {
+                    const T cx = rl(px, 0), cy = rl(py, 0), cz = rl(pz, 0);
+                    fx = rel_coord<T, MK>(t.m, px, cx) * fs;
+                    fy = rel_coord<T, MK>(t.m, py, cy) * fs;
+                    fz = rel_coord<T, MK>(t.m, pz, cz) * fs;
+                    s_leaf[lane] = make_uint4(__float_as_uint(rel_coord<T, MK>(t.m, bx, cx) * fs),
+                                              __float_as_uint(rel_coord<T, MK>(t.m, by, cy) * fs),
+                                              __float_as_uint(rel_coord<T, MK>(t.m, bz, cz) * fs), 0u);
+                    up = rel_upper(wf, relE);
+                    if constexpr (FLOOR) low = rel_lower((float)lo_d, relE);
+                }
+                mark([&](int j) {
+                    const uint4 e = s_leaf[j];
+                    const float d = fpf_sq(fx - __uint_as_float(e.x), fy - __uint_as_float(e.y),
+                                           fz - __uint_as_float(e.z));
+                    if constexpr (FLOOR) return d <= up && d >= low;
+                    else return d <= up;
+                });
+            } else if constexpr (PRE) {
+                // wrapped differences from pre-shifted coordinates
+                s_leaf[lane] = make_uint4(ex, ey, ez, 0u);
+                const float up = wrap_filter_bound_pre((uint64_t)w, wsh);
+                [[maybe_unused]] const float low = wrap_filter_floor_pre((uint64_t)lo_d, wsh);
+                mark([&](int j) {
+                    const uint4 e = s_leaf[j];
+                    const float d = wrap_sq_pre(qxs, qys, qzs, e.x, e.y, e.z);
+                    if constexpr (FLOOR) return d <= up && d >= low;
+                    else return d <= up;
+                });
+            } else {
+                for (int j = 0; j < cnt; ++j) {
+                    const D d = leaf_d2_k<T, MK>(t.m, px, py, pz, rl(bx, j), rl(by, j), rl(bz, j));
+                    bool ok = d <= w;
+                    if constexpr (FLOOR) ok = ok && d >= lo_d;
+                    if (j < 32) clo |= ok ? (1u << j) : 0u;
+                    else chi |= ok ? (1u << (j - 32)) : 0u;
+                }
             }
-            const float wf = fpf_upper((double)w, fE);
-            [[maybe_unused]] const float lf = FLOOR ? fpf_lower((double)lo_d, fE) : 0.0f;
-            constexpr bool WR = MK == MK_WRAP;
-            auto near = [&](int j) -> uint32_t {
-                const uint4 e = s_leaf[j];
-                const float d = fpf_sq(fpf_gap(fqx, __uint_as_float(e.x), fL, WR),
-                                       fpf_gap(fqy, __uint_as_float(e.y), fL, WR),
-                                       fpf_gap(fqz, __uint_as_float(e.z), fL, WR));
-                if constexpr (FLOOR) return (d <= wf && d >= lf) ? 1u : 0u;
-                else return d <= wf ? 1u : 0u;
-            };
-#pragma unroll 4
-            for (int j = c0 - 1; j >= 0; --j) clo = (clo << 1) | near(j);
-#pragma unroll 4
-            for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | near(j);
         } else if constexpr (std::is_same<T, float>::value && MK != MK_ANY) {
             // float coordinates: the exact test, whose distances are floats, so
             // the comparisons are too (a bound no float reaches admits every
@@ -998,17 +1083,13 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
                                       __float_as_uint(bz), 0u);
             const float wf = w > (D)FLT_MAX ? FLT_MAX : (float)w;
             [[maybe_unused]] const float lf = lo_d > (D)FLT_MAX ? HUGE_VALF : (float)lo_d;
-            auto near = [&](int j) -> uint32_t {
+            mark([&](int j) {
                 const uint4 e = s_leaf[j];
                 const float d = leaf_f32<MK>(t.m, px, py, pz, __uint_as_float(e.x),
                                              __uint_as_float(e.y), __uint_as_float(e.z));
-                if constexpr (FLOOR) return (d <= wf && d >= lf) ? 1u : 0u;
-                else return d <= wf ? 1u : 0u;
-            };
-#pragma unroll 4
-            for (int j = c0 - 1; j >= 0; --j) clo = (clo << 1) | near(j);
-#pragma unroll 4
-            for (int j = cnt - 1; j >= 32; --j) chi = (chi << 1) | near(j);
+                if constexpr (FLOOR) return d <= wf && d >= lf;
+                else return d <= wf;
+            });
         } else {
             auto near = [&](int j) -> bool {
                 const D d = leaf_d2_k<T, MK>(t.m, px, py, pz, rl(bx, j), rl(by, j), rl(bz, j));
@@ -1038,7 +1119,7 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
                 cand &= ~(hi_m & ~((1ull << a0) - 1));
             }
         }
-        c.leaves += (uint32_t)cnt;
+        c.leaves += (C)cnt;
         // One insertion round: each lane takes its lowest remaining candidate.
         // Integer periodic metrics need only the low 32 bits of coordinates.
         auto round = [&]() {
@@ -1165,11 +1246,13 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             }
         }
         if (scan_cnt > 0) scan_range(scan_first, scan_cnt, window);
-        // Over the budget: the walk ends as if nothing were left.  (A branch out
+        // Over the limit: the walk ends as if nothing were left.  (A branch out
         // of the loop here made the allocator keep two copies of the list.)
-        if (c.leaves > stop) {
-            sp = 0;
-            next = -1;
+        if constexpr (!FLOOR || CoordTraits<T>::fp) {
+            if (c.leaves > stop) {
+                sp = 0;
+                next = -1;
+            }
         }
         while (next < 0 && sp > 0) {
             const int cn = uni(stk[--sp]);

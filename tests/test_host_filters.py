@@ -9,7 +9,7 @@ HIPCC = "/opt/rocm/bin/hipcc"
 
 
 @pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not installed")
-@pytest.mark.parametrize("name", ["open_filter_check"])
+@pytest.mark.parametrize("name", ["open_filter_check", "relative_filter_check"])
 def test_filter_never_rejects_a_leaf_within_the_bound(tmp_path, name):
     exe = str(tmp_path / name)
     subprocess.check_call([HIPCC, "-O2", "-std=c++17", "-ffp-contract=off", "--cuda-host-only",
