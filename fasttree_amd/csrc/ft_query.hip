@@ -564,8 +564,9 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
 // level costs one round trip to memory: both children's boxes, ranges and
 // links are loaded together and the stack holds them; a row that is full is
 // only counted.  Counts and CSR of 5M clustered doubles (60 hits a query) 30.5
-// -> 18.1 ms, 200k queries of 3M 64-bit points (at most 64 hits kept) 9.0 ->
-// 3.0 ms; runs of at most 32 / 48 / 64 leaves 20.1 / 18.5 / 18.1 ms.
+// -> 16.5 ms, long rows by waves; 200k queries of 3M 64-bit points (at most 64
+// hits kept) 8.5 -> 4.2 ms; runs of at most 32 / 48 / 64 leaves 20.1 / 18.5 /
+// 18.1 ms before the long rows.
 constexpr int RANGE_DROP_DEPTH = STACK_DEPTH - 2;  // 62
 
 // Where a range query's hits go: counts, fixed-stride rows, CSR rows.
