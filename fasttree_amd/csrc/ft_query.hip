@@ -548,9 +548,9 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
 // points inside the root box), so a wave's 64 queries are neighbours.
 //
 // Leaf test.  A float32 squared distance from coordinates relative to the
-// packet's middle query (fpf_*, whose error bound then follows the packet's
-// extent instead of the box's) tells most pairs apart: surely inside, surely
-// outside, and a few for the exact test.  Rounded relative coordinates q, x of
+// packet's middle query, or another where that is not finite (fpf_*, whose error
+// bound then follows the packet's extent instead of the box's), tells most pairs
+// apart: surely inside, surely outside, and a few for the exact test.  Rounded relative coordinates q, x of
 // a pair at gap g: |x| <= |q| + g, so the float gap is within (1 + 2u) g +
 // 2u |q|, which fpf_upper / fpf_lower cover with E = 2.02 u max|q| and the
 // doubles' own rounding.  Periodic boxes use it while every query is within a
@@ -669,7 +669,7 @@ __global__ __launch_bounds__(64) void range_packet_kernel(DTree<T> t, RangeSrc<T
         f_out = __double2float_rd(RM2);
         g_out = __double2float_ru(rm2);
     } else if constexpr (REL) {
-        const int mid = (blk * 64 + 32 < nq) ? 32 : 0;
+        const int mid = centre_lane<T>(active, px, py, pz, blk * 64 + 32 < nq ? 32 : 0);
         cx = rl(px, mid); cy = rl(py, mid); cz = rl(pz, mid);
         if (active) {
             fx = rel_coord<T, MK>(t.m, px, cx);

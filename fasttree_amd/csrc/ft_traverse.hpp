@@ -194,6 +194,21 @@ __host__ __device__ __forceinline__ float rel_coord(const Metric &m, T a, T c) {
         return a >= c ? (float)(T)(a - c) : -(float)(T)(c - a);
     }
 }
+// The lane whose query relative coordinates are taken from: the first at or after
+// `from` (else the first of all) with three finite coordinates.  Relative to one
+// that has none, every lane's coordinates would be NaN, and the filters would
+// reject what the other queries need.  (None finite: no lane has a neighbour.)
+template <typename T>
+__device__ __forceinline__ int centre_lane(bool active, T x, T y, T z, int from) {
+    if constexpr (CoordTraits<T>::fp) {
+        const uint64_t m = __ballot(active && __builtin_isfinite(x) && __builtin_isfinite(y) &&
+                                    __builtin_isfinite(z));
+        const uint64_t up = m >> from << from;
+        return uni(m ? __builtin_ctzll(up ? up : m) : from);
+    } else {
+        return from;
+    }
+}
 // Bounds of float32 squared distances taken from relative coordinates.  With
 // u = 2^-24, a query at |q| <= ext and a leaf at gap g on an axis (so |x| <=
 // |q| + g), the float gap is within (1 + 2u) g + E, E = 2.02 u ext (+ what the
@@ -916,8 +931,8 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             qmz = pz & mask;
         }
     }
-    // The float32 leaf filter works on coordinates relative to the first lane's
-    // query (rel_coord): three subtractions, a product and two fmas a leaf.  A
+    // The float32 leaf filter works on coordinates relative to one lane's query
+    // (centre_lane, rel_coord): three subtractions, a product and two fmas a leaf.  A
     // periodic metric needs no wrap there while every lane's bound and the
     // lanes' extent stay within a quarter period: a leaf within a bound is then
     // not wrapped, and one beyond half a period is outside either way.  (k = 32
@@ -932,8 +947,10 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
     [[maybe_unused]] float rel_w = -1.f, relE = 0.f;
     // an integer gap is shifted down by dshift: the filter works in those units
     [[maybe_unused]] const float fs = IPF ? 1.0f / (float)(1ull << t.m.dshift) : 1.0f;
+    [[maybe_unused]] int cl = 0;
     if constexpr (REL) {
-        const T cx = rl(px, 0), cy = rl(py, 0), cz = rl(pz, 0);
+        cl = centre_lane<T>(active, px, py, pz, 0);
+        const T cx = rl(px, cl), cy = rl(py, cl), cz = rl(pz, cl);
         float ext = 0.f;
         if (active)
             ext = fmaxf(fabsf(rel_coord<T, MK>(t.m, px, cx)),
@@ -1037,7 +1054,7 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
                     up = wf;
                     if constexpr (FLOOR) low = (float)(uint64_t)lo_d * (1.0f - 0x1p-20f);
                 } else {
-                    const T cx = rl(px, 0), cy = rl(py, 0), cz = rl(pz, 0);
+                    const T cx = rl(px, cl), cy = rl(py, cl), cz = rl(pz, cl);
                     fx = rel_coord<T, MK>(t.m, px, cx) * fs;
                     fy = rel_coord<T, MK>(t.m, py, cy) * fs;
                     fz = rel_coord<T, MK>(t.m, pz, cz) * fs;

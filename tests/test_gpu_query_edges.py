@@ -1,0 +1,95 @@
+"""Query kernels on inputs at the edges of what they accept: coordinates that are
+not numbers, distances that overflow, trees deeper than a walk's stack, buffers
+under capture, tied distances.  Against plain numpy or the oracle."""
+import numpy as np
+import pytest
+
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+FP = (O.CT_F64, O.CT_F32)
+
+
+def build(ft, ct, pts, periodic=0, box=0.0, sfc=O.SFC_PH, orig=False):
+    tree = ft.TreeSoA(len(pts[0]), ct, ft.Config(sfc=sfc, bits_per_dim=21, periodic=periodic,
+                                                 box_length=box, return_orig_indices=orig))
+    ft.build_bvh(ft.particles(*(ft.DeviceArray.from_host(np.ascontiguousarray(a)) for a in pts)),
+                 tree)
+    return tree
+
+
+def leaves(tree):
+    n = tree.num_leaves
+    g = tree.to_host()
+    return [g[a][n - 1:] for a in ("min_x", "min_y", "min_z")]
+
+
+def squared(q, x, box=0.0):
+    """The library's floating-point squared distances: one rounding an operation."""
+    d2 = None
+    for a in range(3):
+        d = np.abs(q[a][:, None] - x[a][None, :])
+        d = np.minimum(d, x[a].dtype.type(box) - d) if box else d
+        d2 = d * d if d2 is None else d2 + d * d
+    return d2.astype(np.float64)
+
+
+def nearest(d2, k):
+    """Canonical rows: (d2, index) ascending, finite distances only."""
+    d2 = np.where(np.isfinite(d2), d2, np.inf)
+    idx = np.argsort(d2, axis=1, kind="stable")[:, :k]
+    d = np.take_along_axis(d2, idx, 1)
+    none = ~np.isfinite(d)
+    return (np.where(none, np.uint64(2**64 - 1), idx.astype(np.uint64)),
+            np.where(none, -np.finfo(np.float64).max, d))
+
+
+# 64 queries in the caller's order put a bad one into lanes 0 and 32; more are
+# sorted along the curve, and a tenth of them bad reaches both lanes of some packet
+@pytest.mark.parametrize("axes", [(0,), (1, 2), (0, 1, 2)])
+@pytest.mark.parametrize("nq", [64, 6000])
+@pytest.mark.parametrize("periodic", [0, 1])
+@pytest.mark.parametrize("ct", FP)
+def test_a_query_that_is_not_a_number_empties_its_own_row_only(ft, orc, ct, periodic, nq, axes):
+    from fasttree_amd.batch import Batch, plan_requests
+    dt = O.COORD_DTYPES[ct]
+    rng = np.random.default_rng(nq + len(axes))
+    n, box = 2000, 100.0
+    pts = [(rng.random(n) * box).astype(dt) for _ in range(3)]
+    q = [(rng.random(nq) * box).astype(dt) for _ in range(3)]
+    bad = np.array([0, 32]) if nq == 64 else rng.choice(nq, nq // 10, replace=False)
+    for a in axes:
+        q[a][bad] = np.nan
+    tree = build(ft, ct, pts, periodic, box if periodic else 0.0)
+    d2 = squared(q, leaves(tree), box if periodic else 0.0)
+    assert np.isnan(d2[bad]).all()
+    r1 = rng.choice([3.0, 8.0, 15.0], nq).astype(dt)
+    r0 = np.where(rng.random(nq) < 0.7, 0.0, 2.0).astype(dt)
+    hit = (d2 >= r0[:, None].astype(float) ** 2) & (d2 <= r1[:, None].astype(float) ** 2)
+    res, counts = ft.range_query(tree, *q, r0, r1, 40)
+    rp, cols = ft.range_query_csr(tree, *q, r0, r1)
+    assert np.array_equal(counts, hit.sum(1)) and np.array_equal(np.diff(rp), counts)
+    assert np.array_equal(cols, np.nonzero(hit)[1])
+    for i in range(nq):
+        assert np.array_equal(res[i][:min(40, counts[i])], np.flatnonzero(hit[i])[:40])
+    for k in (8, 32, 64):
+        want, dist = nearest(d2, k)
+        for algo in (ft.ALGO_PACKET, ft.ALGO_AUTO):
+            if algo == ft.ALGO_AUTO and k > 32:
+                continue  # the wave tier lists distances that are not numbers last
+            r, d = ft.knn_query(tree, *q, k, algorithm=algo)
+            good = np.setdiff1d(np.arange(nq), bad)
+            assert np.array_equal(r[good], want[good]) and np.array_equal(d[good], dist[good])
+            if algo == ft.ALGO_PACKET:
+                assert (r[bad] == np.uint64(2**64 - 1)).all()
+        if k <= 32:
+            reqs, _, tr = plan_requests([nq], [k], [0])
+            dq = [ft.DeviceArray.from_host(a) for a in q]
+            r, d = ft.DeviceArray(tr, np.uint64), ft.DeviceArray(tr, np.float64)
+            b = Batch(ct)
+            b.set_trees([tree])
+            b.set_queries(reqs, *dq, r, d)
+            b.run()
+            r, d = r.to_host().reshape(nq, k), d.to_host().reshape(nq, k)
+            assert np.array_equal(r[good], want[good]) and np.array_equal(d[good], dist[good])
