@@ -293,6 +293,7 @@ __global__ __launch_bounds__(64) void merge_knn_kernel(DTree<T> t, QSrc<T> qs, i
 struct PacketArgs {
     int nq, k, excl, bucket, ibits;
     int width;   // queries per packet (16, 32 or 64): lanes at or above it idle
+    int full;    // passes of 32: a row with a slot left empty goes to the listed pass
     uint32_t stop;  // leaves a packet may scan before its queries are handed over
     int window;  // self queries over all leaves: leaves pre-scanned on each side
     uint64_t *stats;
@@ -315,7 +316,7 @@ struct PacketArgs {
 // ===========================================================================
 template <typename T, int S, int MK, bool LISTED = false>
 __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, int nq, int k,
-                                                       int excl, QueryMap qm,
+                                                       int excl, uint64_t cap, QueryMap qm,
                                                        uint64_t *__restrict__ res,
                                                        typename CoordTraits<T>::D *__restrict__ dists,
                                                        uint64_t *__restrict__ stats) {
@@ -331,7 +332,7 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
         const int self = excl ? rank : -1;
         const int anchor = rank >= 0 ? rank : descend_rank_v<T, MK>(t, px, py, pz);
         WaveList<S> L;
-        L.init(k);
+        L.init(k, cap);
         wave_walk<T, S, MK>(t, px, py, pz, self, anchor, L, c, &wbuf[threadIdx.x >> 6]);
         L.store(k, res, dists, (size_t)q, lane);
     };
@@ -446,9 +447,9 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
                                         whi, r0, lo, 0, 0, a.stop);
             if (active) {
                 bool r = false;
-                if constexpr (FPK) r = h.tied() || (SEEDED && h.missing(kk));
+                if constexpr (FPK) r = h.tied() || ((SEEDED || a.full) && h.missing(kk));
                 else if constexpr (PACKED) r = h.needs_exact(kk);
-                else if constexpr (SEEDED) r = h.missing(kk) > 0;
+                else r = (SEEDED || a.full) && h.missing(kk) > 0;
                 redo = redo || r;
                 if constexpr (FPK) {
                     int bad = 0;
@@ -1224,16 +1225,16 @@ static inline int bit_length(uint64_t v) {
 // 0.3 ms with one wave each).
 template <typename T, int MK>
 static int launch_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq, int k,
-                         int excl, const QueryMap &qm, uint64_t *res,
+                         int excl, uint64_t cap, const QueryMap &qm, uint64_t *res,
                          typename CoordTraits<T>::D *d) {
     if (k <= 128) {
         const dim3 g(xcd_grid(std::min<unsigned>(blocks_for(nq, 4), 2048u))), b(256);
         if (k <= 64)
             hipLaunchKernelGGL((wave_knn_kernel<T, 1, MK, true>), g, b, 0, s, dt, qs, nq, k, excl,
-                               qm, res, d, (uint64_t *)nullptr);
+                               cap, qm, res, d, (uint64_t *)nullptr);
         else
             hipLaunchKernelGGL((wave_knn_kernel<T, 2, MK, true>), g, b, 0, s, dt, qs, nq, k, excl,
-                               qm, res, d, (uint64_t *)nullptr);
+                               cap, qm, res, d, (uint64_t *)nullptr);
     } else {
         size_t lds = 0;
         const int lanes = lds_lanes<T>(k, LANE_STACK_CANON, lds);
@@ -1352,8 +1353,8 @@ static uint32_t packet_leaf_limit(int64_t nq, int64_t n, int k, int width, bool 
 // host round trip.  The wave tier answers every query itself.
 template <typename T, int MK>
 static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq, int k,
-                         int excl, int algo, int bucket, int topk, int window, int width,
-                         const uint32_t *order,
+                         int excl, int algo, bool automatic, int bucket, int topk, int window,
+                         int width, const uint32_t *order,
                          const typename CoordTraits<T>::D *seed, uint64_t *res,
                          typename CoordTraits<T>::D *d, uint64_t *stats, const RerunBuf *rr) {
     constexpr bool INTD = !CoordTraits<T>::fp;
@@ -1361,9 +1362,18 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     const uint32_t stop = algo == FT_ALGO_PACKET && !seed && topk != FT_TOPK_LDS_HEAP
                               ? packet_leaf_limit(nq, dt.n, k, width, !qs.qx && !qs.leaf_ids, !INTD)
                               : ~0u;
+    // Neighbours at an infinite distance, or at none (a NaN coordinate): the packet
+    // tier has none, the wave tier puts them after the finite ones.  Which of the
+    // two a call shows follows from its algorithm and k alone, not from the tier
+    // that its numbers of queries and leaves lead to: the automatic choice shows
+    // none up to k = 32 and all above, an explicit one its tier's (exact re-runs of
+    // seeded queries and of full stacks: the wave tier's).
+    const bool none = !INTD && !seed && (automatic ? k <= 32 : algo == FT_ALGO_PACKET);
+    const uint64_t cap = none ? 0x7fefffffffffffffull : ~0ull;  // (the bits of DBL_MAX)
+    const bool full = !INTD && automatic && k > 32 && algo == FT_ALGO_PACKET;
     // (float coordinates' keys are exact: nothing to leave without a seed)
     const bool cuts = INTD || (std::is_same<T, double>::value && k > 1);
-    const bool leaves_slots = algo == FT_ALGO_PACKET ? (cuts || seed || stop != ~0u)
+    const bool leaves_slots = algo == FT_ALGO_PACKET ? (cuts || seed || full || stop != ~0u)
                                                      : algo != FT_ALGO_WAVE;
     if (leaves_slots) {
         if (!rr) {  // the stream's own buffers, grown to nq
@@ -1388,6 +1398,7 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         // 114.7 / 112.7 / 111.9 / 113.8 ms).
         const int spread = qs.leaf_ids ? (int)std::min<int64_t>(4, std::max<int64_t>(1, dt.n / std::max(nq, 1))) : 1;
         a.window = window * spread;
+        a.full = full;
         a.stop = stop;
         a.stats = stats;
         // k above 32 with integer coordinates: multi-pass register tier by
@@ -1409,8 +1420,8 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     } else if (algo == FT_ALGO_WAVE) {
         const dim3 g(xcd_grid(blocks_for(nq, 4))), b(256);
 #define FT_WAVE_LAUNCH(S_)                                                                      \
-    hipLaunchKernelGGL((wave_knn_kernel<T, S_, MK>), g, b, 0, s, dt, qs, nq, k, excl, qm, res, d, \
-                       stats)
+    hipLaunchKernelGGL((wave_knn_kernel<T, S_, MK>), g, b, 0, s, dt, qs, nq, k, excl, cap, qm, \
+                       res, d, stats)
         if (k <= 64) FT_WAVE_LAUNCH(1);
         else if (k <= 128) FT_WAVE_LAUNCH(2);
         else if (k <= 256) FT_WAVE_LAUNCH(4);
@@ -1445,7 +1456,7 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
                            (const uint32_t *)rr->count);
         FT_CHECK_LAUNCH();
     }
-    return launch_listed<T, MK>(s, dt, qs, nq, k, excl, qm, res, d);
+    return launch_listed<T, MK>(s, dt, qs, nq, k, excl, cap, qm, res, d);
 }
 
 template <typename T>
@@ -1490,6 +1501,7 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
     if (opts) o = *opts;
     uint64_t *stats = o.stats;
     int algo = o.algorithm;
+    const bool automatic = algo == FT_ALGO_AUTO;
     if (o.mode == FT_MODE_REFERENCE) {
         if (o.seed_bound) return fail(FT_EINVAL, "a seed bound needs canonical mode");
         if (external && k > 32) {
@@ -1556,11 +1568,11 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
     const int width = o.group_width ? o.group_width : (nq < WIDE_PACKETS_FROM ? 32 : 64);
     switch (metric_kind<T>(dt.m)) {
     case MK_WRAP:
-        return run_canonical<T, MK_WRAP>(s, dt, qs, nq, k, excl, algo, bucket, o.topk, window,
-                                         width, order, seed, res, dists, stats, rr);
+        return run_canonical<T, MK_WRAP>(s, dt, qs, nq, k, excl, algo, automatic, bucket, o.topk,
+                                         window, width, order, seed, res, dists, stats, rr);
     case MK_OPEN:
-        return run_canonical<T, MK_OPEN>(s, dt, qs, nq, k, excl, algo, bucket, o.topk, window,
-                                         width, order, seed, res, dists, stats, rr);
+        return run_canonical<T, MK_OPEN>(s, dt, qs, nq, k, excl, algo, automatic, bucket, o.topk,
+                                         window, width, order, seed, res, dists, stats, rr);
     default:
         return fail(FT_EINVAL, "unsupported metric: periodic integer coordinates need B <= 31");
     }

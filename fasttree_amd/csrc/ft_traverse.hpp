@@ -1664,13 +1664,15 @@ template <int S> struct WaveList {
     uint64_t wd;  // the k-th entry (wave-uniform): pruning and admission bound
     uint32_t wi;
     int ks, kl;   // its slot and lane
-    __device__ inline void init(int k) {
+    // cap: distance bits above which nothing is taken (those of the largest
+    // finite distance leave out infinite ones and those that are not numbers).
+    __device__ inline void init(int k, uint64_t cap = ~0ull) {
 #pragma unroll
         for (int s = 0; s < S; ++s) {
-            d[s] = ~0ull;
+            d[s] = cap;
             i[s] = ~0u;
         }
-        wd = ~0ull;
+        wd = cap;
         wi = ~0u;
         ks = (k - 1) >> 6;
         kl = (k - 1) & 63;

@@ -28,10 +28,11 @@ def leaves(tree):
 def squared(q, x, box=0.0):
     """The library's floating-point squared distances: one rounding an operation."""
     d2 = None
-    for a in range(3):
-        d = np.abs(q[a][:, None] - x[a][None, :])
-        d = np.minimum(d, x[a].dtype.type(box) - d) if box else d
-        d2 = d * d if d2 is None else d2 + d * d
+    with np.errstate(over="ignore"):
+        for a in range(3):
+            d = np.abs(q[a][:, None] - x[a][None, :])
+            d = np.minimum(d, x[a].dtype.type(box) - d) if box else d
+            d2 = d * d if d2 is None else d2 + d * d
     return d2.astype(np.float64)
 
 
@@ -93,3 +94,45 @@ def test_a_query_that_is_not_a_number_empties_its_own_row_only(ft, orc, ct, peri
             b.run()
             r, d = r.to_host().reshape(nq, k), d.to_host().reshape(nq, k)
             assert np.array_equal(r[good], want[good]) and np.array_equal(d[good], dist[good])
+
+
+# Few queries (a wave each), many (packets, with and without a leaf limit), and
+# above k = 32 the passes that the automatic choice takes instead of waves
+@pytest.mark.parametrize("name", ["overflow", "not a number"])
+@pytest.mark.parametrize("n,nq", [(200, 50), (200, 160_000), (3000, 200), (3000, 160_000)])
+@pytest.mark.parametrize("ct", FP)
+def test_distances_that_are_not_finite_do_not_depend_on_the_tier(ft, orc, ct, n, nq, name):
+    dt = O.COORD_DTYPES[ct]
+    rng = np.random.default_rng(n + nq)
+    pts = [(rng.random(n) * 100).astype(dt) for _ in range(3)]
+    if name == "overflow":  # five points whose distance to the others is infinite
+        far = np.array(1e160 if ct == O.CT_F64 else 1e25, dt)
+        for a in pts:
+            a[n - 5:] += far
+    else:  # five points with three coordinates each
+        pts[1][5:] = np.nan
+    tree = build(ft, ct, pts)
+    x = leaves(tree)
+    pick = rng.integers(0, n, nq)
+    pick[:40] = np.flatnonzero(np.isfinite(x[1]) & (x[1] > 1000 if name == "overflow" else x[1] < 200))[
+        rng.integers(0, 5, 40)]
+    q = [np.ascontiguousarray(a[pick]) for a in x]
+    rows = np.unique(np.r_[:40, rng.integers(0, nq, 300)])
+    d2 = squared([a[rows] for a in q], x)
+    ids = np.arange(n, dtype=np.int32)
+    for k in (4, 8, 32):
+        want, dist = nearest(d2, k)
+        r, d = ft.knn_query(tree, *q, k)
+        assert np.array_equal(r[rows], want) and np.array_equal(d[rows], dist)
+        for call in (lambda **o: ft.self_knn_query(tree, k, **o),
+                     lambda **o: ft.self_knn_query_subset(tree, ids, k, **o)):
+            # (the per-lane tier tests a leaf as a box, which drops a NaN axis)
+            tiers = [ft.ALGO_PACKET] + [ft.ALGO_PLAIN] * (name == "overflow")
+            for a, b in ((call(), call(algorithm=t)) for t in tiers):
+                assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    for k in (33, 64):  # the wave tier's rows: every point, those last
+        for call in (lambda **o: ft.knn_query(tree, *q, k, **o),
+                     lambda **o: ft.self_knn_query(tree, k, max_k=64, **o),
+                     lambda **o: ft.self_knn_query_subset(tree, ids, k, **o)):
+            a, b = call(), call(algorithm=ft.ALGO_WAVE)
+            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1], equal_nan=True)
