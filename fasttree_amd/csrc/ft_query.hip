@@ -332,7 +332,8 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
         const int self = excl ? rank : -1;
         const int anchor = rank >= 0 ? rank : descend_rank_v<T, MK>(t, px, py, pz);
         WaveList<S> L;
-        L.init(k, cap);
+        // (integer distances and k above 128 have no cap: constant there)
+        L.init(k, CoordTraits<T>::fp && S <= 2 ? cap : ~0ull);
         wave_walk<T, S, MK>(t, px, py, pz, self, anchor, L, c, &wbuf[threadIdx.x >> 6]);
         L.store(k, res, dists, (size_t)q, lane);
     };
@@ -447,9 +448,9 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
                                         whi, r0, lo, 0, 0, a.stop);
             if (active) {
                 bool r = false;
-                if constexpr (FPK) r = h.tied() || ((SEEDED || a.full) && h.missing(kk));
+                if constexpr (FPK) r = h.tied() || ((SEEDED || a.full) && h.unfilled());
                 else if constexpr (PACKED) r = h.needs_exact(kk);
-                else r = (SEEDED || a.full) && h.missing(kk) > 0;
+                else r = (SEEDED || a.full) && h.unfilled();
                 redo = redo || r;
                 if constexpr (FPK) {
                     int bad = 0;

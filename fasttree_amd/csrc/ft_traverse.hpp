@@ -465,6 +465,7 @@ template <typename D, int M> struct TopK {
             }
         }
     }
+    __device__ inline bool unfilled() const { return i[M - 1] == INT32_MAX; }
     // Number of live slots still holding the initial sentinel.
     __device__ inline int missing(int k) const {
         int c = 0;
@@ -677,6 +678,8 @@ template <int M> struct KeySlots {
         return kept;
     }
     __device__ inline bool empty(int s) const { return (key[s] & imask) == imask; }
+    // The last slot is empty, i.e. any is (they are sorted).
+    __device__ inline bool unfilled() const { return empty(M - 1); }
     // A live slot is still empty.
     __device__ inline bool missing(int k) const {
         bool bad = false;
