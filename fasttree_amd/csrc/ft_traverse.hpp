@@ -587,13 +587,15 @@ __device__ __forceinline__ double key_f64(uint64_t k) { return __longlong_as_dou
 __device__ __forceinline__ uint64_t key_u64(double k) { return (uint64_t)__double_as_longlong(k); }
 
 // The M sorted key slots and what works on whole keys.
-template <int M> struct KeySlots {
+// WIDE: keys up to the largest finite double (below BIAS + 2^61 otherwise).
+template <int M, bool WIDE = false> struct KeySlots {
     static constexpr bool kPacked = true;
     static constexpr bool kSortFill = true;
     // insertion rounds per trip of the leaf loop (measured: two from 32 slots)
     static constexpr int kRoundsPerTrip = M >= 32 ? 2 : 1;
     static constexpr uint64_t BIAS = 1ull << 62;
-    static constexpr uint64_t NOKEY = BIAS | (1ull << 61);  // above every key, still finite
+    // above every key, still finite
+    static constexpr uint64_t NOKEY = WIDE ? 0x7fefffffffffffffull : BIAS | (1ull << 61);
     uint64_t key[M];
     uint64_t imask;  // the index bits; all ones: an empty slot
     // The k live slots start as the sentinel `sent`.
@@ -748,8 +750,10 @@ template <int M> struct TopKPacked : KeySlots<M> {
 // costs the same two instructions a slot (a compare, a lexicographic tie test
 // and three selects before: 7).  Non-negative doubles and floats order as
 // their bit patterns do.
-//  * float coordinates: every squared distance is a float, so BIAS | its 31
-//    bits << 30 | index holds it exactly (indices are below 2^30 - 1).
+//  * float coordinates: every squared distance is a float, so BIAS + its 31
+//    bits << 31 | index holds it exactly, with any index that a caller may give
+//    (ft_build_tree: up to 2^31 - 2).  Read as a double, the key of a finite
+//    distance has an exponent field of at most 0x7FB.
 //  * double coordinates: BIAS | the top 61 - ib of the distance's 63 bits << ib
 //    | leaf rank.  The low ib + 2 bits (at most 32 of the 52 of the mantissa)
 //    are cut off, so keys order distances that differ above the cut; bounds
@@ -763,13 +767,13 @@ template <int M> struct TopKPacked : KeySlots<M> {
 //    mantissa: about one query in 100,000); where they are common, on a regular
 //    grid, the packet kernel hands whole packets to its exact instantiation.
 // ---------------------------------------------------------------------------
-template <typename T, int M> struct TopKFp : KeySlots<M> {
-    using B = KeySlots<M>;
+template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>::value> {
+    using B = KeySlots<M, std::is_same<T, float>::value>;
     using B::key;
     using B::imask;
     static constexpr bool kCut = std::is_same<T, double>::value;
     static constexpr bool kRankKeys = kCut;  // keys hold leaf ranks, not returned indices
-    static constexpr int kFloatShift = 30;
+    static constexpr int kFloatShift = 31;
     uint64_t rejected;  // kCut only
     __device__ inline uint64_t pack(double d, uint64_t i) const {
         if constexpr (kCut) return B::BIAS | (((uint64_t)__double_as_longlong(d) >> 2) & ~imask) | i;

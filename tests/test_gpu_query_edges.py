@@ -136,3 +136,32 @@ def test_distances_that_are_not_finite_do_not_depend_on_the_tier(ft, orc, ct, n,
                      lambda **o: ft.self_knn_query_subset(tree, ids, k, **o)):
             a, b = call(), call(algorithm=ft.ALGO_WAVE)
             assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1], equal_nan=True)
+
+
+# build_tree takes the original indices from its caller: any that an int32 holds
+@pytest.mark.parametrize("base", [0, (1 << 30) - 250, (1 << 31) - 501])
+@pytest.mark.parametrize("ct", FP)
+def test_original_indices_of_any_size(ft, orc, ct, base):
+    n, dt = 500, O.COORD_DTYPES[ct]
+    rng = np.random.default_rng(3)
+    pts = [(rng.random(n) * 100).astype(dt) for _ in range(3)]
+    for a in pts:
+        a[::5] = a[0]  # ties, ordered by the index
+    cfg = ft.Config(sfc=O.SFC_MORTON, bits_per_dim=21, return_orig_indices=True)
+    key = ft.sfc_encode(*pts, cfg, bbox=ft.compute_bbox(*pts))
+    o = np.argsort(key, kind="stable")
+    s = [np.ascontiguousarray(a[o]) for a in pts]
+    orig = (rng.permutation(n) + base).astype(np.int32)
+    tree = ft.TreeSoA(n, ct, cfg)
+    dev = ft.DeviceArray.from_host
+    ft.build_tree(tree, dev(key[o]), *(dev(a) for a in s), dev(np.arange(n, dtype=np.uint32)),
+                  dev(np.zeros(n, np.int8)), dev(orig))
+    d2 = squared(s, s)
+    d2[np.arange(n), np.arange(n)] = np.inf
+    col = np.argsort(orig)
+    for k in (1, 4, 8, 16, 32, 64):
+        want, dist = nearest(d2[:, col], k)
+        want = orig[col][want.astype(np.int64)]
+        for algo in (ft.ALGO_PACKET, ft.ALGO_AUTO):
+            r, d = ft.self_knn_query(tree, k, max_k=64, algorithm=algo)
+            assert np.array_equal(d, dist) and np.array_equal(r, want.astype(np.uint64))
