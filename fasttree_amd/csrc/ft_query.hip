@@ -1376,11 +1376,12 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     const bool cuts = INTD || (std::is_same<T, double>::value && k > 1);
     const bool leaves_slots = algo == FT_ALGO_PACKET ? (cuts || seed || full || stop != ~0u)
                                                      : algo != FT_ALGO_WAVE;
+    if (!rr) {  // the stream's own buffers, grown to nq (also where this call leaves
+                // nothing: see query_order_ensure)
+        FT_TRY(rerun_ensure(s, (size_t)nq));
+        rr = &stream_bufs(s).rr;
+    }
     if (leaves_slots) {
-        if (!rr) {  // the stream's own buffers, grown to nq
-            FT_TRY(rerun_ensure(s, (size_t)nq));
-            rr = &stream_bufs(s).rr;
-        }
         hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, s, rr->count);
     }
     const QueryMap qm{order, leaves_slots ? rr->list : nullptr, leaves_slots ? rr->count : nullptr,
@@ -1460,9 +1461,11 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
     return launch_listed<T, MK>(s, dt, qs, nq, k, excl, cap, qm, res, d);
 }
 
-template <typename T>
-static int query_order(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq,
-                       const uint32_t *&order) {
+// The stream's buffers for ordering nq queries.  Every call that may order its
+// queries makes sure of them, also one that leaves them as they are: a call
+// captured later, which may not grow a buffer, then finds them large enough
+// whichever tier either of the two takes.
+static int query_order_ensure(hipStream_t s, int nq) {
     StreamBufs &sb = stream_bufs(s);
     QueryOrderBuf &g_qorder = sb.qo;
     if (g_qorder.cap < (size_t)nq) {
@@ -1482,6 +1485,14 @@ static int query_order(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int
         g_qorder.S.block = nullptr;
         g_qorder.S.cap_n = 0;
     }
+    return scratch_ensure_public(g_qorder.S, (size_t)nq);
+}
+
+template <typename T>
+static int query_order(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq,
+                       const uint32_t *&order) {
+    FT_TRY(query_order_ensure(s, nq));
+    QueryOrderBuf &g_qorder = stream_bufs(s).qo;
     hipLaunchKernelGGL((query_key_kernel<T>), dim3(blocks_for(nq, 256)), dim3(256), 0, s, dt, qs,
                        nq, g_qorder.keys);
     FT_CHECK_LAUNCH();
@@ -1557,8 +1568,10 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
     const int bucket = o.leaf_bucket > 0 ? std::min(o.leaf_bucket, 64) : 64;
     const uint32_t *order = nullptr;
     if (algo == FT_ALGO_WAVE && k > WAVE_MAX_K) algo = FT_ALGO_GROUPED;
-    if ((algo == FT_ALGO_PACKET || algo == FT_ALGO_WAVE) && (qs.qx || qs.leaf_ids) && nq > (algo == FT_ALGO_WAVE ? UNORDERED_WAVES : 64))
-        FT_TRY(query_order<T>(s, dt, qs, nq, order));
+    if ((algo == FT_ALGO_PACKET || algo == FT_ALGO_WAVE) && (qs.qx || qs.leaf_ids) && nq > 64) {
+        if (algo == FT_ALGO_WAVE && nq <= UNORDERED_WAVES) FT_TRY(query_order_ensure(s, nq));
+        else FT_TRY(query_order<T>(s, dt, qs, nq, order));
+    }
     // auto: 192 leaves on each side (self k = 32 at 10M clustered points: 64 /
     // 128 / 192 / 256 / 384 took 19.17 / 18.93 / 18.80 / 18.77 / 18.81 ms;
     // 192 was also as fast or faster at k = 1 to 64, for subsets and for
@@ -1665,6 +1678,7 @@ template <typename T, int MK>
 static int range_walk(hipStream_t s, const DTree<T> &dt, const RangeSrc<T> &src, int nq,
                       const RangeOut &out) {
     if (few_range_queries(nq, dt.n)) {
+        FT_TRY(query_order_ensure(s, nq));
         const QueryMap qm{nullptr, nullptr, nullptr, nullptr};
         hipLaunchKernelGGL((range_wave_kernel<T, MK, false>), dim3(xcd_grid(blocks_for(nq, 4))),
                            dim3(256), 0, s, dt, src, nq, qm, out);

@@ -165,3 +165,52 @@ def test_original_indices_of_any_size(ft, orc, ct, base):
         for algo in (ft.ALGO_PACKET, ft.ALGO_AUTO):
             r, d = ft.self_knn_query(tree, k, max_k=64, algorithm=algo)
             assert np.array_equal(d, dist) and np.array_equal(r, want.astype(np.uint64))
+
+
+# A first call on the stream is small; the second sizes the buffers and takes a
+# wave per query (or leaves no slot); the captured one takes packets
+@pytest.mark.parametrize("name", ["sorted waves", "unsorted waves", "float packets", "range"])
+def test_buffers_fit_a_captured_call_of_another_tier(ft, orc, name):
+    rng = np.random.default_rng(7)
+    ct = O.CT_F32 if name == "float packets" else O.CT_U64
+    dt = O.COORD_DTYPES[ct]
+    pts = [rng.integers(0, 1 << 21, 200_000).astype(dt) for _ in range(3)]
+    tree = build(ft, ct, pts)
+    nq = {"sorted waves": 60_000, "unsorted waves": 20_000, "float packets": 170_000}.get(name, 20_000)
+    q = [ft.DeviceArray.from_host(rng.integers(0, 1 << 21, nq).astype(dt)) for _ in range(3)]
+    s = ft.Stream()
+    if name == "range":
+        few = build(ft, ct, [a[:300] for a in pts])  # 20,000 queries of 300 points: packets
+        r = [ft.DeviceArray.from_host(np.full(nq, v, dt)) for v in (0, 200_000)]
+        out = ft.DeviceArray(nq * 30, np.int32), ft.DeviceArray(nq, np.int32)
+        call = lambda: ft.range_query(few, *q, *r, 30, *out, stream=s)
+        warm = lambda: ft.range_query(tree, *q, *r, 30, *out, stream=s)
+    else:
+        out = ft.DeviceArray(nq * 32, np.uint64), ft.DeviceArray(nq * 32, ft.dist_dtype(ct))
+        pk = ft.ALGO_PACKET
+        call = lambda: ft.knn_query(tree, *q, 8, *out, stream=s, algorithm=pk)
+        if name == "float packets":
+            warm = lambda: ft.knn_query(tree, *q, 1, *out, stream=s, algorithm=ft.ALGO_WAVE)
+        else:
+            warm = lambda: ft.knn_query(tree, *q, 32 if name == "sorted waves" else 8, *out, stream=s)
+    small = [ft.DeviceArray.from_host(rng.integers(0, 1 << 21, 300).astype(dt)) for _ in range(3)]
+    tmp = ft.DeviceArray(2400, np.uint64), ft.DeviceArray(2400, ft.dist_dtype(ct))
+    ft.knn_query(tree, *small, 8, *tmp, stream=s, algorithm=ft.ALGO_PACKET)
+    warm()
+    s.synchronize()
+    with ft.Graph(s) as g:
+        call()
+    used = nq if name == "range" else nq * 8
+    got = []
+    for _ in range(3):
+        for a in out:
+            a.zero()
+        g.launch()
+        s.synchronize()
+        got.append([a.to_host()[:used] for a in out])
+    call()
+    s.synchronize()
+    want = [a.to_host()[:used] for a in out]
+    for rows in got:
+        assert np.array_equal(rows[1], want[1])
+        assert name == "range" or np.array_equal(rows[0], want[0])
