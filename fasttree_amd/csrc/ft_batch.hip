@@ -201,7 +201,9 @@ __global__ __launch_bounds__(64) void batch_packet_kernel(BatchView<T> b,
         const int r0 = run_start(descend_rank<T, MK>(t, rl(px, src), rl(py, src), rl(pz, src)), t.n);
         const int wlo = r0 - BATCH_WINDOW > 0 ? r0 - BATCH_WINDOW : 0;
         const int whi = r0 + 64 + BATCH_WINDOW < t.n ? r0 + 64 + BATCH_WINDOW : t.n;
-        bool redo = false;
+        // lanes left to the exact pass, as a mask of the wave (packet_knn_kernel)
+        const uint64_t act = __ballot(active);
+        uint64_t redo = 0;
         static_assert(!MULTI || !HEAP, "passes need the register tier");
         if constexpr (MULTI) {
             // k above M: passes of M, each above the previous pass's last key.
@@ -214,12 +216,10 @@ __global__ __launch_bounds__(64) void batch_packet_kernel(BatchView<T> b,
                 // one walk instance for every pass (the first with floor 0)
                 packet_walk<T, H, MK, true>(t, q.bucket, active, px, py, pz, -1, h, stk, c, wlo,
                                             whi, r0, lo);
-                if (active) {
-                    if constexpr (PACKED) redo = redo || h.needs_exact(kk);
-                    if (!redo)
-                        h.store_part(kk, b.res + q.result_first, b.dists + q.result_first,
-                                     (size_t)local, k, base);
-                }
+                if constexpr (PACKED) redo |= __ballot(h.needs_exact(kk)) & act;
+                if (((act & ~redo) >> lane) & 1)
+                    h.store_part(kk, b.res + q.result_first, b.dists + q.result_first,
+                                 (size_t)local, k, base);
                 lo = h.next_floor();
             }
         } else {
@@ -228,13 +228,11 @@ __global__ __launch_bounds__(64) void batch_packet_kernel(BatchView<T> b,
             if constexpr (PACKED) h.init(k, ~0ull, 32 - __clz(t.n));
             else h.init(k, dist_max<D>());
             packet_walk<T, H, MK>(t, q.bucket, active, px, py, pz, -1, h, stk, c, wlo, whi, r0);
-            if (active) {
-                if constexpr (PACKED) redo = h.needs_exact(k);
-                if (!redo)
-                    h.store(k, b.res + q.result_first, b.dists + q.result_first, (size_t)local);
-            }
+            if constexpr (PACKED) redo = __ballot(h.needs_exact(k)) & act;
+            if (((act & ~redo) >> lane) & 1)
+                h.store(k, b.res + q.result_first, b.dists + q.result_first, (size_t)local);
         }
-        if (active && redo) {
+        if ((redo >> lane) & 1) {
             const uint32_t s2 = atomicAdd(b.rerun_count, 1u);
             if (s2 < b.rerun_cap) b.rerun[s2] = q.entry_first + e;
         }

@@ -44,22 +44,21 @@ struct QueryMap {
     int32_t *packets;       // direct passes of cut keys: packets left whole, appended
 };
 
-// Appends the wave's slots with `left` set, one atomic per wave.  `rerun`: they
-// count as exact re-runs (a query the direct pass could not answer exactly,
-// rather than a packet handed over).  Called by whole waves.
-__device__ inline void append_slots(const QueryMap &qm, bool left, int slot, bool rerun) {
-    const uint64_t m = __ballot(left);
-    if (!m) return;
+// Appends the slots of the lanes in `left` (a wave mask), one atomic per wave.
+// `rerun`: they count as exact re-runs (queries the direct pass could not answer
+// exactly, rather than a packet handed over).  Called by whole waves.
+__device__ inline void append_slots(const QueryMap &qm, uint64_t left, int slot, bool rerun) {
+    if (!left) return;
     const int lane = threadIdx.x & 63;
     uint32_t base = 0;
     if (lane == 0) {
-        base = atomicAdd(&qm.count[0], (uint32_t)__popcll(m));
-        if (rerun) atomicAdd(&qm.count[1], (uint32_t)__popcll(m));
+        base = atomicAdd(&qm.count[0], (uint32_t)__popcll(left));
+        if (rerun) atomicAdd(&qm.count[1], (uint32_t)__popcll(left));
     }
     base = (uint32_t)uni((int)base);
-    if (left)
-        qm.list[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
-                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = slot;
+    if ((left >> lane) & 1)
+        qm.list[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(left >> 32),
+                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)left, 0u))] = slot;
 }
 
 __device__ inline void append_packet(const QueryMap &qm, int blk) {
@@ -96,7 +95,7 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_reg_kernel(
     const bool ovf = lane_reg_walk<T, M, GROUPED, STACK_DEPTH, MK>(
         t, active, px, py, pz, self, h, stk, LANE_BLOCK, lane, visits, inserts);
     if (active && !ovf) h.store(k, res, dists, (size_t)q);
-    append_slots(qm, active && ovf, slot, true);
+    append_slots(qm, __ballot(active && ovf), slot, true);
     wave_add_stats(stats, 0, visits);
     wave_add_stats(stats, 4, inserts);
 }
@@ -145,7 +144,7 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_lds_kernel(
                 }
             }
         }
-        if constexpr (!REF && !LISTED) append_slots(qm, left, slot, true);
+        if constexpr (!REF && !LISTED) append_slots(qm, __ballot(left), slot, true);
         if (!LISTED) break;
     }
     wave_add_stats(stats, 0, visits);
@@ -410,6 +409,9 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     if (active) load_query(t, qs, q, px, py, pz, self);
     const int rank = self;  // the query's leaf rank (self queries), else -1
     if (!a.excl) self = -1;
+    // Which queries are left to the listed pass is kept as masks of the wave, voted
+    // outside divergent branches.
+    const uint64_t act = __ballot(active);
     // Window pre-scan.  Self queries over all leaves: the packet is leaf ranks
     // [r0, r0 + 64), so its neighbours along the curve are the leaves on
     // either side.  Subset and external queries (Morton-ordered, so a
@@ -430,7 +432,8 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
         // k above M (register tier): ceil(k / M) passes, each taking the M
         // nearest (d2, index) above the previous pass's last one, stored in
         // place.
-        bool redo = false, whole = false;
+        uint64_t redo = 0;  // lanes left to the listed pass
+        bool whole = false;
         typename H::Floor lo = H::no_floor();
         for (int base = 0; base < k; base += M) {
             const int kk = k - base < M ? k - base : M;
@@ -446,32 +449,25 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             // one walk instance for every pass (the first with no floor)
             packet_walk<T, H, MK, true>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo,
                                         whi, r0, lo, 0, 0, a.stop);
-            if (active) {
-                bool r = false;
-                if constexpr (FPK) r = h.tied() || ((SEEDED || a.full) && h.unfilled());
-                else if constexpr (PACKED) r = h.needs_exact(kk);
-                else r = (SEEDED || a.full) && h.unfilled();
-                redo = redo || r;
-                if constexpr (FPK) {
-                    int bad = 0;
-                    if (!redo) {
-                        bad = h.template store_row<MK>(kk, res, dists, (size_t)q, k, base, t, px,
-                                                       py, pz);
-                        asm volatile("" : "+v"(bad));
-                    }
-                    redo = redo || bad != 0;
-                } else {
-                    if (!redo) h.store_part(kk, res, dists, (size_t)q, k, base);
-                }
-            }
+            bool r = false;
+            if constexpr (FPK) r = h.tied() | ((SEEDED || a.full) && h.unfilled());
+            else if constexpr (PACKED) r = h.needs_exact(kk);
+            else r = (SEEDED || a.full) && h.unfilled();
+            redo |= __ballot(r) & act;
+            const bool row = ((act & ~redo) >> lane) & 1;
+            if constexpr (FPK)
+                redo |= act & __ballot(h.template store_row<MK>(row, kk, res, dists, (size_t)q, k,
+                                                                base, t, px, py, pz));
+            else if (row) h.store_part(kk, res, dists, (size_t)q, k, base);
             lo = h.next_floor();
             if constexpr (H::kRankKeys) {
-                whole = !SEEDED && __popcll(__ballot(redo)) >= TIED_LANES;
+                whole = !SEEDED && __popcll(redo) >= TIED_LANES;
                 if (whole) break;
             }
         }
-        if (whole) append_packet(qm, blk);
-        else append_slots(qm, active && (redo || c.leaves > a.stop), slot, c.leaves <= a.stop);
+        const bool over = c.leaves > a.stop;
+        if (whole && !over) append_packet(qm, blk);
+        else append_slots(qm, over ? act : redo, slot, !over);
     } else {
         H h;
         if constexpr (HEAP) h.key = heap_mem;
@@ -496,29 +492,19 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
         }
         packet_walk<T, H, MK>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo, whi, r0,
                               H::no_floor(), flo, fhi, a.stop);
-        bool left = false;
-        if (active) {
-            left = c.leaves > a.stop;
-            if constexpr (FPK) left = left || h.tied() || (SEEDED && h.missing(k));
-            else if constexpr (PACKED) left = left || h.needs_exact(k);
-            else if constexpr (SEEDED) left = left || h.missing(k) > 0;
-            if constexpr (!FPK) {
-                if (!left) h.store(k, res, dists, (size_t)q);
-            }
-        }
-        if constexpr (FPK) {
-            // (a 32-bit word kept opaque: as a lane mask, the lanes that had
-            // left before this branch lost their bit in it)
-            int bad = 0;
-            if (active && !left) {
-                bad = h.template store_row<MK>(k, res, dists, (size_t)q, k, 0, t, px, py, pz);
-                asm volatile("" : "+v"(bad));
-            }
-            left = left || bad != 0;
-        }
-        if (H::kRankKeys && c.leaves <= a.stop && __popcll(__ballot(left)) >= TIED_LANES && !SEEDED)
-            append_packet(qm, blk);
-        else append_slots(qm, left, slot, c.leaves <= a.stop);
+        const bool over = c.leaves > a.stop;
+        bool r = false;
+        if constexpr (FPK) r = h.tied() | (SEEDED && h.unfilled());
+        else if constexpr (PACKED) r = h.needs_exact(k);
+        else if constexpr (SEEDED) r = h.unfilled();
+        uint64_t left = over ? act : __ballot(r) & act;
+        const bool row = ((act & ~left) >> lane) & 1;
+        if constexpr (FPK)
+            left |= act & __ballot(h.template store_row<MK>(row, k, res, dists, (size_t)q, k, 0, t,
+                                                            px, py, pz));
+        else if (row) h.store(k, res, dists, (size_t)q);
+        if (H::kRankKeys && !SEEDED && !over && __popcll(left) >= TIED_LANES) append_packet(qm, blk);
+        else append_slots(qm, left, slot, !over);
     }
     if (lane == 0 && a.stats) {
         atomicAdd((unsigned long long *)&a.stats[0], (unsigned long long)c.nodes);
@@ -1782,7 +1768,7 @@ __global__ __launch_bounds__(256) void csr_copy_kernel(const int32_t *__restrict
 __global__ __launch_bounds__(256) void csr_overflow_kernel(const int32_t *__restrict__ counts,
                                                            int nq, QueryMap qm) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    append_slots(qm, q < nq && counts[q] > CSR_POOL, q, false);
+    append_slots(qm, __ballot(q < nq && counts[q] > CSR_POOL), q, false);
 }
 
 int scan_entry(hipStream_t s, const int32_t *counts, int nq, int64_t *row_ptr);

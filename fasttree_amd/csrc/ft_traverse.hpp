@@ -719,8 +719,8 @@ template <int M> struct TopKPacked : KeySlots<M> {
     __device__ inline bool beats_worst(uint64_t d, int32_t i) const { return make(d, i) < key[M - 1]; }
     __device__ inline void insert(bool take, uint64_t d, int32_t i) { B::insert_key(take, make(d, i)); }
     // Sentinels left in live slots, or a saturated k-th distance.
-    __device__ inline bool needs_exact(int k) const {
-        return (dist_of(key[M - 1]) >= sat) | B::missing(k);
+    __device__ inline bool needs_exact(int) const {
+        return (dist_of(key[M - 1]) >= sat) | B::unfilled();
     }
     __device__ inline uint64_t floor_d(uint64_t lo) const { return dist_of(lo); }
     __device__ inline bool above(uint64_t lo, uint64_t d, int32_t i) const { return make(d, i) >= lo; }
@@ -822,11 +822,12 @@ template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>:
             any |= (s > M - k) & (((key[s] ^ key[s - 1]) & ~imask) == 0) & !B::empty(s);
         return any;
     }
-    // Entries [base, base + k) of row q (row length k_row); double coordinates
-    // recompute them.  Returns true if they are not in (d, index) order.
+    // Entries [base, base + k) of row q (row length k_row), written by the lanes
+    // with `row`; double coordinates recompute them.  Every lane of the wave calls
+    // it and is told whether its entries are out of (d, index) order.
     template <int MK, typename Tr>
-    __device__ inline bool store_row(int k, uint64_t *res, double *dists, size_t q, int k_row,
-                                     int base, const Tr &t, T px, T py, T pz) const {
+    __device__ inline bool store_row(bool row, int k, uint64_t *res, double *dists, size_t q,
+                                     int k_row, int base, const Tr &t, T px, T py, T pz) const {
         const size_t o = q * (size_t)k_row + (size_t)base;
         const int off = t.n - 1;
         bool bad = false;
@@ -849,8 +850,10 @@ template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>:
                 } else {
                     d = d_hi(key[s]);
                 }
-                res[j] = ok ? (uint64_t)(uint32_t)i : ~0ull;
-                dists[j] = ok ? d : missing_dist<double>();
+                if (row) {
+                    res[j] = ok ? (uint64_t)(uint32_t)i : ~0ull;
+                    dists[j] = ok ? d : missing_dist<double>();
+                }
             }
         }
         return bad;
@@ -1484,6 +1487,8 @@ __device__ inline int run_start(int rc, int n) {
 //    key, 32-bit index) can fill, so results never depend on the stack size.
 // GROUPED: the wave skips a node unless some active lane still needs it
 // (any_of_group, src/hlbvh.hpp:1563-1566); results do not depend on it.
+// Overflows are counted, not flagged: a lane's flag that is set between wave
+// votes is what the structurizer option in build.py does not keep.
 // ---------------------------------------------------------------------------
 template <typename T, int M, bool GROUPED, int DEPTH, int MK>
 __device__ __forceinline__ bool lane_reg_walk(const DTree<T> &t, bool active, T px, T py, T pz,
@@ -1493,7 +1498,7 @@ __device__ __forceinline__ bool lane_reg_walk(const DTree<T> &t, bool active, T 
                                               int wlo = 0, int whi = 0) {
     using D = typename CoordTraits<T>::D;
     const int n = t.n;
-    bool overflow = false;
+    int overflow = 0;
     int sp = 0;
     if (active) stk[(sp++) * lanes + lane] = 0;
     while (sp > 0) {
@@ -1527,11 +1532,11 @@ __device__ __forceinline__ bool lane_reg_walk(const DTree<T> &t, bool active, T 
                     stk[(sp++) * lanes + lane] = r;
                 }
             } else {
-                overflow = true;
+                ++overflow;
             }
         }
     }
-    return overflow;
+    return overflow != 0;
 }
 
 template <typename T, bool REF, bool GROUPED, int DEPTH, int MK>
@@ -1543,7 +1548,7 @@ __device__ __forceinline__ bool lane_heap_walk(const DTree<T> &t, int k, bool ac
                                                uint64_t &inserts) {
     using D = typename CoordTraits<T>::D;
     const int n = t.n;
-    bool overflow = false;
+    int overflow = 0;
     int sp = 0;
     if (active) stk[(sp++) * lanes + lane] = 0;
     while (sp > 0) {
@@ -1574,11 +1579,11 @@ __device__ __forceinline__ bool lane_heap_walk(const DTree<T> &t, int k, bool ac
             } else if (REF) {
                 ++drops;
             } else {
-                overflow = true;
+                ++overflow;
             }
         }
     }
-    return overflow;
+    return overflow != 0;
 }
 
 

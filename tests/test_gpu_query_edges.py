@@ -214,3 +214,28 @@ def test_buffers_fit_a_captured_call_of_another_tier(ft, orc, name):
     for rows in got:
         assert np.array_equal(rows[1], want[1])
         assert name == "range" or np.array_equal(rows[0], want[0])
+
+
+# Seeded queries whose distances tie: seeds that hold too few neighbours, the k-th
+# distance itself and more, one lane beside the other
+@pytest.mark.parametrize("k", [4, 8, 16, 32, 64])
+@pytest.mark.parametrize("name", ["grid", "rounded grid"])
+@pytest.mark.parametrize("ct", FP)
+def test_seeds_on_tied_distances(ft, orc, ct, name, k):
+    i = np.arange(3375)
+    pts = [(i // 225).astype(float), (i // 15 % 15).astype(float), (i % 15).astype(float)]
+    if name == "rounded grid":  # equal but for the last bits
+        pts = [a * 0.1 + 0.05 for a in pts]
+    pts = [a.astype(O.COORD_DTYPES[ct]) for a in pts]
+    side = 15.0 if name == "grid" else 1.5
+    for periodic in (0, 1):
+        tree = build(ft, ct, pts, periodic, side if periodic else 0.0)
+        t = O.build_bvh(ct, *pts, sfc=O.SFC_PH, bits=21, periodic=periodic,
+                        box=side if periodic else 0.0)
+        rb, db = O.knn_bruteforce(t, k, True)
+        rng = np.random.default_rng(k)
+        for share in (0.0, 0.02, 0.4):  # of the seeds too small
+            seed = db[:, -1] * rng.choice([1.0, 1.5, 4.0], len(i))
+            seed = np.where(rng.random(len(i)) < share, db[:, k // 2] * 0.5, seed)
+            r, d = ft.self_knn_query(tree, k, max_k=64, seed_bound=ft.DeviceArray.from_host(seed))
+            assert np.array_equal(d, db) and np.array_equal(r, rb)
