@@ -322,15 +322,8 @@ __global__ __launch_bounds__(64) void batch_wave_kernel(BatchView<T> b,
             const int anchor = descend_rank_v<T, MK>(t, px, py, pz);
             WaveList<S> L;
             L.init(q.k);
-            if (wave_walk<T, S, MK>(t, px, py, pz, -1, anchor, L, c, &wbuf)) {
-                if (lane == 0) {
-                    const uint32_t s2 = atomicAdd(b.rerun_count, 1u);
-                    if (s2 < b.rerun_cap) b.rerun[s2] = q.entry_first + e;
-                }
-            } else {
-                L.store(q.k, b.res + q.result_first, b.dists + q.result_first, (size_t)local,
-                        lane);
-            }
+            wave_walk<T, S, MK>(t, px, py, pz, -1, anchor, L, c, &wbuf);
+            L.store(q.k, b.res + q.result_first, b.dists + q.result_first, (size_t)local, lane);
         }
     }
     if (lane == 0 && b.stats) {

@@ -332,8 +332,9 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
         const int anchor = rank >= 0 ? rank : descend_rank_v<T, MK>(t, px, py, pz);
         WaveList<S> L;
         // (integer distances and k above 128 have no cap: constant there)
-        L.init(k, CoordTraits<T>::fp && S <= 2 ? cap : ~0ull);
-        wave_walk<T, S, MK>(t, px, py, pz, self, anchor, L, c, &wbuf[threadIdx.x >> 6]);
+        const uint64_t top = CoordTraits<T>::fp && S <= 2 ? cap : ~0ull;
+        L.init(k, top);
+        wave_walk<T, S, MK>(t, px, py, pz, self, anchor, L, c, &wbuf[threadIdx.x >> 6], top);
         L.store(k, res, dists, (size_t)q, lane);
     };
     if constexpr (LISTED) {

@@ -1679,6 +1679,11 @@ template <int S> struct WaveList {
     // cap: distance bits above which nothing is taken (those of the largest
     // finite distance leave out infinite ones and those that are not numbers).
     __device__ inline void init(int k, uint64_t cap = ~0ull) {
+        clear(cap);
+        ks = (k - 1) >> 6;
+        kl = (k - 1) & 63;
+    }
+    __device__ inline void clear(uint64_t cap) {
 #pragma unroll
         for (int s = 0; s < S; ++s) {
             d[s] = cap;
@@ -1686,8 +1691,6 @@ template <int S> struct WaveList {
         }
         wd = cap;
         wi = ~0u;
-        ks = (k - 1) >> 6;
-        kl = (k - 1) & 63;
     }
     __device__ inline void refresh() {
         uint64_t xd = d[0];
@@ -1788,12 +1791,13 @@ struct WaveBuf {
 // the results (-1: none); anchor = a leaf rank near the query (-1: none).
 // The 64 (S + 2) leaves around the anchor are inserted first, so the walk
 // starts with a finite bound; it then skips them (and any subtree inside
-// them).  Returns true if the stack would overflow (never for a tree over
-// distinct (64-bit key, 32-bit index) strings, whose depth is below 97).
+// them).  A tree over distinct (64-bit key, 32-bit index) strings is less than
+// 97 levels deep and never fills the stack; where a deserialised one does, the
+// list (initialised with cap) starts anew over every leaf.
 template <typename T, int S, int MK>
-__device__ __forceinline__ bool wave_walk(const DTree<T> &t, T px, T py, T pz, int self,
+__device__ __forceinline__ void wave_walk(const DTree<T> &t, T px, T py, T pz, int self,
                                           int anchor, WaveList<S> &L, WaveCounters &c,
-                                          WaveBuf *buf) {
+                                          WaveBuf *buf, uint64_t cap = ~0ull) {
     using D = typename CoordTraits<T>::D;
     const int lane = threadIdx.x & 63;
     const int n = t.n;
@@ -1881,17 +1885,18 @@ __device__ __forceinline__ bool wave_walk(const DTree<T> &t, T px, T py, T pz, i
         w1 = w0 + nwin < n ? w0 + nwin : n;
         for (int r0 = w0; r0 < w1; r0 += 64) scan(r0, w1 - r0 < 64 ? w1 - r0 : 64, false);
         flush();
-        if (w0 == 0 && w1 == n) return false;
+        if (w0 == 0 && w1 == n) return;
     }
     if (n <= 64) {
         scan(0, n, true);
         flush();
-        return false;
+        return;
     }
     // stack entry e: lane e & 63 of register (e >> 6)
     uint32_t sn0 = 0, sn1 = 0, sd0l = 0, sd0h = 0, sd1l = 0, sd1h = 0;
     int sp = 0;
     int node = 0;
+    bool full = false;
     while (true) {
         ++c.nodes;
         if (node >= off) {
@@ -1926,7 +1931,10 @@ __device__ __forceinline__ bool wave_walk(const DTree<T> &t, T px, T py, T pz, i
                 const int nn = uni(lfirst ? l : r), fn = uni(lfirst ? r : l);
                 const uint64_t dn = lfirst ? dl : dr, df = lfirst ? dr : dl;
                 if (df <= L.wd) {
-                    if (sp >= 128) return true;
+                    if (sp >= 128) {
+                        full = true;
+                        break;
+                    }
                     const uint32_t lo = (uint32_t)df, hi = (uint32_t)(df >> 32);
                     const bool at = lane == (sp & 63);
                     if (sp < 64) {
@@ -1967,8 +1975,12 @@ __device__ __forceinline__ bool wave_walk(const DTree<T> &t, T px, T py, T pz, i
         }
         if (!found) break;
     }
+    if (full) {
+        L.clear(cap);
+        nbuf = 0;
+        for (int r0 = 0; r0 < n; r0 += 64) scan(r0, n - r0 < 64 ? n - r0 : 64, false);
+    }
     flush();
-    return false;
 }
 
 }  // namespace ft

@@ -239,3 +239,48 @@ def test_seeds_on_tied_distances(ft, orc, ct, name, k):
             seed = np.where(rng.random(len(i)) < share, db[:, k // 2] * 0.5, seed)
             r, d = ft.self_knn_query(tree, k, max_k=64, seed_bound=ft.DeviceArray.from_host(seed))
             assert np.array_equal(d, db) and np.array_equal(r, rb)
+
+
+def list_shaped(ft, tree, order):
+    """`tree` reshaped into a list: internal node i holds leaf i and node i + 1, its
+    leaves in `order` -- a valid tree, as many levels deep as it has leaves."""
+    n = tree.num_leaves
+    ct = tree.coord_type
+    cs, m, buf = np.dtype(O.COORD_DTYPES[ct]).itemsize, 2 * n - 1, bytearray(tree.serialize())
+    sizes = [m * cs] * 6 + [(n - 1) * 4] * 2 + [m * 4, m * 4, m, m * 4, n * 8] + [(n - 1) * 4] * 2
+    at = 64 + 16 + np.r_[0, np.cumsum(sizes)]
+    view = lambda i, dt: np.frombuffer(buf, dt, sizes[i] // np.dtype(dt).itemsize, at[i])
+    for a in range(6):
+        c = view(a, O.COORD_DTYPES[ct])
+        c[n - 1:] = c[n - 1:][order]
+        acc = np.maximum if a % 2 else np.minimum
+        c[:n - 1] = acc.accumulate(c[n - 1:][::-1])[::-1][:n - 1]
+    i = np.arange(n - 1)
+    left, right, parent = view(6, np.int32), view(7, np.int32), view(8, np.int32)
+    left[:], right[:] = n - 1 + i, np.where(i + 1 < n - 1, i + 1, 2 * n - 2)
+    parent[0], parent[left], parent[right] = -1, i, i
+    view(13, np.int32)[:], view(14, np.int32)[:] = i, n - 1
+    return ft.TreeSoA.deserialize(bytes(buf))
+
+
+# A wave's stack holds 128 entries.  Lists of 64 to 1,024 neighbours; the leaves in
+# random order, so that many more than 128 stay within the first bound
+@pytest.mark.parametrize("k", [32, 64, 128, 200, 1000])
+@pytest.mark.parametrize("ct", [O.CT_F64, O.CT_U32])
+def test_trees_deeper_than_a_walk_s_stack(ft, orc, ct, k):
+    rng = np.random.default_rng(k)
+    n, nq, side = 3000, 100, 1000.0
+    dt = O.COORD_DTYPES[ct]
+    pts = [(rng.random(n) * side).astype(dt) for _ in range(3)]
+    tree = list_shaped(ft, build(ft, ct, pts), rng.permutation(n))
+    x = [a.astype(np.float64) for a in leaves(tree)]
+    q = [(rng.random(nq) * side).astype(dt) for _ in range(3)]
+    want, dist = nearest(squared([a.astype(np.float64) for a in q], x), k)
+    r, d = ft.knn_query(tree, *q, k, max_k=1024)
+    assert np.array_equal(d, dist) and np.array_equal(r, want)
+    ids = rng.permutation(n)[:nq].astype(np.int32)
+    d2 = squared([a[ids] for a in x], x)
+    d2[np.arange(nq), ids] = np.inf
+    want, dist = nearest(d2, k)
+    r, d = ft.self_knn_query_subset(tree, ids, k, max_k=1024, algorithm=ft.ALGO_WAVE)
+    assert np.array_equal(d, dist) and np.array_equal(r, want)
