@@ -39,30 +39,29 @@ struct QueryMap {
     const uint32_t *order;  // slot -> query (null: identity)
     int32_t *list;          // direct passes: slots left to the listed pass, appended;
                             // LISTED: the slots to run
-    uint32_t *count;        // [0] list entries, [1] those that count as exact re-runs,
+    uint32_t *count;        // [0] list entries, [1] queries of the packets left whole,
                             // [2] entries of packets
     int32_t *packets;       // direct passes of cut keys: packets left whole, appended
 };
 
 // Appends the slots of the lanes in `left` (a wave mask), one atomic per wave.
-// `rerun`: they count as exact re-runs (queries the direct pass could not answer
-// exactly, rather than a packet handed over).  Called by whole waves.
-__device__ inline void append_slots(const QueryMap &qm, uint64_t left, int slot, bool rerun) {
+// Called by whole waves.
+__device__ inline void append_slots(const QueryMap &qm, uint64_t left, int slot) {
     if (!left) return;
     const int lane = threadIdx.x & 63;
     uint32_t base = 0;
-    if (lane == 0) {
-        base = atomicAdd(&qm.count[0], (uint32_t)__popcll(left));
-        if (rerun) atomicAdd(&qm.count[1], (uint32_t)__popcll(left));
-    }
+    if (lane == 0) base = atomicAdd(&qm.count[0], (uint32_t)__popcll(left));
     base = (uint32_t)uni((int)base);
     if ((left >> lane) & 1)
         qm.list[base + __builtin_amdgcn_mbcnt_hi((uint32_t)(left >> 32),
                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)left, 0u))] = slot;
 }
 
-__device__ inline void append_packet(const QueryMap &qm, int blk) {
-    if ((threadIdx.x & 63) == 0) qm.packets[atomicAdd(&qm.count[2], 1u)] = blk;
+// Appends packet blk, whose queries are the lanes in `act`.
+__device__ inline void append_packet(const QueryMap &qm, int blk, uint64_t act) {
+    if ((threadIdx.x & 63) != 0) return;
+    qm.packets[atomicAdd(&qm.count[2], 1u)] = blk;
+    atomicAdd(&qm.count[1], (uint32_t)__popcll(act));
 }
 
 __device__ inline int slot_query(const QueryMap &qm, int slot) {
@@ -95,7 +94,7 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_reg_kernel(
     const bool ovf = lane_reg_walk<T, M, GROUPED, STACK_DEPTH, MK>(
         t, active, px, py, pz, self, h, stk, LANE_BLOCK, lane, visits, inserts);
     if (active && !ovf) h.store(k, res, dists, (size_t)q);
-    append_slots(qm, __ballot(active && ovf), slot, true);
+    append_slots(qm, __ballot(active && ovf), slot);
     wave_add_stats(stats, 0, visits);
     wave_add_stats(stats, 4, inserts);
 }
@@ -144,7 +143,7 @@ __global__ __launch_bounds__(LANE_BLOCK) void lane_knn_lds_kernel(
                 }
             }
         }
-        if constexpr (!REF && !LISTED) append_slots(qm, __ballot(left), slot, true);
+        if constexpr (!REF && !LISTED) append_slots(qm, __ballot(left), slot);
         if (!LISTED) break;
     }
     wave_add_stats(stats, 0, visits);
@@ -467,8 +466,10 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             }
         }
         const bool over = c.leaves > a.stop;
-        if (whole && !over) append_packet(qm, blk);
-        else append_slots(qm, over ? act : redo, slot, !over);
+        if (whole && !over) append_packet(qm, blk, act);
+        else append_slots(qm, over ? act : redo, slot);
+        // (its packet has counted the query already)
+        if (LISTED && lane == 0 && redo) atomicSub(&qm.count[1], (uint32_t)__popcll(redo));
     } else {
         H h;
         if constexpr (HEAP) h.key = heap_mem;
@@ -485,7 +486,8 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
                                                             py, pz, r0, &fst, flo, fhi);
                 if constexpr (H::kRankKeys) {
                     if (__popcll(__ballot(active && h.agreeing(k))) >= TIED_LANES) {
-                        append_packet(qm, blk);
+                        append_packet(qm, blk, act);
+                        wave_add_stats(a.stats, 4, c.inserts);
                         return;
                     }
                 }
@@ -504,8 +506,9 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             left |= act & __ballot(h.template store_row<MK>(row, k, res, dists, (size_t)q, k, 0, t,
                                                             px, py, pz));
         else if (row) h.store(k, res, dists, (size_t)q);
-        if (H::kRankKeys && !SEEDED && !over && __popcll(left) >= TIED_LANES) append_packet(qm, blk);
-        else append_slots(qm, left, slot, !over);
+        if (H::kRankKeys && !SEEDED && !over && __popcll(left) >= TIED_LANES)
+            append_packet(qm, blk, act);
+        else append_slots(qm, left, slot);
     }
     if (lane == 0 && a.stats) {
         atomicAdd((unsigned long long *)&a.stats[0], (unsigned long long)c.nodes);
@@ -1185,7 +1188,7 @@ static int rerun_ensure(hipStream_t s, size_t n) {
 __global__ void zero_counts_kernel(uint32_t *count) {
     if (threadIdx.x < 3) count[threadIdx.x] = 0;
 }
-__global__ void add_count_kernel(uint64_t *stats, const uint32_t *count) { stats[3] += count[1]; }
+__global__ void add_count_kernel(uint64_t *stats, const uint32_t *count) { stats[3] += count[0] + count[1]; }
 
 static inline int bit_length(uint64_t v) {
     int b = 0;
@@ -1214,15 +1217,15 @@ static inline int bit_length(uint64_t v) {
 template <typename T, int MK>
 static int launch_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, int nq, int k,
                          int excl, uint64_t cap, const QueryMap &qm, uint64_t *res,
-                         typename CoordTraits<T>::D *d) {
+                         typename CoordTraits<T>::D *d, uint64_t *stats) {
     if (k <= 128) {
         const dim3 g(xcd_grid(std::min<unsigned>(blocks_for(nq, 4), 2048u))), b(256);
         if (k <= 64)
             hipLaunchKernelGGL((wave_knn_kernel<T, 1, MK, true>), g, b, 0, s, dt, qs, nq, k, excl,
-                               cap, qm, res, d, (uint64_t *)nullptr);
+                               cap, qm, res, d, stats);
         else
             hipLaunchKernelGGL((wave_knn_kernel<T, 2, MK, true>), g, b, 0, s, dt, qs, nq, k, excl,
-                               cap, qm, res, d, (uint64_t *)nullptr);
+                               cap, qm, res, d, stats);
     } else {
         size_t lds = 0;
         const int lanes = lds_lanes<T>(k, LANE_STACK_CANON, lds);
@@ -1230,7 +1233,7 @@ static int launch_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         const unsigned g = std::min<unsigned>(blocks_for(nq, lanes), 4096u);
         hipLaunchKernelGGL((lane_knn_lds_kernel<T, false, true, true, MK>), dim3(g),
                            dim3(LANE_BLOCK), lds, s, dt, qs, nq, k, excl, lanes, qm, res, d,
-                           (uint64_t *)nullptr);
+                           stats);
     }
     FT_CHECK_LAUNCH();
     return FT_OK;
@@ -1396,7 +1399,6 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         if (!heap) {
             FT_BY_M(k, (launch_packet_m<T, M, false, MK>(s, dt, qs, a, qm, seed, res, d)));
             if constexpr (std::is_same<T, double>::value) {
-                a.stats = nullptr;
                 a.stop = ~0u;
                 if (k > 1) launch_packets_listed<T, MK>(s, dt, qs, a, qm, res, d);
             }
@@ -1445,7 +1447,8 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
                            (const uint32_t *)rr->count);
         FT_CHECK_LAUNCH();
     }
-    return launch_listed<T, MK>(s, dt, qs, nq, k, excl, cap, qm, res, d);
+    // (the work of a seed's exact re-runs is not counted, only their number)
+    return launch_listed<T, MK>(s, dt, qs, nq, k, excl, cap, qm, res, d, seed ? nullptr : stats);
 }
 
 // The stream's buffers for ordering nq queries.  Every call that may order its
@@ -1769,7 +1772,7 @@ __global__ __launch_bounds__(256) void csr_copy_kernel(const int32_t *__restrict
 __global__ __launch_bounds__(256) void csr_overflow_kernel(const int32_t *__restrict__ counts,
                                                            int nq, QueryMap qm) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    append_slots(qm, __ballot(q < nq && counts[q] > CSR_POOL), q, false);
+    append_slots(qm, __ballot(q < nq && counts[q] > CSR_POOL), q);
 }
 
 int scan_entry(hipStream_t s, const int32_t *counts, int nq, int64_t *row_ptr);

@@ -120,8 +120,9 @@ typedef struct ft_query_opts {
     int32_t mode;        /* FT_MODE_*                                                   */
     int32_t algorithm;   /* FT_ALGO_*                                                   */
     int32_t group_width; /* FT_ALGO_PACKET: queries that share one walk (16, 32 or 64; */
-                         /* 0 = 64), the reference's sub-group width W, one wavefront   */
-                         /* per group; other algorithms walk per lane.  Same results.   */
+                         /* 0 = 64, or 32 where the queries are few), the reference's   */
+                         /* sub-group width W, one wavefront per group; other           */
+                         /* algorithms walk per lane.  Same results.                    */
     int32_t leaf_bucket; /* FT_ALGO_PACKET: subtrees with at most this many leaves are    */
                          /* scanned as one contiguous run of leaf slots (1..64, 0 = auto) */
     int32_t topk;        /* FT_TOPK_*: top-k container of the packet traversal            */
@@ -131,7 +132,8 @@ typedef struct ft_query_opts {
                             /* Canonical mode only.  Results are unchanged by it.       */
     uint64_t *stats;     /* optional device uint64_t[8] counters, accumulated:           */
                          /* [0] nodes visited [1] leaves tested [2] stack overflows     */
-                         /* [3] queries re-run exactly [4] heap insertions              */
+                         /* [3] queries answered by a second pass [4] heap insertions   */
+                         /* (the second pass of seeded queries is counted in [3] only)  */
                          /* packet walks, per wave: [5] insertion rounds [6] rounds     */
                          /* that ran the insertion chain                                */
     int32_t window;      /* FT_ALGO_PACKET self queries: leaves scanned on each side of  */

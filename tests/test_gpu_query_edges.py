@@ -284,3 +284,34 @@ def test_trees_deeper_than_a_walk_s_stack(ft, orc, ct, k):
     want, dist = nearest(d2, k)
     r, d = ft.self_knn_query_subset(tree, ids, k, max_k=1024, algorithm=ft.ALGO_WAVE)
     assert np.array_equal(d, dist) and np.array_equal(r, want)
+
+
+# Every query's neighbours are insertions of some pass, and a query is in [3] when
+# the pass that answered it was the second: packets whose distances tie (whole or a
+# few of their lanes), packets over their leaf limit, passes of 32
+@pytest.mark.parametrize("k", [8, 32, 64])
+@pytest.mark.parametrize("name", ["grid", "half grid", "wide packets", "scattered"])
+def test_counters_cover_the_second_pass(ft, orc, name, k):
+    rng = np.random.default_rng(k)
+    i = np.arange(24_389)
+    pts = [(i // 841).astype(float), (i // 29 % 29).astype(float), (i % 29).astype(float)]
+    if name == "half grid":
+        pts = [a + (i > 12_000) * rng.random(len(i)) * 0.3 for a in pts]
+    if name in ("wide packets", "scattered"):
+        pts = [rng.random(3000) ** 4 for _ in range(3)]
+    tree = build(ft, O.CT_F64, pts)
+    stats = ft.DeviceArray(8, np.uint64).zero()
+    if name in ("wide packets", "scattered"):
+        nq = 160_000
+        q = [np.r_[rng.random(nq // 2) ** 4, rng.random(nq // 2)] for _ in range(3)]
+        ft.knn_query(tree, *q, k, stats=stats,
+                     algorithm=ft.ALGO_AUTO if name == "wide packets" else ft.ALGO_PACKET)
+    else:
+        nq = len(i)
+        ft.self_knn_query(tree, k, max_k=64, algorithm=ft.ALGO_PACKET, stats=stats)
+    st = stats.to_host()
+    print(name, k, st)
+    assert st[4] >= nq * k and st[1] * 64 >= nq * k and st[0] > 0
+    assert st[3] <= nq
+    if name == "grid":
+        assert st[3] > 0.9 * nq
