@@ -39,9 +39,9 @@ struct QueryMap {
     const uint32_t *order;  // slot -> query (null: identity)
     int32_t *list;          // direct passes: slots left to the listed pass, appended;
                             // LISTED: the slots to run
-    uint32_t *count;        // [0] list entries, [1] queries of the packets left whole,
-                            // [2] entries of packets
-    int32_t *packets;       // direct passes of cut keys: packets left whole, appended
+    uint32_t *count;        // [0] list entries, [1] queries of the packets left whole
+                            // (where the caller counts)
+    int32_t *packets;       // direct passes of cut keys: per packet, 1 if left whole
 };
 
 // Appends the slots of the lanes in `left` (a wave mask), one atomic per wave.
@@ -57,11 +57,13 @@ __device__ inline void append_slots(const QueryMap &qm, uint64_t left, int slot)
                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)left, 0u))] = slot;
 }
 
-// Appends packet blk, whose queries are the lanes in `act`.
-__device__ inline void append_packet(const QueryMap &qm, int blk, uint64_t act) {
+// Leaves packet blk, whose queries are the lanes in `act`, to the exact pass.  A
+// flag per packet, not a list: appending 15,600 packets of a lattice took 300 us
+// of atomics on one word, and a list loses the packets' order along the curve.
+__device__ inline void leave_packet(const QueryMap &qm, int blk, uint64_t act, bool counting) {
     if ((threadIdx.x & 63) != 0) return;
-    qm.packets[atomicAdd(&qm.count[2], 1u)] = blk;
-    atomicAdd(&qm.count[1], (uint32_t)__popcll(act));
+    qm.packets[blk] = 1;
+    if (counting) atomicAdd(&qm.count[1], (uint32_t)__popcll(act));
 }
 
 __device__ inline int slot_query(const QueryMap &qm, int slot) {
@@ -361,22 +363,26 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
 // Packed-key packets: at least 4 waves per SIMD (128 VGPRs), 11 % faster than
 // 3 at k = 32.  With the walk's counters in 32 bits the k = 32 kernel spills
 // nothing (72 bytes a lane before: 10M clustered points 16.9 -> 16.7 ms).  The
-// passes of 32 spill (integers 244 bytes, doubles 56) and are faster so than at
-// 3 waves (k = 64 subset of 20M doubles 30.8 against 35.5 ms; of 2M integers
-// 20.5 against 21.4).  Exact pairs of doubles keep their natural 3 waves.
+// passes of 32 spill a little (integers up to 76 bytes, doubles up to 112) and
+// are faster so than at 3 waves (k = 64 subset of 20M doubles 30.8 against 35.5
+// ms).  Exact pairs of doubles run 3 waves (k = 32: 172 registers, two waves,
+// without the bound: a rounded lattice of 1M 4.2 against 3.5 ms).
 //
 // CUT keys (double coordinates, TopKFp): a packet whose queries have many
-// distances that agree above the cut -- regular grids, coincident particles --
-// is left whole to the LISTED instantiation, which takes its packets from
-// qm.packets and keeps exact (d, index) pairs.  It is found out by its fill
-// (equal neighbours among the k curve neighbours of a quarter of the lanes)
-// or at the end (a quarter of the lanes tied).  A lattice of 1M doubles takes
-// 0.95 / 1.56 / 3.36 ms at k = 8 / 16 / 32 this way (0.78 / 1.34 / 3.04 with
-// exact pairs only; 6.3 / 7.4 / 10.2 with a wave for each tied query).
-constexpr int TIED_LANES = 16;
+// distances that agree above the cut -- rounded grids -- is left whole to the
+// LISTED instantiation, which takes the packets flagged in qm.packets and keeps
+// exact (d, index) pairs.  It is found out by its fill (equal neighbours among
+// the k curve neighbours of a quarter of the lanes), by its first run of leaves
+// where there is no fill, or at the end (a quarter of the lanes tied).  Exact
+// pairs for every packet, as before there were packed keys, against now, us:
+// rounded lattice of 1M, self k = 8 / 16 / 32 879 / 1546 / 3475 against 923 /
+// 1514 / 3515; 400k external queries on its points 1258 / 1863 / 3501 against
+// 1468 / 2048 / 3754; 250k of its leaves 741 / 1053 / 2181 against 711 / 1041 /
+// 2217.  Packets whose points are on a coarse enough grid (KeyGrid) need none of
+// it: lattice of 1M, spacing 1, 1035 / 1557 / 3474 against 849 / 1027 / 1723.
 template <typename T, int M, bool HEAP, bool SEEDED, bool PACKED, int MK, bool MULTI = false,
           bool LISTED = false>
-__global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
+__global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_kernel(
     DTree<T> t, QSrc<T> qs, PacketArgs a, QueryMap qm,
     const typename CoordTraits<T>::D *__restrict__ seed, uint64_t *__restrict__ res,
     typename CoordTraits<T>::D *__restrict__ dists) {
@@ -395,12 +401,12 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     const int lane = threadIdx.x;
     const int k = a.k;
     PacketCountersFor<T, MULTI> c;
-    if constexpr (LISTED) {
-        if (blockIdx.x >= qm.count[2]) return;
-    }
-    const int blk = LISTED ? uni(qm.packets[blockIdx.x]) : xcd_block();
+    const int blk = xcd_block();
     const int W = a.width;
     if (blk * W >= a.nq) return;  // padding block of the XCD-ordered grid
+    if constexpr (LISTED) {
+        if (!uni(qm.packets[blk])) return;
+    }
     const int slot = blk * W + lane;
     const bool active = lane < W && slot < a.nq;
     const int q = active ? slot_query(qm, slot) : 0;
@@ -412,6 +418,15 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
     // Which queries are left to the listed pass is kept as masks of the wave, voted
     // outside divergent branches.
     const uint64_t act = __ballot(active);
+    const int tie_min = W / 4;  // tied lanes that make a packet a tied one
+    KeyGrid kg;
+    [[maybe_unused]] bool grid = false;  // every point so far is on kg's grid
+    if constexpr (FPK && H::kRankKeys) {
+        const bool in = px >= t.mnx[0] && px <= t.mxx[0] && py >= t.mny[0] && py <= t.mxy[0] &&
+                        pz >= t.mnz[0] && pz <= t.mxz[0];
+        grid = !t.orig_indices && kg.init(t, a.ibits) &&
+               !__any(active && !(in && kg.on(px, py, pz)));
+    }
     // Window pre-scan.  Self queries over all leaves: the packet is leaf ranks
     // [r0, r0 + 64), so its neighbours along the curve are the leaves on
     // either side.  Subset and external queries (Morton-ordered, so a
@@ -433,6 +448,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
         // nearest (d2, index) above the previous pass's last one, stored in
         // place.
         uint64_t redo = 0;  // lanes left to the listed pass
+        [[maybe_unused]] uint64_t few = 0;  // of them: those whose seed held too few
         bool whole = false;
         typename H::Floor lo = H::no_floor();
         for (int base = 0; base < k; base += M) {
@@ -447,29 +463,38 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
             if constexpr (PACKED) h.init(kk, bound, a.ibits);
             else h.init(kk, bound);
             // one walk instance for every pass (the first with no floor)
-            packet_walk<T, H, MK, true>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo,
-                                        whi, r0, lo, 0, 0, a.stop);
+            const bool ties =
+                packet_walk<T, H, MK, true>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo,
+                                            whi, r0, lo, 0, 0, a.stop, base ? 0 : kk, tie_min, kg,
+                                            grid);
             bool r = false;
-            if constexpr (FPK) r = h.tied() | ((SEEDED || a.full) && h.unfilled());
+            if constexpr (FPK) r = !grid & h.tied();
             else if constexpr (PACKED) r = h.needs_exact(kk);
             else r = (SEEDED || a.full) && h.unfilled();
-            redo |= __ballot(r) & act;
-            const bool row = ((act & ~redo) >> lane) & 1;
+            redo |= (ties ? ~0ull : __ballot(r)) & act;
             if constexpr (FPK)
-                redo |= act & __ballot(h.template store_row<MK>(row, kk, res, dists, (size_t)q, k,
-                                                                base, t, px, py, pz));
-            else if (row) h.store_part(kk, res, dists, (size_t)q, k, base);
+                if (SEEDED || a.full) few |= __ballot(h.unfilled()) & act;
+            const bool row = ((act & ~redo) >> lane) & 1;
+            if constexpr (FPK) {
+                volatile int32_t *bad = stk + lane;  // (the walk's stack is free again)
+                *bad = 0;
+                if (row)
+                    h.template store_row<MK>(kk, res, dists, (size_t)q, k, base, t, px, py, pz, bad);
+                redo |= act & __ballot(*bad != 0);
+            } else if (row) {
+                h.store_part(kk, res, dists, (size_t)q, k, base);
+            }
             lo = h.next_floor();
             if constexpr (H::kRankKeys) {
-                whole = !SEEDED && __popcll(redo) >= TIED_LANES;
+                whole = ties || __popcll(redo) >= tie_min;
                 if (whole) break;
             }
         }
-        const bool over = c.leaves > a.stop;
-        if (whole && !over) append_packet(qm, blk, act);
-        else append_slots(qm, over ? act : redo, slot);
+        const bool over = c.leaves >= a.stop;
+        if (H::kRankKeys && whole && !over) leave_packet(qm, blk, act, a.stats);
+        else append_slots(qm, over ? act : redo | few, slot);
         // (its packet has counted the query already)
-        if (LISTED && lane == 0 && redo) atomicSub(&qm.count[1], (uint32_t)__popcll(redo));
+        if (LISTED && lane == 0 && redo && a.stats) atomicSub(&qm.count[1], (uint32_t)__popcll(redo));
     } else {
         H h;
         if constexpr (HEAP) h.key = heap_mem;
@@ -477,38 +502,48 @@ __global__ __launch_bounds__(64, PACKED ? 4 : 2) void packet_knn_kernel(
         if constexpr (PACKED) h.init(k, bound, a.ibits);
         else h.init(k, bound);
         int flo = 0, fhi = 0;
+        int tie_k = k;  // (0: the fill has looked for ties)
+        bool ties = false;
         if constexpr (H::kSortFill) {
             // self queries over all leaves: lane = leaf rank r0 + lane; the
             // window (>= 32 leaves on each side) covers every filled rank
             if (!qs.qx && !qs.leaf_ids && a.window >= 32) {
                 __shared__ FillStage<T> fst;
                 c.inserts += (uint32_t)fill_from_run<T, MK>(t, h, k, active, self >= 0, rank, px,
-                                                            py, pz, r0, &fst, flo, fhi);
-                if constexpr (H::kRankKeys) {
-                    if (__popcll(__ballot(active && h.agreeing(k))) >= TIED_LANES) {
-                        append_packet(qm, blk, act);
-                        wave_add_stats(a.stats, 4, c.inserts);
-                        return;
-                    }
-                }
+                                                            py, pz, r0, &fst, flo, fhi, kg, grid);
+                tie_k = 0;
+                if constexpr (H::kRankKeys)
+                    ties = !grid && __popcll(__ballot(h.agreeing(k)) & act) >= tie_min;
             }
         }
-        packet_walk<T, H, MK>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo, whi, r0,
-                              H::no_floor(), flo, fhi, a.stop);
-        const bool over = c.leaves > a.stop;
+        // (a packet tied by its fill still enters the walk, which ends at the root: a
+        // way out here, with its store before the walk's loads, made those vector
+        // loads, 5 % of k = 16 of 2M points)
+        ties |= packet_walk<T, H, MK>(t, a.bucket, active, px, py, pz, self, h, stk, c,
+                                      ties ? 0 : wlo, ties ? 0 : whi, r0, H::no_floor(), flo, fhi,
+                                      ties ? 0u : a.stop, tie_k, tie_min, kg, grid);
+        const bool over = c.leaves >= a.stop;
         bool r = false;
-        if constexpr (FPK) r = h.tied() | (SEEDED && h.unfilled());
+        if constexpr (FPK) r = !grid & h.tied();
         else if constexpr (PACKED) r = h.needs_exact(k);
         else if constexpr (SEEDED) r = h.unfilled();
-        uint64_t left = over ? act : __ballot(r) & act;
+        uint64_t left = (over || ties ? ~0ull : __ballot(r)) & act;
         const bool row = ((act & ~left) >> lane) & 1;
-        if constexpr (FPK)
-            left |= act & __ballot(h.template store_row<MK>(row, k, res, dists, (size_t)q, k, 0, t,
-                                                            px, py, pz));
-        else if (row) h.store(k, res, dists, (size_t)q);
-        if (H::kRankKeys && !SEEDED && !over && __popcll(left) >= TIED_LANES)
-            append_packet(qm, blk, act);
-        else append_slots(qm, left, slot);
+        if constexpr (FPK) {
+            volatile int32_t *bad = stk + lane;  // (the walk's stack is free)
+            *bad = 0;
+            if (row) h.template store_row<MK>(k, res, dists, (size_t)q, k, 0, t, px, py, pz, bad);
+            left |= act & __ballot(*bad != 0);
+        } else if (row) {
+            h.store(k, res, dists, (size_t)q);
+        }
+        if (H::kRankKeys && !over && (ties || __popcll(left) >= tie_min)) {
+            leave_packet(qm, blk, act, a.stats);
+        } else {
+            // (seeds that were too small do not make a packet a tied one)
+            if constexpr (FPK && SEEDED) left |= __ballot(h.unfilled()) & act;
+            append_slots(qm, left, slot);
+        }
     }
     if (lane == 0 && a.stats) {
         atomicAdd((unsigned long long *)&a.stats[0], (unsigned long long)c.nodes);
@@ -1184,9 +1219,11 @@ static int rerun_ensure(hipStream_t s, size_t n) {
     return FT_OK;
 }
 
-// Starts a direct pass's list (QueryMap::count).
-__global__ void zero_counts_kernel(uint32_t *count) {
-    if (threadIdx.x < 3) count[threadIdx.x] = 0;
+// Starts a direct pass's list (QueryMap::count) and clears its packets' flags.
+__global__ __launch_bounds__(256) void zero_counts_kernel(uint32_t *count, int32_t *packets, int np) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < 2) count[i] = 0;
+    if (i < np) packets[i] = 0;
 }
 __global__ void add_count_kernel(uint64_t *stats, const uint32_t *count) { stats[3] += count[0] + count[1]; }
 
@@ -1267,7 +1304,7 @@ template <typename T, int MK>
 static void launch_packets_listed(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs,
                                   const PacketArgs &a, const QueryMap &qm, uint64_t *res,
                                   typename CoordTraits<T>::D *d) {
-    const dim3 g(blocks_for(a.nq, a.width));
+    const dim3 g(xcd_grid(blocks_for(a.nq, a.width)));
 #define FT_LISTED(M_, MULTI_)                                                                     \
     hipLaunchKernelGGL((packet_knn_kernel<T, M_, false, false, false, MK, MULTI_, true>), g,      \
                        dim3(64), 0, s, dt, qs, a, qm, (const double *)nullptr, res, d)
@@ -1372,7 +1409,10 @@ static int run_canonical(hipStream_t s, const DTree<T> &dt, const QSrc<T> &qs, i
         rr = &stream_bufs(s).rr;
     }
     if (leaves_slots) {
-        hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, s, rr->count);
+        const bool flags = algo == FT_ALGO_PACKET && std::is_same<T, double>::value;
+        const int np = flags ? (int)blocks_for(nq, width) : 0;
+        hipLaunchKernelGGL(zero_counts_kernel, dim3(blocks_for(std::max(np, 2), 256)), dim3(256), 0,
+                           s, rr->count, rr->packets, np);
     }
     const QueryMap qm{order, leaves_slots ? rr->list : nullptr, leaves_slots ? rr->count : nullptr,
                       leaves_slots ? rr->packets : nullptr};
@@ -1821,7 +1861,8 @@ static int range_csr_t(hipStream_t s, const ft_tree &tree, const RangeSrc<T> &sr
             const RerunBuf &rr = stream_bufs(s).rr;
             const QueryMap qm{nullptr, rr.list, rr.count, nullptr};
             const DTree<T> dt = make_dtree<T>(tree);
-            hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(64), 0, s, rr.count);
+            hipLaunchKernelGGL(zero_counts_kernel, dim3(1), dim3(256), 0, s, rr.count,
+                               (int32_t *)nullptr, 0);
             hipLaunchKernelGGL(csr_overflow_kernel, dim3(blocks_for(nq, 256)), dim3(256), 0, s,
                                (const int32_t *)counts, nq, qm);
             const dim3 g(xcd_grid(std::min<unsigned>(blocks_for(nq, 4), 2048u))), b(256);

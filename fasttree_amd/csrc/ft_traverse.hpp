@@ -761,10 +761,13 @@ template <int M> struct TopKPacked : KeySlots<M> {
 //    distance is at most the k-th is offered to the list.  The result is exact
 //    unless two distances agree above the cut: `rejected` keeps the smallest
 //    key that a full list turned away or dropped, and the row, recomputed from
-//    the ranks in double precision, must come out in order.  A query that
-//    fails either test is answered again, exactly.  Near ties are rare where
+//    the ranks in double precision, must come out in order.  (Keys whose distances
+//    have no bit below the cut are in order, since equal distances are ordered by
+//    rank: `rejected` does not count where every point is on a coarse enough grid,
+//    KeyGrid.)  A query that fails either test is answered again, exactly.  Near
+//    ties are rare where
 //    distances are continuous (at 20M points the cut keeps 25 bits of the
-//    mantissa: about one query in 100,000); where they are common, on a regular
+//    mantissa: about one query in 100,000); where they are common, on a rounded
 //    grid, the packet kernel hands whole packets to its exact instantiation.
 // ---------------------------------------------------------------------------
 template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>::value> {
@@ -810,8 +813,8 @@ template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>:
     // dropped sentinel is no distance, and lies above every key of its bound).
     __device__ inline bool tied() const {
         if constexpr (kCut)
-            return ((rejected ^ key[M - 1]) & ~imask) == 0 && !B::empty(M - 1) &&
-                   (rejected & imask) != imask;
+            return (((rejected ^ key[M - 1]) & ~imask) == 0) & !B::empty(M - 1) &
+                   ((rejected & imask) != imask);
         else return false;
     }
     // Two neighbouring live slots agree above the cut.
@@ -822,12 +825,14 @@ template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>:
             any |= (s > M - k) & (((key[s] ^ key[s - 1]) & ~imask) == 0) & !B::empty(s);
         return any;
     }
-    // Entries [base, base + k) of row q (row length k_row), written by the lanes
-    // with `row`; double coordinates recompute them.  Every lane of the wave calls
-    // it and is told whether its entries are out of (d, index) order.
+    // Entries [base, base + k) of row q (row length k_row); double coordinates
+    // recompute them.  Sets *out_of_order if they are not in (d, index) order: a
+    // word in LDS and volatile, since the lanes that call it are in a divergent
+    // branch, out of which a flag would not come (TRAVERSAL_FLAGS in build.py).
     template <int MK, typename Tr>
-    __device__ inline bool store_row(bool row, int k, uint64_t *res, double *dists, size_t q,
-                                     int k_row, int base, const Tr &t, T px, T py, T pz) const {
+    __device__ inline void store_row(int k, uint64_t *res, double *dists, size_t q, int k_row,
+                                     int base, const Tr &t, T px, T py, T pz,
+                                     volatile int32_t *out_of_order) const {
         const size_t o = q * (size_t)k_row + (size_t)base;
         const int off = t.n - 1;
         bool bad = false;
@@ -850,13 +855,33 @@ template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>:
                 } else {
                     d = d_hi(key[s]);
                 }
-                if (row) {
-                    res[j] = ok ? (uint64_t)(uint32_t)i : ~0ull;
-                    dists[j] = ok ? d : missing_dist<double>();
-                }
+                res[j] = ok ? (uint64_t)(uint32_t)i : ~0ull;
+                dists[j] = ok ? d : missing_dist<double>();
             }
         }
-        return bad;
+        if constexpr (kCut) *out_of_order = bad ? 1 : 0;
+    }
+};
+
+// A grid of spacing 2^-p on which every squared distance inside the root box fits
+// the bits that cut keys keep.  Differences are multiples k 2^-p with k 2^-p <= R <
+// 2^r, R the largest side of the root box (queries outside it are off the grid), so
+// d2 is a multiple of 2^-2p below 2^(2r + 2) and has at most 2 (p + r) + 2 of the
+// 51 - ib significant bits of a key.  Grid and coarsely rounded points meet it;
+// others fail at the packet's queries, before any leaf is looked at.
+struct KeyGrid {
+    double scale = 0.0;  // 2^p
+    template <typename T> __device__ inline bool init(const DTree<T> &t, int ibits) {
+        const double R = fmax(t.mxx[0] - t.mnx[0], fmax(t.mxy[0] - t.mny[0], t.mxz[0] - t.mnz[0]));
+        const int r = (int)((__double2hiint(R) >> 20) & 0x7FF) - 1022;
+        const int p = (49 - ibits) / 2 - r;
+        if (!(R < 0x1p100) || p > 100 || p < -100) return false;
+        scale = __hiloint2double((1023 + p) << 20, 0);
+        return !t.m.periodic || whole(t.m.box);
+    }
+    __device__ inline bool whole(double v) const { return rint(v * scale) == v * scale; }
+    __device__ inline bool on(double x, double y, double z) const {
+        return whole(x) & whole(y) & whole(z);
     }
 };
 
@@ -875,9 +900,13 @@ template <typename T, int M> struct TopKFp : KeySlots<M, std::is_same<T, float>:
 // from the lane's results (-1: none); inactive lanes take no candidates.
 // [fill_lo, fill_hi): leaf ranks the caller already put into this lane's h
 // (fill_from_run); the window pre-scan skips them.
-// stop: the walk ends, with h unfinished, once c.leaves exceeds it (the lanes'
+// stop: the walk ends, with h unfinished, once c.leaves reaches it (the lanes'
 // regions have too little in common); not in the integers' multi-pass walks,
 // whose registers it would spill.
+// tie_k: lists of cut keys with that many entries are looked over after the first
+// run of the window pre-scan; where at least tie_min lanes hold distances that
+// agree, the walk ends there and returns true.
+// grid: cut keys; cleared by the first scanned leaf that is off kg's grid.
 // ===========================================================================
 constexpr int PK_STACK = 128;
 
@@ -894,13 +923,12 @@ using PacketCountersFor =
     PacketCounters<typename std::conditional<MULTI && !CoordTraits<T>::fp, uint64_t, uint32_t>::type>;
 
 template <typename T, typename H, int MK, bool FLOOR = false, typename C>
-__device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
+__device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
                                             T pz, int self, H &h, int32_t *stk,
-                                            PacketCounters<C> &c, int win_lo = 0, int win_hi = 0,
-                                            int win_mid = 0,
-                                            typename H::Floor lo = H::no_floor(),
-                                            int fill_lo = 0, int fill_hi = 0,
-                                            uint32_t stop = ~0u) {
+                                            PacketCounters<C> &c, int win_lo, int win_hi,
+                                            int win_mid, typename H::Floor lo, int fill_lo,
+                                            int fill_hi, uint32_t stop, int tie_k, int tie_min,
+                                            const KeyGrid &kg, bool &grid) {
     using D = typename CoordTraits<T>::D;
     const int lane = threadIdx.x & 63;
     const int n = t.n;
@@ -948,7 +976,12 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
     // not wrapped, and one beyond half a period is outside either way.  (k = 32
     // of 10M periodic integers 16.65 -> 15.75 ms against wrapped differences,
     // subset k = 64 of 20M doubles 31.9 -> 30.8, whose error bound now follows
-    // the packet's extent; packets over the limits keep the older form.)
+    // the packet's extent.)  Over the limits, as while a list is not full, periodic
+    // integers take wrapped differences, doubles the exact test.  (Doubles over the
+    // limits throughout, k = 32, 300k queries of 100 / 300 / 5,000 periodic points:
+    // 422 / 393 / 642 us, 432 / 557 / 984 with wrapped differences of the floats.
+    // Both forms in one kernel cost it a wave per SIMD: self k = 16 of 2M 2.58 ->
+    // 2.85 ms.)
     constexpr bool IPF = !CoordTraits<T>::fp && MK == MK_OPEN;
     constexpr bool REL = PRE || IPF || F64;
     // (the passes of periodic integers have no registers for it: 20.6 -> 21.4 ms)
@@ -1037,6 +1070,9 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
             s_x[lane] = bx;
             s_y[lane] = by;
             s_z[lane] = bz;
+        }
+        if constexpr (H::kRankKeys) {
+            if (grid) grid = !__any(lane < cnt && !kg.on(bx, by, bz));
         }
         // Bit j: the filter passes leaf j, shifted in from the top, leaves taken
         // last to first; unrolled so that several broadcast reads are in flight
@@ -1207,10 +1243,21 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
     // and keeps the insertions that a tighter bound would reject few; the walk
     // then skips these leaves.
     const bool window = win_hi > win_lo;
+    bool ties = false;
     if (window) {
         const int own_hi = win_mid + 64 < win_hi ? win_mid + 64 : win_hi;
         scan_range(win_mid, own_hi - win_mid, false);
         int le = win_mid, rs = own_hi;
+        if constexpr (H::kRankKeys) {
+            // (the walk ends as over the limit; a return here spilled 300 registers)
+            if (tie_k > 0 && !grid)
+                ties = __popcll(__ballot(active && h.agreeing(tie_k))) >= tie_min;
+            if (ties) {
+                stop = 0;
+                le = win_lo;
+                rs = win_hi;
+            }
+        }
         while (le > win_lo || rs < win_hi) {
             if (le > win_lo) {
                 const int lb = le - 64 > win_lo ? le - 64 : win_lo;
@@ -1276,7 +1323,7 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
         // Over the limit: the walk ends as if nothing were left.  (A branch out
         // of the loop here made the allocator keep two copies of the list.)
         if constexpr (!FLOOR || CoordTraits<T>::fp) {
-            if (c.leaves > stop) {
+            if (c.leaves >= stop) {
                 sp = 0;
                 next = -1;
             }
@@ -1288,6 +1335,20 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
         if (next < 0) break;
         node = next;
     }
+    return ties;
+}
+
+// The walk of lists without cut keys.
+template <typename T, typename H, int MK, bool FLOOR = false, typename C>
+__device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
+                                            T pz, int self, H &h, int32_t *stk,
+                                            PacketCounters<C> &c, int win_lo, int win_hi,
+                                            int win_mid,
+                                            typename H::Floor lo = H::no_floor()) {
+    static_assert(!H::kRankKeys, "cut keys need the tie arguments");
+    bool grid = false;
+    packet_walk<T, H, MK, FLOOR>(t, bucket, active, px, py, pz, self, h, stk, c, win_lo, win_hi,
+                                 win_mid, lo, 0, 0, ~0u, 0, 0, KeyGrid{}, grid);
 }
 
 // ---------------------------------------------------------------------------
@@ -1298,7 +1359,7 @@ __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool 
 // insertion rounds, and a tight bound before the window pre-scan.  Leaves
 // [r0 - 32, r0 + 96) are staged in LDS (st: 128 entries) so each lane reads
 // its candidates without shuffles.  Returns this lane's filled rank range
-// [flo, fhi) for the window pre-scan to skip.  k <= 32.
+// [flo, fhi) for the window pre-scan to skip.  k <= 32.  grid: as in packet_walk.
 // ---------------------------------------------------------------------------
 template <typename T> struct FillStage {
     T x[128], y[128], z[128];
@@ -1308,7 +1369,8 @@ template <typename T> struct FillStage {
 template <typename T, int MK, typename H>
 __device__ __forceinline__ int fill_from_run(const DTree<T> &t, H &h, int k, bool active,
                                              bool excl, int rank, T px, T py, T pz, int r0,
-                                             FillStage<T> *st, int &flo, int &fhi) {
+                                             FillStage<T> *st, int &flo, int &fhi,
+                                             const KeyGrid &kg, bool &grid) {
     const int lane = threadIdx.x & 63;
     const int n = t.n, off = n - 1;
     const int base = r0 - 32;
@@ -1320,6 +1382,9 @@ __device__ __forceinline__ int fill_from_run(const DTree<T> &t, H &h, int k, boo
             st->y[e] = t.mny[off + j];
             st->z[e] = t.mnz[off + j];
             st->idx[e] = H::kRankKeys ? j : ret_index(t, off + j);
+        }
+        if constexpr (H::kRankKeys) {
+            if (grid) grid = !__any(j >= 0 && j < n && !kg.on(st->x[e], st->y[e], st->z[e]));
         }
     }
     __syncthreads();  // the block is this one wave

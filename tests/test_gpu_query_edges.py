@@ -290,11 +290,13 @@ def test_trees_deeper_than_a_walk_s_stack(ft, orc, ct, k):
 # the pass that answered it was the second: packets whose distances tie (whole or a
 # few of their lanes), packets over their leaf limit, passes of 32
 @pytest.mark.parametrize("k", [8, 32, 64])
-@pytest.mark.parametrize("name", ["grid", "half grid", "wide packets", "scattered"])
+@pytest.mark.parametrize("name", ["grid", "rounded grid", "half grid", "wide packets", "scattered"])
 def test_counters_cover_the_second_pass(ft, orc, name, k):
     rng = np.random.default_rng(k)
     i = np.arange(24_389)
     pts = [(i // 841).astype(float), (i // 29 % 29).astype(float), (i % 29).astype(float)]
+    if name != "grid":  # distances that agree but for their last bits
+        pts = [a * 0.1 + 0.05 for a in pts]
     if name == "half grid":
         pts = [a + (i > 12_000) * rng.random(len(i)) * 0.3 for a in pts]
     if name in ("wide packets", "scattered"):
@@ -313,5 +315,55 @@ def test_counters_cover_the_second_pass(ft, orc, name, k):
     print(name, k, st)
     assert st[4] >= nq * k and st[1] * 64 >= nq * k and st[0] > 0
     assert st[3] <= nq
-    if name == "grid":
+    if name == "rounded grid":
         assert st[3] > 0.9 * nq
+
+
+def gridded(name, n, seed):
+    """Doubles whose distances tie: on a grid that cut keys hold exactly, on one too
+    fine for them, on a rounded one, and the first with single points off it."""
+    rng = np.random.default_rng(seed)
+    pts = [rng.integers(0, 16, n) / 16.0 for _ in range(3)]
+    if name == "far from the origin":
+        return [a + 2.0**30 for a in pts]
+    if name == "too fine":  # distances differ far below the cut
+        return [a + rng.integers(0, 2, n) * 2.0**-44 for a in pts]
+    if name == "rounded":
+        return [(a + 1 / 32) / 0.9999123 for a in pts]
+    if name == "single points off":
+        off = rng.choice(n, 5, replace=False)
+        for a in pts:
+            a[off] += 2.0**-44
+    return pts
+
+
+# Packets of 16, 32 and 64 (a quarter of their lanes makes them tied ones); with a
+# fill, with none, in passes; equal distances ordered by rank and by original index
+@pytest.mark.parametrize("width", [16, 32, 64])
+@pytest.mark.parametrize("k", [3, 8, 20, 32, 40])
+@pytest.mark.parametrize("name", ["exact", "far from the origin", "too fine", "rounded",
+                                  "single points off"])
+def test_tied_doubles_on_grids(ft, orc, name, k, width):
+    n = 3000
+    pts = gridded(name, n, k)
+    rng = np.random.default_rng(k)
+    ids = rng.permutation(n)[:1000].astype(np.int32)
+    far = [np.r_[a[ids], a[ids[:300]] + 1 / 64] for a in pts]  # between the points too
+    for periodic, orig, box in ((0, False, 0.0), (1, False, 2.0), (1, False, 1.0000001), (0, True, 0.0)):
+        if periodic and name == "far from the origin":
+            continue  # (a periodic box holds its points)
+        if periodic and box < 1.01 and name == "rounded":
+            box = 1.1
+        tree = build(ft, O.CT_F64, pts, periodic, box, orig=orig)
+        t = O.build_bvh(O.CT_F64, *pts, sfc=O.SFC_PH, bits=21, periodic=periodic, box=box,
+                        orig_indices=int(orig))
+        o = dict(algorithm=ft.ALGO_PACKET, group_width=width)
+        rb, db = O.knn_bruteforce(t, k, True)
+        r, d = ft.self_knn_query(tree, k, max_k=64, **o)
+        assert np.array_equal(d, db) and np.array_equal(r, rb)
+        r, d = ft.self_knn_query_subset(tree, ids, k, **o)
+        assert np.array_equal(d, db[ids]) and np.array_equal(r, rb[ids])
+        q = [np.mod(a, box) for a in far] if periodic else far
+        rb, db = O.knn_bruteforce(t, k, queries=q)
+        r, d = ft.knn_query(tree, *q, k, **o)
+        assert np.array_equal(d, db) and np.array_equal(r, rb)
