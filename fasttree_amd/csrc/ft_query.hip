@@ -684,8 +684,7 @@ __global__ __launch_bounds__(64) void range_packet_kernel(DTree<T> t, RangeSrc<T
         }
         RM2f = wrap_filter_bound_pre((uint64_t)RM2, wsh);
     }
-    // Leaf filter: pairs at a float distance below f_in are inside r_max, above
-    // f_out outside it; below g_out nearer than r_min, above g_in not.
+    // Leaf filter (RangeFilter).
     [[maybe_unused]] T cx = T(0), cy = T(0), cz = T(0);
     [[maybe_unused]] float fx = 0.f, fy = 0.f, fz = 0.f;
     [[maybe_unused]] float f_in = 0.f, f_out = 0.f, g_in = -1.f, g_out = -1.f;
@@ -705,23 +704,11 @@ __global__ __launch_bounds__(64) void range_packet_kernel(DTree<T> t, RangeSrc<T
         }
         const float ext = wave_max_f32(fmaxf(fabsf(fx), fmaxf(fabsf(fy), fabsf(fz))));
         const float rad = wave_max_f32((float)sqrt((double)RM2) * (1.0f + 0x1p-20f));
-        double E = 2.02 * 0x1p-24 * (double)ext;
-        if constexpr (CoordTraits<T>::fp) {
-            const double mq = fmax(fabs((double)cx), fmax(fabs((double)cy), fabs((double)cz)));
-            E += 0x1p-50 * (mq + (double)ext + (MK == MK_WRAP ? t.m.box : 0.0));
-        }
+        const double E = rel_err<T, MK>(t.m, ext, cx, cy, cz);
         const float period = CoordTraits<T>::fp ? (float)t.m.box : (float)(1ull << t.m.bits);
-        filter = (MK == MK_WRAP ? ext + rad < 0.249f * period : true) && rad < 1.0e18f &&
-                 ext < 1.0e18f && t.m.dshift == 0;
-        // (below 1e-30 the floats' own underflow would count: left to the exact test)
-        auto sure = [](float v) { return v < 1.0e-30f ? 0.f : v; };
-        f_out = fmaxf(fpf_upper((double)RM2, E), 1.0e-30f);
-        f_in = sure(fpf_lower((double)RM2, E));
-        if (!(rm2 <= D(0))) {
-            g_in = fmaxf(fpf_upper((double)rm2, E), 1.0e-30f);
-            g_out = sure(fpf_lower((double)rm2, E));
-        }
-        if (RM2 != RM2 || rm2 != rm2) f_in = f_out = -1.f;  // a NaN radius has no hits
+        filter = (MK == MK_WRAP ? ext + rad < 0.249f * period : true) && rad < 1.0e18f && ext < 1.0e18f;
+        const RangeFilter rf = range_filter<D>(rm2, RM2, E);
+        f_in = rf.f_in; f_out = rf.f_out; g_in = rf.g_in; g_out = rf.g_out;
     }
     const bool inner = __any(!(rm2 <= D(0)));
     auto node_near = [&](int nd) -> bool {

@@ -143,15 +143,15 @@ __host__ __device__ __forceinline__ float wrap_filter_bound_pre(uint64_t w, int 
 __host__ __device__ __forceinline__ float wrap_filter_floor_pre(uint64_t lo, int sh) {
     return (float)lo * (1.0f - 0x1p-20f) * (float)(1ull << (2 * sh));
 }
-// Float32 pre-filter for double coordinates (and for integers in an open box,
-// whose conversion to float is as exact).  With u = 2^-24, coordinates of
+// Float32 distances of double coordinates.  With u = 2^-24, coordinates of
 // magnitude at most M and period L, the float gap of one axis (both points
 // rounded to float, one subtraction, for a periodic metric min(g, fl(L) - g))
 // is within (1 + u) g + E of the double gap g, E = 1.01 u (L + 4M) (periodic)
 // or 2.02 u M (open); the float sum of the three squares (a product, two
 // fmas) is within a factor 1 + 3.01u.  So a leaf with d2 <= w has a float
 // squared distance at most fpf_upper(w, E), and one with d2 >= lo at least
-// fpf_lower(lo, E): the filter never rejects a leaf the exact test accepts.
+// fpf_lower(lo, E).  (The kernels take coordinates relative to a query, whose E is
+// rel_err; fpf_gap and fpf_err are the form for coordinates as they are.)
 __host__ __device__ __forceinline__ float fpf_gap(float q, float x, float L, bool wrap) {
     const float g = fabsf(q - x);
     return wrap ? fminf(g, L - g) : g;
@@ -217,6 +217,15 @@ __device__ __forceinline__ int centre_lane(bool active, T x, T y, T z, int from)
 // above that of any leaf with d2 >= lo: all in float, with the rounding of the
 // conversion, the root (2 ulp) and the products covered; below 1e-30 the
 // floats' underflow is left out of it.
+template <typename T, int MK>
+__host__ __device__ __forceinline__ double rel_err(const Metric &m, float ext, T cx, T cy, T cz) {
+    double E = 2.02 * 0x1p-24 * (double)ext;
+    if constexpr (CoordTraits<T>::fp) {
+        const double mc = fmax(fabs((double)cx), fmax(fabs((double)cy), fabs((double)cz)));
+        E += 0x1p-50 * (mc + (double)ext + (MK == MK_WRAP ? m.box : 0.0));
+    }
+    return E;
+}
 __host__ __device__ __forceinline__ float rel_upper(float w, float E) {
     w = w < 1.0e-30f ? 1.0e-30f : w;
     const float b = __builtin_sqrtf(w * (1.0f + 0x1p-22f)) * (1.0f + 0x1p-21f) + 1.75f * E;
@@ -225,6 +234,25 @@ __host__ __device__ __forceinline__ float rel_upper(float w, float E) {
 __host__ __device__ __forceinline__ float rel_lower(float lo, float E) {
     const float b = __builtin_sqrtf(lo * (1.0f - 0x1p-22f)) * (1.0f - 0x1p-21f) - 1.75f * E;
     return lo < 1.0e-30f || !(b > 0.0f) ? 0.0f : b * b * (1.0f - 0x1p-20f);
+}
+
+// Range filter: of pairs at float distance d, those below f_in are inside r_max,
+// those above f_out outside it, those below g_out nearer than r_min and those above
+// g_in not; the rest take the exact test.  hi, lo: the squared radii.  Below 1e-30
+// the floats' own underflow would count: left to the exact test.
+struct RangeFilter {
+    float f_in, f_out, g_in, g_out;
+};
+template <typename D>
+__host__ __device__ __forceinline__ RangeFilter range_filter(D lo, D hi, double E) {
+    auto sure = [](float v) { return v < 1.0e-30f ? 0.f : v; };
+    RangeFilter r{sure(fpf_lower((double)hi, E)), fmaxf(fpf_upper((double)hi, E), 1.0e-30f), -1.f, -1.f};
+    if (!(lo <= D(0))) {
+        r.g_in = fmaxf(fpf_upper((double)lo, E), 1.0e-30f);
+        r.g_out = sure(fpf_lower((double)lo, E));
+    }
+    if (hi != hi || lo != lo) r.f_in = r.f_out = -1.f;  // a NaN radius has no hits
+    return r;
 }
 
 // Float32 squared distance of a leaf, pre-shifted coordinates (scaled by
@@ -988,8 +1016,6 @@ __device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool 
     constexpr bool REL_OK = !(PRE && FLOOR);
     // largest squared bound the filter may be used with (negative: never)
     [[maybe_unused]] float rel_w = -1.f, relE = 0.f;
-    // an integer gap is shifted down by dshift: the filter works in those units
-    [[maybe_unused]] const float fs = IPF ? 1.0f / (float)(1ull << t.m.dshift) : 1.0f;
     [[maybe_unused]] int cl = 0;
     if constexpr (REL) {
         cl = centre_lane<T>(active, px, py, pz, 0);
@@ -1001,19 +1027,13 @@ __device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool 
                               fabsf(rel_coord<T, MK>(t.m, pz, cz))));
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) ext = fmaxf(ext, __shfl_xor(ext, o, 64));
-        ext = rl(ext, 0) * fs;
-        relE = 2.02f * 0x1p-24f * ext;
-        if constexpr (F64) {
-            const double mc = fmax(fabs(cx), fmax(fabs(cy), fabs(cz)));
-            relE += (float)(0x1p-50 * (mc + (double)ext + (MK == MK_WRAP ? t.m.box : 0.0)));
-        }
-        if (IPF && t.m.dshift) relE += 1.0f;  // what the shift drops
+        ext = rl(ext, 0);
+        relE = (float)rel_err<T, MK>(t.m, ext, cx, cy, cz);
         if constexpr (MK == MK_WRAP) {
+            // (integers have at most 21 bits: exact in float)
             const float period = PRE ? (float)(1ull << t.m.bits) : (float)t.m.box;
             const float room = 0.249f * period - ext;
-            // integers up to 22 bits are exact in float (relE covers the rest
-            // only in rel_upper, which they do not use)
-            if (room > 0.f && (!PRE || t.m.bits <= 22)) rel_w = room * room;
+            if (room > 0.f) rel_w = room * room;
         } else if (ext < 1.0e18f) {
             rel_w = __builtin_huge_valf();
         }
@@ -1098,15 +1118,14 @@ __device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool 
                     s_leaf[lane] = make_uint4(__float_as_uint(rel(ex, c0x)), __float_as_uint(rel(ey, c0y)),
                                               __float_as_uint(rel(ez, c0z)), 0u);
                     up = wf;
-                    if constexpr (FLOOR) low = (float)(uint64_t)lo_d * (1.0f - 0x1p-20f);
                 } else {
                     const T cx = rl(px, cl), cy = rl(py, cl), cz = rl(pz, cl);
-                    fx = rel_coord<T, MK>(t.m, px, cx) * fs;
-                    fy = rel_coord<T, MK>(t.m, py, cy) * fs;
-                    fz = rel_coord<T, MK>(t.m, pz, cz) * fs;
-                    s_leaf[lane] = make_uint4(__float_as_uint(rel_coord<T, MK>(t.m, bx, cx) * fs),
-                                              __float_as_uint(rel_coord<T, MK>(t.m, by, cy) * fs),
-                                              __float_as_uint(rel_coord<T, MK>(t.m, bz, cz) * fs), 0u);
+                    fx = rel_coord<T, MK>(t.m, px, cx);
+                    fy = rel_coord<T, MK>(t.m, py, cy);
+                    fz = rel_coord<T, MK>(t.m, pz, cz);
+                    s_leaf[lane] = make_uint4(__float_as_uint(rel_coord<T, MK>(t.m, bx, cx)),
+                                              __float_as_uint(rel_coord<T, MK>(t.m, by, cy)),
+                                              __float_as_uint(rel_coord<T, MK>(t.m, bz, cz)), 0u);
                     up = rel_upper(wf, relE);
                     if constexpr (FLOOR) low = rel_lower((float)lo_d, relE);
                 }
