@@ -2060,9 +2060,28 @@ __device__ __forceinline__ void wave_walk(const DTree<T> &t, T px, T py, T pz, i
         if (!found) break;
     }
     if (full) {
+        // (one at a time: the sort and merge once more here cost the k = 128 walk 2 %)
         L.clear(cap);
         nbuf = 0;
-        for (int r0 = 0; r0 < n; r0 += 64) scan(r0, n - r0 < 64 ? n - r0 : 64, false);
+        for (int r0 = 0; r0 < n; r0 += 64) {
+            const int r = r0 + lane;
+            const int leaf = off + (r < n ? r : r0);
+            const uint64_t cd = dist_bits(
+                leaf_d2_k<T, MK>(t.m, px, py, pz, t.mnx[leaf], t.mny[leaf], t.mnz[leaf]));
+            const uint32_t ci = (uint32_t)ret_index(t, leaf);
+            uint64_t m = __ballot(r < n && r != self && L.admits(cd, ci));
+            while (m) {
+                const int j = __builtin_ctzll(m);
+                m &= m - 1;
+                const uint64_t xd = rl(cd, j);
+                const uint32_t xi = rl32(ci, j);
+                if (L.admits(xd, xi)) {
+                    L.insert_one(xd, xi);
+                    L.refresh();
+                }
+            }
+        }
+        c.leaves += (uint64_t)n;
     }
     flush();
 }
