@@ -421,7 +421,8 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
     const int tie_min = W / 4;  // tied lanes that make a packet a tied one
     KeyGrid kg;
     [[maybe_unused]] bool grid = false;  // every point so far is on kg's grid
-    if constexpr (FPK && H::kRankKeys) {
+    // (not in passes, whose registers it would spill: k = 64 of 20M doubles 2 %)
+    if constexpr (FPK && H::kRankKeys && !MULTI) {
         const bool in = px >= t.mnx[0] && px <= t.mxx[0] && py >= t.mny[0] && py <= t.mxy[0] &&
                         pz >= t.mnz[0] && pz <= t.mxz[0];
         grid = !t.orig_indices && kg.init(t, a.ibits) &&
