@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64) void batch_packet_kernel(BatchView<T> b,
         heap_mem = heap;
     }
     const int lane = threadIdx.x;
-    PacketCountersFor<T, MULTI> c;
+    PacketCounters c;
     while (true) {
         const int it = grab_item(ctr, bnd);
         if (it < 0) break;

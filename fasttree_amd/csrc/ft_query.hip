@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
 // Packed-key packets: at least 4 waves per SIMD (128 VGPRs), 11 % faster than
 // 3 at k = 32.  With the walk's counters in 32 bits the k = 32 kernel spills
 // nothing (72 bytes a lane before: 10M clustered points 16.9 -> 16.7 ms).  The
-// passes of 32 spill a little (integers up to 76 bytes, doubles up to 112) and
+// passes of 32 spill a little (integers up to 52 bytes, doubles up to 76) and
 // are faster so than at 3 waves (k = 64 subset of 20M doubles 30.8 against 35.5
 // ms).  Exact pairs of doubles run 3 waves (k = 32: 172 registers, two waves,
 // without the bound: a rounded lattice of 1M 4.2 against 3.5 ms).
@@ -400,7 +400,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
     }
     const int lane = threadIdx.x;
     const int k = a.k;
-    PacketCountersFor<T, MULTI> c;
+    PacketCounters c;
     const int blk = xcd_block();
     const int W = a.width;
     if (blk * W >= a.nq) return;  // padding block of the XCD-ordered grid

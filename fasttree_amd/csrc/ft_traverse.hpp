@@ -938,22 +938,17 @@ struct KeyGrid {
 // ===========================================================================
 constexpr int PK_STACK = 128;
 
-// One packet's counts, kept in registers through the walk: 32 bits each, but
-// 64 in the integers' multi-pass walks, whose spills the compiler places better
-// so (75 scratch instructions against 167, k = 64 of 10M points 47.9 ms against
-// 59.5).
-template <typename C> struct PacketCounters {
-    C nodes = 0, leaves = 0, inserts = 0, overflow = 0;
-    C rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
+// One packet's counts, kept in registers through the walk (32 bits each: 64 cost
+// the passes of 32 2 %, k = 64 of 10M points 42.9 -> 43.9 ms).
+struct PacketCounters {
+    uint32_t nodes = 0, leaves = 0, inserts = 0, overflow = 0;
+    uint32_t rounds = 0, chains = 0;  // per wave: insertion rounds, and those that ran the chain
 };
-template <typename T, bool MULTI>
-using PacketCountersFor =
-    PacketCounters<typename std::conditional<MULTI && !CoordTraits<T>::fp, uint64_t, uint32_t>::type>;
 
-template <typename T, typename H, int MK, bool FLOOR = false, typename C>
+template <typename T, typename H, int MK, bool FLOOR = false>
 __device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
                                             T pz, int self, H &h, int32_t *stk,
-                                            PacketCounters<C> &c, int win_lo, int win_hi,
+                                            PacketCounters &c, int win_lo, int win_hi,
                                             int win_mid, typename H::Floor lo, int fill_lo,
                                             int fill_hi, uint32_t stop, int tie_k, int tie_min,
                                             const KeyGrid &kg, bool &grid) {
@@ -1201,7 +1196,7 @@ __device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool 
                 cand &= ~(hi_m & ~((1ull << a0) - 1));
             }
         }
-        c.leaves += (C)cnt;
+        c.leaves += (uint32_t)cnt;
         // One insertion round: each lane takes its lowest remaining candidate.
         // Integer periodic metrics need only the low 32 bits of coordinates.
         auto round = [&]() {
@@ -1358,10 +1353,10 @@ __device__ __forceinline__ bool packet_walk(const DTree<T> &t, int bucket, bool 
 }
 
 // The walk of lists without cut keys.
-template <typename T, typename H, int MK, bool FLOOR = false, typename C>
+template <typename T, typename H, int MK, bool FLOOR = false>
 __device__ __forceinline__ void packet_walk(const DTree<T> &t, int bucket, bool active, T px, T py,
                                             T pz, int self, H &h, int32_t *stk,
-                                            PacketCounters<C> &c, int win_lo, int win_hi,
+                                            PacketCounters &c, int win_lo, int win_hi,
                                             int win_mid,
                                             typename H::Floor lo = H::no_floor()) {
     static_assert(!H::kRankKeys, "cut keys need the tie arguments");
