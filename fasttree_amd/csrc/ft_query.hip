@@ -363,7 +363,7 @@ __global__ __launch_bounds__(256) void wave_knn_kernel(DTree<T> t, QSrc<T> qs, i
 // Packed-key packets: at least 4 waves per SIMD (128 VGPRs), 11 % faster than
 // 3 at k = 32.  With the walk's counters in 32 bits the k = 32 kernel spills
 // nothing (72 bytes a lane before: 10M clustered points 16.9 -> 16.7 ms).  The
-// passes of 32 spill a little (integers up to 52 bytes, doubles up to 76) and
+// passes of 32 spill a little (integers up to 52 bytes, doubles up to 80) and
 // are faster so than at 3 waves (k = 64 subset of 20M doubles 30.8 against 35.5
 // ms).  Exact pairs of doubles run 3 waves (k = 32: 172 registers, two waves,
 // without the bound: a rounded lattice of 1M 4.2 against 3.5 ms).
@@ -416,8 +416,8 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
     const int rank = self;  // the query's leaf rank (self queries), else -1
     if (!a.excl) self = -1;
     // Which queries are left to the listed pass is kept as masks of the wave, voted
-    // outside divergent branches.
-    const uint64_t act = __ballot(active);
+    // outside divergent branches (and after the walk, which spills for what it has
+    // to keep).
     const int tie_min = W / 4;  // tied lanes that make a packet a tied one
     KeyGrid kg;
     [[maybe_unused]] bool grid = false;  // every point so far is on kg's grid
@@ -468,6 +468,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
                 packet_walk<T, H, MK, true>(t, a.bucket, active, px, py, pz, self, h, stk, c, wlo,
                                             whi, r0, lo, 0, 0, a.stop, base ? 0 : kk, tie_min, kg,
                                             grid);
+            const uint64_t act = __ballot(active);
             bool r = false;
             if constexpr (FPK) r = !grid & h.tied();
             else if constexpr (PACKED) r = h.needs_exact(kk);
@@ -491,6 +492,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
                 if (whole) break;
             }
         }
+        const uint64_t act = __ballot(active);
         const bool over = c.leaves >= a.stop;
         if (H::kRankKeys && whole && !over) leave_packet(qm, blk, act, a.stats);
         else append_slots(qm, over ? act : redo | few, slot);
@@ -514,7 +516,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
                                                             py, pz, r0, &fst, flo, fhi, kg, grid);
                 tie_k = 0;
                 if constexpr (H::kRankKeys)
-                    ties = !grid && __popcll(__ballot(h.agreeing(k)) & act) >= tie_min;
+                    ties = !grid && __popcll(__ballot(active && h.agreeing(k))) >= tie_min;
             }
         }
         // (a packet tied by its fill still enters the walk, which ends at the root: a
@@ -523,6 +525,7 @@ __global__ __launch_bounds__(64, PACKED ? 4 : (MULTI ? 2 : 3)) void packet_knn_k
         ties |= packet_walk<T, H, MK>(t, a.bucket, active, px, py, pz, self, h, stk, c,
                                       ties ? 0 : wlo, ties ? 0 : whi, r0, H::no_floor(), flo, fhi,
                                       ties ? 0u : a.stop, tie_k, tie_min, kg, grid);
+        const uint64_t act = __ballot(active);
         const bool over = c.leaves >= a.stop;
         bool r = false;
         if constexpr (FPK) r = !grid & h.tied();
@@ -1564,8 +1567,8 @@ static int knn_dispatch(hipStream_t s, const ft_tree *tree, const QSrc<T> &qs, i
     // Canonical mode.  Packet tiers: registers for k <= 32, passes of 32 up
     // to k = 128 where packets share their walks best: every leaf, or queries
     // at least a fifth as many as the leaves up to k = 64 (10M clustered int64
-    // points, passes against the wave tier: self k = 64 / 128 47 / 103 against
-    // 107 / 154 ms, a 20 % subset k = 64 22.8 against 22.6, 1M external queries
+    // points, passes against the wave tier: self k = 64 / 128 43 / 93 against
+    // 107 / 154 ms, a 20 % subset k = 64 19.1 against 22.6, 1M external queries
     // 19.4 against 16.1; 20M doubles: self k = 64 76 against 209 ms, a 20 %
     // subset k = 64 / 128 31 / 67 against 45 / 62).  The wave tier for the
     // others up to k = 1,024 and wherever the queries are few; above k = 1,024
